@@ -5,9 +5,12 @@
 #include "../../include/hermes_amd.h"
 #include "fft_lds.h"
 #include "hermes_common.h"
+#include "pair_radial.h"
 #include "special.h"
 
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 
 namespace {
@@ -241,228 +244,11 @@ __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __r
     }
 }
 
-// j_0 .. j_LMAX at q = 2 pi t (t in turns), FP32.  One hardware sin/cos and the
-// upward recurrence when q >= LMAX + 1 (stable for every order there); otherwise
-// each order on its own (jl_f32: recurrence where q >= l + 1, else the series).
-template <int LMAX>
-__device__ __forceinline__ void radial_jl(double t, float* j) {
-    if (t == 0.0) {
-        j[0] = 1.0f;
-#pragma unroll
-        for (int l = 1; l <= LMAX; ++l) j[l] = 0.0f;
-        return;
-    }
-    const float q = (float)(2.0 * HERMES_PI * t);
-    if (LMAX == 0 || q >= (float)LMAX + 1.0f) {
-        const float fr = (float)(t - floor(t));
-        const float sn = __builtin_amdgcn_sinf(fr), cs = __builtin_amdgcn_cosf(fr);
-        const float iq = __builtin_amdgcn_rcpf(q);
-        j[0] = sn * iq;
-        if (LMAX >= 1) j[1] = (j[0] - cs) * iq;
-#pragma unroll
-        for (int n = 1; n < LMAX; ++n) j[n + 1] = (float)(2 * n + 1) * iq * j[n] - j[n - 1];
-    } else {
-#pragma unroll
-        for (int l = 0; l <= LMAX; ++l) j[l] = jl_f32(l, t);
-    }
-}
-
-// FP64 counterpart, j_0 .. j_LMAX at x = 2 pi t: one sincos and the upward
-// recurrence of jl_f64 when x >= LMAX + 1 (jl_f64 takes the same branch for
-// every order there); otherwise jl_f64 order by order.
-template <int LMAX>
-__device__ __forceinline__ void radial_jl(double t, double* j) {
-    const double x = 2.0 * HERMES_PI * t;
-    if (LMAX >= 1 && x >= (double)LMAX + 1.0) {
-        double sx, cx;
-        sincos(x, &sx, &cx);
-        j[0] = sx / x;
-        j[1] = sx / (x * x) - cx / x;
-#pragma unroll
-        for (int n = 1; n < LMAX; ++n) j[n + 1] = ((2.0 * n + 1.0) / x) * j[n] - j[n - 1];
-    } else {
-#pragma unroll
-        for (int l = 0; l <= LMAX; ++l) j[l] = jl_f64(l, x);
-    }
-}
-
-// Pair reduction for thin shells and m = 0 shell multipoles, grouped by radius.
-// For octant representative (x, y, z) and its 8 aliases a, the window of radius R
-// and order l is sum_a P(a) j_l(2 pi |a| R / L) P_l(a_z / |a|) (times the
-// descriptor's constant: 1 for a shell, N_l0 for a multipole).  The alias geometry
-// (P product, |a|, Legendre values) is computed once per representative and one
-// sin/cos per (alias, radius) serves every order.  Channel c = (radius u, order l)
-// accumulates sum_k K_c(k) Re F1 conj F2 in FP64; chan[u * (LMAX + 1) + l] is the
-// channel of (u, l) or -1.
-// T = float: FP32 windows (FP64 power and accumulation); T = double: all FP64.
-//
-// ROT (FP64 thin shells, equally spaced radii R_u = R0 + u dR): sin and cos of x = 2 pi |a| R_u / L
-// come from those at R0 by rotating through the angle 2 pi |a| dR / L (both reduced from exact turn
-// fractions once per alias), and 1 / x from 1 / (2 pi |a|) times 1 / R_u: four FMAs and two
-// multiplies per (alias, radius) in place of an FP64 sincos and a division.  x < 1 takes radial_jl
-// as before.  Each rotation adds about two ulps to |sin|, |cos| <= 1.
-template <int LMAX, typename T, typename C, bool ROT = false>
-__global__ __launch_bounds__(RED_THREADS) void k_pair_reduce_radial(int L, const C* __restrict__ F1,
-                                                                    const C* __restrict__ F2,
-                                                                    const double* __restrict__ P,
-                                                                    const double* __restrict__ radii_over_L, int nu,
-                                                                    double R0, double dR,
-                                                                    const int* __restrict__ chan, int nch,
-                                                                    double* __restrict__ partial) {
-    static_assert(!ROT || (LMAX == 0 && sizeof(T) == 8), "rotated phases: FP64 thin shells");
-    extern __shared__ double wacc[];  // [waves][nch]
-    const int Lh = L / 2 + 1;
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int nwaves = blockDim.x / 64;
-    for (int i = threadIdx.x; i < nwaves * nch; i += blockDim.x) wacc[i] = 0.0;
-    __syncthreads();
-    const int64_t nrep = (int64_t)Lh * Lh * Lh;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t base = blockIdx.x * (int64_t)blockDim.x; base < nrep; base += stride) {
-        const int64_t r = base + threadIdx.x;
-        const bool active = r < nrep;
-        double power = 0.0;
-        int x = 0, y = 0, z = 0;
-        if (active) {
-            z = (int)(r % Lh);
-            y = (int)((r / Lh) % Lh);
-            x = (int)(r / ((int64_t)Lh * Lh));
-            const int xm = (L - x) % L, ym = (L - y) % L;
-            const int nxm = (xm != x) ? 2 : 1, nym = (ym != y) ? 2 : 1;
-            const double wz = (z == 0 || z == L / 2) ? 1.0 : 2.0;
-            for (int a = 0; a < nxm; ++a)
-                for (int b = 0; b < nym; ++b) {
-                    const int xx = a ? xm : x, yy = b ? ym : y;
-                    const int64_t idx = ((int64_t)xx * L + yy) * Lh + z;
-                    const C f1 = F1[idx], f2 = F2[idx];
-                    power += wz * ((double)f1.x * (double)f2.x + (double)f1.y * (double)f2.y);
-                }
-        }
-        double sa[8];
-        T wl[8][LMAX + 1];
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-            const int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
-            const int ix = ax < 0 ? -ax : ax, iy = ay < 0 ? -ay : ay, iz = az < 0 ? -az : az;
-            const T p = (T)(P[ix] * P[iy] * P[iz]);
-            const int n2 = ax * ax + ay * ay + az * az;
-            sa[a] = sqrt((double)n2);
-            const T mu = n2 ? (T)((double)az / sa[a]) : (T)0;
-            T pm = 1, pc = mu;  // P_0, P_1
-            wl[a][0] = p;
-            if (LMAX >= 1) wl[a][1] = n2 ? p * mu : (T)0;
-#pragma unroll
-            for (int n = 1; n < LMAX; ++n) {
-                const T pn = ((T)(2 * n + 1) * mu * pc - (T)n * pm) / (T)(n + 1);
-                pm = pc;
-                pc = pn;
-                wl[a][n + 1] = n2 ? p * pn : (T)0;
-            }
-        }
-        // ROT: per alias sin, cos at the current radius, the rotation step and 1 / (2 pi |a|) (+inf for
-        // a = 0, which then always takes radial_jl)
-        double sn[8], cs[8], sd[8], cd[8], iqa[8];
-        if (ROT) {
-#pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                const double t0 = sa[a] * R0, td = sa[a] * dR;
-                sincospi(2.0 * (t0 - floor(t0)), &sn[a], &cs[a]);
-                sincospi(2.0 * (td - floor(td)), &sd[a], &cd[a]);
-                iqa[a] = sa[a] > 0.0 ? 1.0 / (2.0 * HERMES_PI * sa[a]) : __builtin_inf();
-            }
-        }
-        for (int u = 0; u < nu; ++u) {
-            const double R = radii_over_L[u];
-            const double iR = ROT ? 1.0 / R : 0.0;
-            T kb[LMAX + 1];
-#pragma unroll
-            for (int l = 0; l <= LMAX; ++l) kb[l] = 0;
-            unsigned small = 0;  // ROT: aliases with x < 1, evaluated below
-#pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                T j[LMAX + 1];
-                if (ROT) {
-                    if (u > 0) {
-                        const double s2 = fma(sn[a], cd[a], cs[a] * sd[a]);
-                        cs[a] = fma(cs[a], cd[a], -(sn[a] * sd[a]));
-                        sn[a] = s2;
-                    }
-                    if (R >= iqa[a]) {  // x = R / iqa >= 1
-                        kb[0] += sn[a] * (iqa[a] * iR) * wl[a][0];
-                    } else {
-                        small |= 1u << a;
-                    }
-                } else {
-                    radial_jl<LMAX>(sa[a] * R, j);
-#pragma unroll
-                    for (int l = 0; l <= LMAX; ++l) kb[l] += j[l] * wl[a][l];
-                }
-            }
-            // one copy of the small-argument path (it is rare: |a| R / L < 1 / (2 pi)), outside the
-            // unrolled alias loop, so its registers do not add to the rotation state's
-            for (; ROT && small; small &= small - 1) {
-                const int a = __builtin_ctz(small);
-                const int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
-                const int ix = ax < 0 ? -ax : ax, iy = ay < 0 ? -ay : ay, iz = az < 0 ? -az : az;
-                const double t = sqrt((double)(ax * ax + ay * ay + az * az)) * R;
-                kb[0] += (T)(jl_f64(0, 2.0 * HERMES_PI * t) * (P[ix] * P[iy] * P[iz]));
-            }
-#pragma unroll
-            for (int l = 0; l <= LMAX; ++l) {
-                const int c = chan[u * (LMAX + 1) + l];
-                if (c >= 0) {
-                    const double v = wave_sum(power * (double)kb[l]);
-                    if (lane == 0) wacc[wave * nch + c] += v;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    for (int b = threadIdx.x; b < nch; b += blockDim.x) {
-        double s = 0.0;
-        for (int w = 0; w < nwaves; ++w) s += wacc[w * nch + b];
-        partial[(int64_t)blockIdx.x * nch + b] = s;
-    }
-}
-
-// First stage of the fixed-order sum of block partials (nblocks rows of nch): groups of
-// PART_GROUP consecutive rows, one thread per (group, column); the kernels below finish over
-// the (nblocks / PART_GROUP) group rows.
-constexpr int PART_GROUP = 64;
-
-__global__ void k_sum_partial_groups(const double* __restrict__ partial, int nblocks, int nch,
-                                     double* __restrict__ gsum) {
-    const int ngroups = (nblocks + PART_GROUP - 1) / PART_GROUP;
-    const int64_t total = (int64_t)ngroups * nch;
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-        const int g = (int)(q / nch), c = (int)(q % nch);
-        const int r1 = min(nblocks, (g + 1) * PART_GROUP);
-        double s = 0.0;
-        for (int r = g * PART_GROUP; r < r1; ++r) s += partial[(int64_t)r * nch + c];
-        gsum[q] = s;
-    }
-}
-
-static inline int part_groups(int nblocks) { return (nblocks + PART_GROUP - 1) / PART_GROUP; }
-
-// out[d] = factor[d] * (sum over rows of channel ch_of[d]), fixed order.
-__global__ void k_plan_out(const double* __restrict__ partial, int nblocks, int nch, const int* __restrict__ ch_of,
+// out[d] = factor[d] * sums[ch_of[d]].
+__global__ void k_plan_out(const double* __restrict__ sums, const int* __restrict__ ch_of,
                            const double* __restrict__ factor, int n_desc, double* __restrict__ out) {
-    for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < n_desc; d += gridDim.x * blockDim.x) {
-        const int c = ch_of[d];
-        double s = 0.0;
-        for (int i = 0; i < nblocks; ++i) s += partial[(int64_t)i * nch + c];
-        out[d] = factor[d] * s;
-    }
-}
-
-__global__ void k_sum_partials(const double* __restrict__ partial, int nblocks, int nd, double* __restrict__ out) {
-    // one thread per output; fixed order -> deterministic
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < nd; b += gridDim.x * blockDim.x) {
-        double s = 0.0;
-        for (int i = 0; i < nblocks; ++i) s += partial[(int64_t)i * nd + b];
-        out[b] = s;
-    }
+    for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < n_desc; d += gridDim.x * blockDim.x)
+        out[d] = factor[d] * sums[ch_of[d]];
 }
 
 // ---------------------------------------------------------------- multipole apply (FP32)
@@ -952,9 +738,9 @@ int hermes_spectrum_mul(hermes_ctx* ctx, int J, int half, int dbl, void* spec, c
 // of even order <= 10 (FP32) or <= 4 (FP64), or the channels do not fit the kernel's LDS.
 struct RadialChannels {
     int LM = 0, nu = 0, nch = 0;
-    int rot = 0;                 // FP64 thin shells at >= 3 equally spaced radii R0 + u dR: rotated phases
+    int rot = 0;                 // >= 3 equally spaced radii R0 + u dR: rotated phases
     double R0 = 0.0, dR = 0.0;
-    std::vector<double> radii;   // R / L per radius
+    std::vector<double> radii;   // |R| / L per radius (the windows are even in R)
     std::vector<int> chan;       // nu x (LM + 1): channel or -1
     std::vector<int> ch_of;      // per descriptor
     std::vector<double> factor;  // per descriptor
@@ -974,7 +760,7 @@ static bool radial_channels(int J, int dbl, const hermes_window_desc* descs, int
     rc.factor.resize(n_desc);
     for (int b = 0; b < n_desc; ++b) {
         const hermes_window_desc& d = descs[b];
-        const double R = d.a0 / L;
+        const double R = std::fabs(d.a0) / L;
         size_t u = 0;
         while (u < rc.radii.size() && rc.radii[u] != R) ++u;
         if (u == rc.radii.size()) {
@@ -988,12 +774,13 @@ static bool radial_channels(int J, int dbl, const hermes_window_desc* descs, int
         rc.factor[b] = d.type == HERMES_WIN_SHELL ? 1.0 : hermes_ylm_cnorm(d.l, 0);
     }
     rc.nu = (int)rc.radii.size();
-    if (dbl && rc.LM == 0 && rc.nu >= 3) {
+    if (rc.nu >= 3) {
         const double r0 = rc.radii[0], d = (rc.radii[rc.nu - 1] - r0) / (rc.nu - 1);
         double rmax = 0.0;
-        for (double r : rc.radii) rmax = std::max(rmax, std::fabs(r));
+        for (double r : rc.radii) rmax = std::max(rmax, r);
         bool uniform = d != 0.0;
-        for (int u = 0; u < rc.nu && uniform; ++u) uniform = std::fabs(rc.radii[u] - (r0 + u * d)) <= 1e-12 * rmax;
+        // a linear binning is met to a few ulps; a phase error grows with 2 pi |a| R / L, up to a few thousand
+        for (int u = 0; u < rc.nu && uniform; ++u) uniform = std::fabs(rc.radii[u] - (r0 + u * d)) <= 1e-14 * rmax;
         if (uniform) {
             rc.rot = 1;
             rc.R0 = r0;
@@ -1003,24 +790,57 @@ static bool radial_channels(int J, int dbl, const hermes_window_desc* descs, int
     return sizeof(double) * (RED_THREADS / 64) * rc.nch <= 64 * 1024;
 }
 
-static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int nblocks, const void* F1, const void* F2,
+// Device table of the radii: R / L, then L / R.
+static std::vector<double> radius_table(const RadialChannels& ch) {
+    std::vector<double> t(2 * (size_t)ch.nu);
+    for (int u = 0; u < ch.nu; ++u) {
+        t[u] = ch.radii[u];
+        t[ch.nu + u] = 1.0 / ch.radii[u];
+    }
+    return t;
+}
+
+static int radial_block_side(int J) { return J >= 8 ? 8 : 4; }
+
+// Rows of partial sums (workgroups) of the radial kernel: a block triple each, at most max_rows.
+static int radial_rows(int J, int max_rows) {
+    const int nb = ((1 << J) / 2 + 1 + radial_block_side(J) - 1) / radial_block_side(J);
+    return std::min(max_rows, hermes_pair::tetra(nb));
+}
+
+static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int rows, const void* F1, const void* F2,
                                 const double* P, const double* d_radii, int nu, int rot, double R0, double dR,
                                 const int* d_chan, int nch, double* partial) {
-    const int L = 1 << J;
-    const size_t shmem = sizeof(double) * (RED_THREADS / 64) * nch;
-#define HERMES_RADIAL(LMV, T, C, ROT)                                                                      \
-    k_pair_reduce_radial<LMV, T, C, ROT><<<nblocks, RED_THREADS, shmem, st>>>(L, (const C*)F1, (const C*)F2, P, \
-                                                                             d_radii, nu, R0, dR, d_chan, nch, partial)
-    if (dbl) {
-        if (LM == 0 && rot) HERMES_RADIAL(0, double, double2, true);
-        else if (LM == 0) HERMES_RADIAL(0, double, double2, false);
-        else HERMES_RADIAL(4, double, double2, false);
-    } else {
-        if (LM == 0) HERMES_RADIAL(0, float, float2, false);
-        else if (LM == 4) HERMES_RADIAL(4, float, float2, false);
-        else HERMES_RADIAL(10, float, float2, false);
-    }
+    using namespace hermes_pair;
+    const int L = 1 << J, bt = radial_block_side(J), nb = (L / 2 + 1 + bt - 1) / bt, nblk = tetra(nb);
+    hipError_t e = hipSuccess;
+    auto go = [&](auto kernel, int threads, auto* f1, auto* f2) {
+        const size_t shmem = sizeof(double) * (threads / 64) * nch;
+        if (shmem > 32 * 1024)  // beside up to 25 KB of powers
+            e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+        if (e == hipSuccess)
+            kernel<<<rows, threads, shmem, st>>>(L, f1, f2, P, d_radii, nu, R0, dR, d_chan, nch, nblk, partial);
+    };
+#define HERMES_RADIAL(LMV, ROT)                                                                                      \
+    do {                                                                                                             \
+        if (dbl && bt == 8) go(k_pair_radial<LMV, ROT, 8, double2>, 256, (const double2*)F1, (const double2*)F2);    \
+        else if (dbl) go(k_pair_radial<LMV, ROT, 4, double2>, 64, (const double2*)F1, (const double2*)F2);           \
+        else if (bt == 8) go(k_pair_radial<LMV, ROT, 8, float2>, 256, (const float2*)F1, (const float2*)F2);         \
+        else go(k_pair_radial<LMV, ROT, 4, float2>, 64, (const float2*)F1, (const float2*)F2);                       \
+    } while (0)
+    if (LM == 0 && rot) HERMES_RADIAL(0, true);
+    else if (LM == 0) HERMES_RADIAL(0, false);
+    else if (LM == 4 && rot) HERMES_RADIAL(4, true);
+    else if (LM == 4) HERMES_RADIAL(4, false);
+    else if (rot) HERMES_RADIAL(10, true);
+    else HERMES_RADIAL(10, false);
 #undef HERMES_RADIAL
+    return e != hipSuccess ? e : hipGetLastError();
+}
+
+static hipError_t sum_columns(hipStream_t st, const double* partial, int rows, int n, double* out) {
+    using namespace hermes_pair;
+    k_sum_columns<<<(n + SUM_COLS - 1) / SUM_COLS, SUM_COLS * SUM_PHASES, 0, st>>>(partial, rows, n, out);
     return hipGetLastError();
 }
 
@@ -1034,6 +854,12 @@ static char* pair_workspace(hermes_ctx* ctx, char* fixed_ws, size_t fixed_cap, s
         return nullptr;
     }
     return fixed_ws;
+}
+
+// Scratch bytes of `rows` rows of n partial sums, their group sums of 64 rows and the result row.  (The group
+// sums are not formed; their room is kept so that the fixed scratch accepts and refuses the same requests.)
+static size_t pair_partial_bytes(int rows, int n) {
+    return sizeof(double) * ((size_t)rows * n + (size_t)((rows + 63) / 64) * n + n);
 }
 
 static int pair_blocks(int J) {
@@ -1050,10 +876,9 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     if (!radial_channels(J, dbl, descs, n_desc, ch)) return false;
     rc = 0;
     const int nu = ch.nu, nch = ch.nch;
-    const size_t off_chan = sizeof(double) * nu;
+    const size_t off_chan = sizeof(double) * 2 * nu;
     const size_t off_part = ((off_chan + sizeof(int) * ch.chan.size() + 255) / 256) * 256;
-    const int ng = part_groups(nblocks);
-    const size_t need = off_part + sizeof(double) * ((size_t)nblocks * nch + (size_t)ng * nch + nch);
+    const size_t need = off_part + pair_partial_bytes(nblocks, nch);
     char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);
     if (!ws) {
         rc = fixed_ws ? 2 : 1;
@@ -1061,25 +886,24 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     }
     double* d_radii = (double*)ws;
     int* d_chan = (int*)(ws + off_chan);
-    double* partial = (double*)(ws + off_part);
-    double* gsum = partial + (size_t)nblocks * nch;
-    double* d_out = gsum + (size_t)ng * nch;
+    double* d_out = (double*)(ws + off_part);
+    double* partial = d_out + nch;
+    const int rows = radial_rows(J, nblocks);
     auto fail = [&](hipError_t e) {
         hermes_set_error("pair reduction: %s", hipGetErrorString(e));
         rc = 1;
         return true;
     };
-    hipError_t e = hipMemcpyAsync(d_radii, ch.radii.data(), sizeof(double) * nu, hipMemcpyHostToDevice, ctx->stream);
+    std::vector<char> tables(off_part);  // radii and channels in one copy
+    const std::vector<double> rt = radius_table(ch);
+    memcpy(tables.data(), rt.data(), off_chan);
+    memcpy(tables.data() + off_chan, ch.chan.data(), sizeof(int) * ch.chan.size());
+    hipError_t e = hipMemcpyAsync(ws, tables.data(), off_part, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess) return fail(e);
-    e = hipMemcpyAsync(d_chan, ch.chan.data(), sizeof(int) * ch.chan.size(), hipMemcpyHostToDevice, ctx->stream);
-    if (e != hipSuccess) return fail(e);
-    if ((e = launch_radial(ctx->stream, J, dbl, ch.LM, nblocks, F1, F2, P, d_radii, nu, ch.rot, ch.R0, ch.dR, d_chan,
+    if ((e = launch_radial(ctx->stream, J, dbl, ch.LM, rows, F1, F2, P, d_radii, nu, ch.rot, ch.R0, ch.dR, d_chan,
                            nch, partial)) != hipSuccess)
         return fail(e);
-    k_sum_partial_groups<<<hermes_blocks((int64_t)ng * nch, 256), 256, 0, ctx->stream>>>(partial, nblocks, nch, gsum);
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e);
-    k_sum_partials<<<hermes_blocks(nch, 64), 64, 0, ctx->stream>>>(gsum, ng, nch, d_out);
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e);
+    if ((e = sum_columns(ctx->stream, partial, rows, nch, d_out)) != hipSuccess) return fail(e);
     std::vector<double> chs(nch);
     e = hipMemcpyAsync(chs.data(), d_out, sizeof(double) * nch, hipMemcpyDeviceToHost, ctx->stream);
     if (e != hipSuccess) return fail(e);
@@ -1092,13 +916,13 @@ struct hermes_pair_plan {
     int J = 0, dbl = 0, LM = 0, nu = 0, nch = 0, n_desc = 0, nblocks = 0;
     int rot = 0;
     double R0 = 0.0, dR = 0.0;
-    char* mem = nullptr;  // radii | chan | ch_of | factor | partial | group sums
+    char* mem = nullptr;  // radii | chan | ch_of | factor | partial | channel sums
     double* radii = nullptr;
     int* chan = nullptr;
     int* ch_of = nullptr;
     double* factor = nullptr;
     double* partial = nullptr;
-    double* gsum = nullptr;
+    double* sums = nullptr;
 };
 
 int hermes_pair_plan_destroy(hermes_pair_plan* plan) {
@@ -1135,12 +959,12 @@ int hermes_pair_plan_create(hermes_ctx* ctx, int J, int dbl, const hermes_window
     p->R0 = ch.R0;
     p->dR = ch.dR;
     p->n_desc = n_desc;
-    p->nblocks = pair_blocks(J);
+    p->nblocks = radial_rows(J, pair_blocks(J));
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t o_chan = al(sizeof(double) * ch.nu), o_chof = o_chan + al(sizeof(int) * ch.chan.size()),
+    const size_t o_chan = al(sizeof(double) * 2 * ch.nu), o_chof = o_chan + al(sizeof(int) * ch.chan.size()),
                  o_fac = o_chof + al(sizeof(int) * n_desc), o_part = o_fac + al(sizeof(double) * n_desc),
-                 o_gs = o_part + al(sizeof(double) * (size_t)p->nblocks * ch.nch),
-                 total = o_gs + sizeof(double) * (size_t)part_groups(p->nblocks) * ch.nch;
+                 o_sums = o_part + al(sizeof(double) * (size_t)p->nblocks * ch.nch),
+                 total = o_sums + sizeof(double) * (size_t)ch.nch;
     if (hipMalloc(&p->mem, total) != hipSuccess) {
         delete p;
         hermes_set_error("hermes_pair_plan_create: hipMalloc of %zu bytes failed", total);
@@ -1151,8 +975,9 @@ int hermes_pair_plan_create(hermes_ctx* ctx, int J, int dbl, const hermes_window
     p->ch_of = (int*)(p->mem + o_chof);
     p->factor = (double*)(p->mem + o_fac);
     p->partial = (double*)(p->mem + o_part);
-    p->gsum = (double*)(p->mem + o_gs);
-    hipError_t e = hipMemcpy(p->radii, ch.radii.data(), sizeof(double) * ch.nu, hipMemcpyHostToDevice);
+    p->sums = (double*)(p->mem + o_sums);
+    const std::vector<double> rt = radius_table(ch);
+    hipError_t e = hipMemcpy(p->radii, rt.data(), sizeof(double) * rt.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->chan, ch.chan.data(), sizeof(int) * ch.chan.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->ch_of, ch.ch_of.data(), sizeof(int) * n_desc, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->factor, ch.factor.data(), sizeof(double) * n_desc, hipMemcpyHostToDevice);
@@ -1171,12 +996,9 @@ int hermes_pair_reduce_planned(hermes_ctx* ctx, const hermes_pair_plan* plan, co
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
     HERMES_CHECK_HIP(launch_radial(ctx->stream, plan->J, plan->dbl, plan->LM, plan->nblocks, F1, F2, P, plan->radii,
                                    plan->nu, plan->rot, plan->R0, plan->dR, plan->chan, plan->nch, plan->partial));
-    const int ng = part_groups(plan->nblocks);
-    k_sum_partial_groups<<<hermes_blocks((int64_t)ng * plan->nch, 256), 256, 0, ctx->stream>>>(
-        plan->partial, plan->nblocks, plan->nch, plan->gsum);
-    HERMES_LAUNCH_CHECK();
-    k_plan_out<<<hermes_blocks(plan->n_desc, 64), 64, 0, ctx->stream>>>(plan->gsum, ng, plan->nch, plan->ch_of,
-                                                                       plan->factor, plan->n_desc, out_dev);
+    HERMES_CHECK_HIP(sum_columns(ctx->stream, plan->partial, plan->nblocks, plan->nch, plan->sums));
+    k_plan_out<<<hermes_blocks(plan->n_desc, 64), 64, 0, ctx->stream>>>(plan->sums, plan->ch_of, plan->factor,
+                                                                       plan->n_desc, out_dev);
     HERMES_LAUNCH_CHECK();
     return 0;
 }
@@ -1205,24 +1027,21 @@ static int pair_reduce_impl(hermes_ctx* ctx, int J, int dbl, const void* F1, con
         int rc = -1;
         if (pair_reduce_radial(ctx, J, dbl, F1, F2, P, descs, n_desc, nblocks, out_host, fixed_ws, fixed_cap, rc))
             return rc;
+        HERMES_REQUIRE(sizeof(double) * (RED_THREADS / 64) * n_desc <= 64 * 1024, "too many windows for one fused pass");
     }
-    const int ng = part_groups(nblocks);
-    size_t need = sizeof(hermes_window_desc) * n_desc + sizeof(float) * n_desc + 64 +
-                  sizeof(double) * ((size_t)nblocks * n_desc + (size_t)ng * n_desc + n_desc);
+    size_t need = sizeof(hermes_window_desc) * n_desc + sizeof(float) * n_desc + 64 + pair_partial_bytes(nblocks, n_desc);
     char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);
     if (!ws) return fixed_ws ? 2 : 1;
     hermes_window_desc* d_desc = (hermes_window_desc*)ws;
     float* d_cn = (float*)(ws + sizeof(hermes_window_desc) * n_desc);
     double* partial = (double*)(ws + ((sizeof(hermes_window_desc) * n_desc + sizeof(float) * n_desc + 63) / 64) * 64);
-    double* gsum = partial + (size_t)nblocks * n_desc;
-    double* d_out = gsum + (size_t)ng * n_desc;
+    double* d_out = partial + (size_t)nblocks * n_desc;
     std::vector<float> cn(n_desc);
     for (int b = 0; b < n_desc; ++b)
         cn[b] = descs[b].type == HERMES_WIN_SHELL_MULTIPOLE ? (float)hermes_ylm_cnorm(descs[b].l, 0) : 0.0f;
     HERMES_CHECK_HIP(hipMemcpyAsync(d_desc, descs, sizeof(hermes_window_desc) * n_desc, hipMemcpyHostToDevice, ctx->stream));
     HERMES_CHECK_HIP(hipMemcpyAsync(d_cn, cn.data(), sizeof(float) * n_desc, hipMemcpyHostToDevice, ctx->stream));
     size_t shmem = sizeof(double) * (RED_THREADS / 64) * n_desc;
-    HERMES_REQUIRE(shmem <= 64 * 1024, "too many windows for one fused pass");
     bool gen = false;
     for (int b = 0; b < n_desc; ++b) gen = gen || (descs[b].type >= HERMES_WIN_RING && descs[b].axis == 3);
     if (dbl && gen)
@@ -1238,11 +1057,7 @@ static int pair_reduce_impl(hermes_ctx* ctx, int J, int dbl, const void* F1, con
         k_pair_reduce<float2, false, false><<<nblocks, RED_THREADS, shmem, ctx->stream>>>(
             L, (const float2*)F1, (const float2*)F2, P, d_desc, d_cn, n_desc, partial);
     HERMES_LAUNCH_CHECK();
-    k_sum_partial_groups<<<hermes_blocks((int64_t)ng * n_desc, 256), 256, 0, ctx->stream>>>(partial, nblocks, n_desc,
-                                                                                            gsum);
-    HERMES_LAUNCH_CHECK();
-    k_sum_partials<<<hermes_blocks(n_desc, 64), 64, 0, ctx->stream>>>(gsum, ng, n_desc, d_out);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(sum_columns(ctx->stream, partial, nblocks, n_desc, d_out));
     HERMES_CHECK_HIP(hipMemcpyAsync(out_host, d_out, sizeof(double) * n_desc, hipMemcpyDeviceToHost, ctx->stream));
     HERMES_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     return 0;

@@ -1,0 +1,56 @@
+"""The grouped pair-reduction kernels against the general one on the same spectra.
+
+A sphere descriptor added to a list sends the whole list through the general kernel, which evaluates every
+window at every alias: the reference here.  Tolerance: |K| <= 1 and the sums are FP64, so both differ from the
+exact value by the phase error 2 pi |a| R / L * 2^-53 < 1e-13 (arguments below 1000) and, with rotated phases,
+by 2 ulps per radius, each times sum |F1 F2| <= scale; 1e-12 of scale covers them.
+"""
+
+import numpy as np
+import pytest
+
+from oracle import scaling
+
+pytestmark = pytest.mark.gpu
+
+
+def _spectra(phi, J, dtype, seed):
+    import torch
+    from pyhermes_amd import kernels
+    L = 1 << J
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    f1 = torch.randn((L, L, L), generator=gen, device="cuda", dtype=torch.float64)
+    f2 = f1 + 0.5 * torch.randn((L, L, L), generator=gen, device="cuda", dtype=torch.float64)
+    P = kernels.as_device(scaling.fourier_power_spectrum(phi, 0, 1, L, 1024), torch.float64)
+    scale = float((f1.square().mean() * f2.square().mean()).sqrt()) * L ** 6
+    return kernels.rfftn(f1.to(dtype)), kernels.rfftn(f2.to(dtype)), P, scale
+
+
+def _compare(phi, J, dtype, descs, seed):
+    import torch
+    from pyhermes_amd import kernels
+    F1, F2, P, scale = _spectra(phi, J, dtype, seed)
+    got = kernels.pair_reduce(F1, F2, P, descs)
+    again = kernels.pair_reduce(F1, F2, P, descs)
+    np.testing.assert_array_equal(got, again)
+    G1, G2 = F1.to(torch.complex128), F2.to(torch.complex128)
+    ref = kernels.pair_reduce(G1, G2, P, descs + [kernels.window_desc("sphere", 2.0)])[:-1]
+    assert np.abs(got - ref).max() <= 1e-12 * scale, np.abs(got - ref).max() / scale
+
+
+RADII = {"linear": lambda L: np.linspace(0.02 * L, 0.3 * L, 7), "uneven": lambda L: np.array([0.0, 0.3, 1.7, 0.31 * L]),
+         "one": lambda L: np.array([2.5]), "from_zero": lambda L: np.linspace(0.0, 0.4 * L, 5)}
+
+
+@pytest.mark.parametrize("J", [1, 2, 3, 5, 7, 8])
+@pytest.mark.parametrize("spacing", sorted(RADII))
+@pytest.mark.parametrize("ells,dtype", [((0,), "float64"), ((0, 2, 4), "float64"), ((2, 4), "float32"),
+                                        ((0, 6, 10), "float32")])
+def test_radial_kernel_matches_general(phi, J, spacing, ells, dtype):
+    """Shells and multipoles: blocks of 4 (J < 8) and 8, rotated and direct phases, radii down to 0 (series)."""
+    import torch
+    from pyhermes_amd import kernels
+    descs = [kernels.window_desc("shell_multipole", R, l=l) if l else kernels.window_desc("shell", R)
+             for l in ells for R in RADII[spacing](1 << J)]
+    print(f"radial J={J} {spacing} l={ells} {dtype}", flush=True)
+    _compare(phi, J, getattr(torch, dtype), descs, 100 + J)
