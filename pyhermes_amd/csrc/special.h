@@ -16,70 +16,80 @@
 #define HERMES_PI 3.14159265358979323846
 
 // ------------------------------------------------------------------ FP64 faithful
-// Cylindrical Bessel J0(x) and J1(x), x >= 0, to FP64 rounding (the reference's jn_numba,
+// Cylindrical Bessel J_NU(x), NU = 0 or 1, x = 2 pi t >= 0, to FP64 rounding (the reference's jn_numba,
 // special_functions.py:131-270, uses 8-digit rational approximations instead):
-//   x <= 4       the power series sum_k (-x^2/4)^k / (k! (k+nu)!) (x/2)^nu (largest term 4, so little
-//                cancellation);
+//   x <= 4       the power series (x/2)^NU sum_k (-x^2/4)^k / (k! (k+NU)!) (largest term 4, so little
+//                cancellation), by Horner's rule;
 //   4 < x < 25   Miller's backward recurrence J_{n-1} = (2n/x) J_n - J_{n+1} from n = x + 10 sqrt(x) + 30,
 //                normalised by J0 + 2 (J2 + J4 + ...) = 1 (values stay below 1e60 on the way down);
-//   x >= 25      Hankel's asymptotic expansion J_nu = sqrt(2/(pi x)) (P cos w - Q sin w),
-//                w = x - (2 nu + 1) pi/4, with a_k = a_{k-1} (4 nu^2 - (2k-1)^2) / (8k) and
-//                P = sum (-1)^k a_{2k} / x^{2k}, Q = sum (-1)^k a_{2k+1} / x^{2k+1}, summed while the
-//                terms fall (their smallest is about e^{-2x}).
-__host__ __device__ inline void bessel_j01_f64(double x, double& j0, double& j1) {
-    if (x <= 4.0) {
-        const double h = -0.25 * x * x;
-        double t0 = 1.0, t1 = 0.5 * x, s0 = 1.0, s1 = t1;
-        for (int k = 1; k <= 24; ++k) {
-            t0 *= h / ((double)k * k);
-            t1 *= h / ((double)k * (k + 1));
-            s0 += t0;
-            s1 += t1;
+//   x >= 25      Hankel's asymptotic expansion sqrt(2/(pi x)) (P cos w - Q sin w), w = x - (2 NU + 1) pi/4, with
+//                a_k = a_{k-1} (4 NU^2 - (2k-1)^2) / (8k), P = sum (-1)^k a_{2k} / x^{2k} and
+//                Q = sum (-1)^k a_{2k+1} / x^{2k+1}, by Horner's rule up to k = 25 (below 1e-17 at x = 25);
+//                sin and cos of x from the exact turn fraction t - floor(t).
+template <int NU>
+struct BesselCoef {
+    static constexpr int NS = 18, NH = 13;
+    double series[NS + 1];      // (-1)^k / (k! (k + NU)!)
+    double hp[NH], hq[NH];      // (-1)^k a_{2k}, (-1)^k a_{2k+1}
+    constexpr BesselCoef() : series{}, hp{}, hq{} {
+        double t = 1.0;
+        for (int k = 0; k <= NS; ++k) {
+            series[k] = t;
+            t /= -(double)((k + 1) * (k + 1 + NU));
         }
-        j0 = s0;
-        j1 = s1;
-        return;
+        double a = 1.0;
+        for (int k = 0; k < 2 * NH; ++k) {
+            const double sg = (k / 2) % 2 ? -1.0 : 1.0;
+            if (k % 2) hq[k / 2] = sg * a;
+            else hp[k / 2] = sg * a;
+            a *= (4.0 * NU * NU - (2.0 * k + 1.0) * (2.0 * k + 1.0)) / (8.0 * (k + 1.0));
+        }
+    }
+};
+
+template <int NU>
+__device__ inline double bessel_j_f64(double t) {
+    constexpr BesselCoef<NU> B{};
+    const double x = 2.0 * HERMES_PI * t;
+    if (x <= 4.0) {
+        const double h = 0.25 * x * x;
+        double s = B.series[BesselCoef<NU>::NS];
+#pragma unroll
+        for (int k = BesselCoef<NU>::NS - 1; k >= 0; --k) s = fma(s, h, B.series[k]);
+        return NU ? 0.5 * x * s : s;
     }
     if (x < 25.0) {
         const int n0 = 2 * (((int)(x + 10.0 * sqrt(x)) + 30) / 2);  // even start
         const double tox = 2.0 / x;
-        double jp = 0.0, jc = 1e-30, even_sum = 0.0, a0 = 0.0, a1 = 0.0;
-        for (int n = n0; n >= 1; --n) {
-            const double jm = n * tox * jc - jp;  // J_{n-1}
-            jp = jc;
-            jc = jm;
-            if (n == 1) {
-                a0 = jc;
-                a1 = jp;
-            } else if (((n - 1) & 1) == 0) {
-                even_sum += jc;  // J_{n-1} with n - 1 even and >= 2
-            }
+        // two steps at a time: jp = J_n (even n), jc = J_{n-1}; even_sum gathers J_2, J_4, ...
+        double jp = 0.0, jc = 1e-30, even_sum = 0.0;
+        for (int n = n0; n >= 2; n -= 2) {
+            jp = fma((double)n * tox, jc, -jp);          // J_{n-1} from J_n (jc), J_{n+1} (jp)
+            jc = fma((double)(n - 1) * tox, jp, -jc);    // J_{n-2}
+            even_sum += jc;
         }
-        const double norm = a0 + 2.0 * even_sum;
-        j0 = a0 / norm;
-        j1 = a1 / norm;
-        return;
+        const double norm = 2.0 * even_sum - jc;  // J0 + 2 (J2 + J4 + ...), jc = J0 counted twice in the sum
+        return (NU ? jp : jc) / norm;
     }
-    double out[2];
-    for (int nu = 0; nu < 2; ++nu) {
-        const double mu4 = 4.0 * nu * nu;
-        double a = 1.0, P = 1.0, Q = 0.0, prev = 1e300, xp = 1.0;
-        for (int k = 1; k <= 60; ++k) {
-            a *= (mu4 - (2.0 * k - 1.0) * (2.0 * k - 1.0)) / (8.0 * k);
-            xp *= x;
-            const double term = a / xp;
-            if (fabs(term) >= prev || fabs(term) < 1e-17) break;
-            prev = fabs(term);
-            // k odd -> Q, k even -> P; sign (-1)^{floor(k/2)}
-            const double sg = ((k / 2) & 1) ? -1.0 : 1.0;
-            if (k & 1) Q += sg * term;
-            else P += sg * term;
-        }
-        const double w = x - (2.0 * nu + 1.0) * 0.25 * HERMES_PI;
-        out[nu] = sqrt(2.0 / (HERMES_PI * x)) * (P * cos(w) - Q * sin(w));
+    const double r = 1.0 / x, r2 = r * r;
+    double P = B.hp[BesselCoef<NU>::NH - 1], Q = B.hq[BesselCoef<NU>::NH - 1];
+#pragma unroll
+    for (int k = BesselCoef<NU>::NH - 2; k >= 0; --k) {
+        P = fma(P, r2, B.hp[k]);
+        Q = fma(Q, r2, B.hq[k]);
     }
-    j0 = out[0];
-    j1 = out[1];
+    Q *= r;
+    // cos w and sin w from those of x: w = x - pi/4 (NU = 0) or x - 3 pi/4 (NU = 1); 1/sqrt(2) in the factor
+    double s, c;
+    sincospi(2.0 * (t - floor(t)), &s, &c);
+    const double cw = NU ? s - c : c + s, sw = NU ? -(s + c) : s - c;
+    return sqrt(r * (1.0 / HERMES_PI)) * (P * cw - Q * sw);
+}
+
+// Perpendicular factor of the line-of-sight windows at q = 2 pi t, t = k_perp R: J0 (ring, cylshell) or 2 J1(q)/q.
+__device__ inline double los_perp_f64(bool ring, double t) {
+    if (ring) return bessel_j_f64<0>(t);
+    return t == 0.0 ? 1.0 : bessel_j_f64<1>(t) / (HERMES_PI * t);
 }
 
 __device__ inline double jl_f64(int l, double x) {
@@ -207,13 +217,8 @@ __device__ inline double los_window_f64(int type, double ki, double kj, double k
         const double u = axis == 0 ? kj : ki, v = axis == 2 ? kj : kk;  // the two perpendicular components
         kperp2 = u * u + v * v;
     }
-    const double qperp = 2.0 * HERMES_PI * sqrt(kperp2) * R;
     const double qpar = 2.0 * HERMES_PI * kpar * H;
-    double j0, j1;
-    bessel_j01_f64(qperp, j0, j1);
-    const double perp = (type == HERMES_WIN_RING || type == HERMES_WIN_CYLSHELL)
-                            ? j0
-                            : (qperp == 0.0 ? 1.0 : 2.0 * j1 / qperp);
+    const double perp = los_perp_f64(type == HERMES_WIN_RING || type == HERMES_WIN_CYLSHELL, sqrt(kperp2) * R);
     const double par = (type == HERMES_WIN_RING || type == HERMES_WIN_DISK)
                            ? cos(qpar)
                            : (qpar == 0.0 ? 1.0 : sin(qpar) / qpar);

@@ -5,6 +5,7 @@
 #include "../../include/hermes_amd.h"
 #include "fft_lds.h"
 #include "hermes_common.h"
+#include "pair_los.h"
 #include "pair_radial.h"
 #include "special.h"
 
@@ -912,6 +913,66 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     return true;
 }
 
+// The separable path of hermes_pair_reduce for line-of-sight windows that share one coordinate axis; false
+// (rc untouched) when some window is of another kind or axis.
+static bool pair_reduce_los(hermes_ctx* ctx, int J, int dbl, const void* F1, const void* F2, const double* P,
+                            const hermes_window_desc* descs, int n_desc, int nblocks, double* out_host, char* fixed_ws,
+                            size_t fixed_cap, int& rc) {
+    using namespace hermes_pair;
+    for (int b = 0; b < n_desc; ++b)
+        if (descs[b].type < HERMES_WIN_RING || descs[b].axis > 2 || descs[b].axis != descs[0].axis) return false;
+    rc = 0;
+    auto fail = [&](hipError_t e) {
+        hermes_set_error("pair reduction: %s", hipGetErrorString(e));
+        rc = 1;
+        return true;
+    };
+    const int L = 1 << J, Lh = L / 2 + 1, nptile = (Lh * Lh + LOS_ROWS - 1) / LOS_ROWS, ntile = (n_desc + 15) / 16;
+    const int ncol = ntile * 16, rows = std::min(nptile, 1024);
+    // window tiles split over workgroups (multiples of the 4 waves) until about 1024 of them share the chip; each
+    // group forms the powers of its positions again
+    int groups = (1024 + rows - 1) / rows;
+    groups = std::max(1, std::min(groups, (ntile + 3) / 4));
+    const int tpb = ((ntile + groups - 1) / groups + 3) / 4 * 4;
+    groups = (ntile + tpb - 1) / tpb;
+    const size_t off_tab = (sizeof(hermes_window_desc) * n_desc + 255) / 256 * 256;
+    const size_t off_out = off_tab + sizeof(double) * (size_t)los_par_pad(L) * ncol;
+    const size_t need = std::max(off_out + sizeof(double) * ((size_t)rows + 1) * n_desc,
+                                 sizeof(hermes_window_desc) * n_desc + sizeof(float) * n_desc + 64 +
+                                     pair_partial_bytes(nblocks, n_desc));
+    char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);
+    if (!ws) {
+        rc = fixed_ws ? 2 : 1;
+        return true;
+    }
+    hermes_window_desc* d_desc = (hermes_window_desc*)ws;
+    double* tab = (double*)(ws + off_tab);
+    double* d_out = (double*)(ws + off_out);
+    double* partial = d_out + n_desc;
+    hipError_t e = hipMemcpyAsync(d_desc, descs, sizeof(hermes_window_desc) * n_desc, hipMemcpyHostToDevice, ctx->stream);
+    if (e != hipSuccess) return fail(e);
+    k_los_par_table<<<hermes_blocks((int64_t)los_par_pad(L) * ncol, 256, 4096), 256, 0, ctx->stream>>>(L, P, d_desc, n_desc,
+                                                                                                ncol, tab);
+    if ((e = hipGetLastError()) != hipSuccess) return fail(e);
+    const size_t shmem = sizeof(double) * ((size_t)los_par_pad(L) * LOS_PITCH + (size_t)tpb * 16);
+    auto go = [&](auto kernel, auto* f1, auto* f2) {
+        if (shmem > 48 * 1024)
+            e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+        if (e != hipSuccess) return;
+        kernel<<<dim3(rows, groups), LOS_THREADS, shmem, ctx->stream>>>(L, descs[0].axis, f1, f2, P, d_desc, n_desc, tab,
+                                                                        ncol, tpb, nptile, partial);
+        e = hipGetLastError();
+    };
+    if (dbl) go(k_pair_los<double2>, (const double2*)F1, (const double2*)F2);
+    else go(k_pair_los<float2>, (const float2*)F1, (const float2*)F2);
+    if (e != hipSuccess) return fail(e);
+    if ((e = sum_columns(ctx->stream, partial, rows, n_desc, d_out)) != hipSuccess) return fail(e);
+    if ((e = hipMemcpyAsync(out_host, d_out, sizeof(double) * n_desc, hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
+        return fail(e);
+    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return fail(e);
+    return true;
+}
+
 struct hermes_pair_plan {
     int J = 0, dbl = 0, LM = 0, nu = 0, nch = 0, n_desc = 0, nblocks = 0;
     int rot = 0;
@@ -1028,6 +1089,8 @@ static int pair_reduce_impl(hermes_ctx* ctx, int J, int dbl, const void* F1, con
         if (pair_reduce_radial(ctx, J, dbl, F1, F2, P, descs, n_desc, nblocks, out_host, fixed_ws, fixed_cap, rc))
             return rc;
         HERMES_REQUIRE(sizeof(double) * (RED_THREADS / 64) * n_desc <= 64 * 1024, "too many windows for one fused pass");
+        if (pair_reduce_los(ctx, J, dbl, F1, F2, P, descs, n_desc, nblocks, out_host, fixed_ws, fixed_cap, rc))
+            return rc;
     }
     size_t need = sizeof(hermes_window_desc) * n_desc + sizeof(float) * n_desc + 64 + pair_partial_bytes(nblocks, n_desc);
     char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);

@@ -54,3 +54,30 @@ def test_radial_kernel_matches_general(phi, J, spacing, ells, dtype):
              for l in ells for R in RADII[spacing](1 << J)]
     print(f"radial J={J} {spacing} l={ells} {dtype}", flush=True)
     _compare(phi, J, getattr(torch, dtype), descs, 100 + J)
+
+
+@pytest.mark.parametrize("J,axis,n_windows,dtype", [(1, 2, 3, "float64"), (3, 0, 16, "float64"), (4, 1, 17, "float32"),
+                                                    (5, 2, 70, "float64"), (6, 0, 33, "float32"), (6, 1, 1, "float64"),
+                                                    (7, 2, 100, "float64"), (8, 1, 5, "float64")])
+def test_axis_line_of_sight_kernel_matches_general(phi, J, axis, n_windows, dtype):
+    """Ring / disk / cylshell / cylinder windows along one axis (tiles of 16 windows and 16 positions with
+    remainders, several window groups): Bessel arguments from 0 through all three ranges."""
+    import torch
+    from pyhermes_amd import kernels
+    L = 1 << J
+    rng = np.random.default_rng(J)
+    types = ("ring", "disk", "cylshell", "cylinder")
+    descs = [kernels.window_desc(types[i % 4], 0.45 * L * rng.random() if i else 0.0, 0.4 * L * rng.random() if i != 2
+                                 else 0.0, axis=axis) for i in range(n_windows)]
+    print(f"line of sight J={J} axis={axis} n={n_windows} {dtype}", flush=True)
+    _compare(phi, J, getattr(torch, dtype), descs, 200 + J)
+
+
+def test_mixed_axes_keep_the_general_kernel(phi):
+    import torch
+    from pyhermes_amd import kernels
+    F1, F2, P, scale = _spectra(phi, 5, torch.float64, 9)
+    descs = [kernels.window_desc("ring", 3.0, 1.0 + i, axis=i) for i in range(3)]
+    got = kernels.pair_reduce(F1, F2, P, descs)
+    one = np.array([kernels.pair_reduce(F1, F2, P, [d])[0] for d in descs])
+    assert np.abs(got - one).max() <= 1e-12 * scale
