@@ -171,6 +171,12 @@ typedef struct {
 int hermes_window_build_full_profile(hermes_ctx *ctx, int J, const double *P, const hermes_radial_profile *prof,
                                      int l, int m, int dbl, void *out);
 
+/* out = spec * K * scale for that kernel K in FP64, without storing it: spec and out (different arrays) are full
+ * (L, L, L) complex128 spectra.  The window build and product of one field @ radial_multipole window
+ * (corr3pcf_multipoles.py:267-321 with convolution.py:291-295). */
+int hermes_window_apply_full_f64(hermes_ctx *ctx, int J, const double *P, const hermes_radial_profile *prof, int l,
+                                 int m, double scale, const void *spec, void *out);
+
 /* Real rFFT-layout kernel (L, L, L/2+1) of one isotropic window, summed over the
  * 8 aliases with |phi_hat|^2 weights P (L+1 values).  Replaces
  * calculate_real_window_octant_array_numba + fold_octant_window_to_rfft_kernel,

@@ -71,6 +71,8 @@ _SIGNATURES.update({
                            _dpp],
     "hermes_window_build_full_profile": [c_void_p, c_int, c_void_p, ctypes.POINTER(RadialProfile), c_int, c_int,
                                          c_int, c_void_p],
+    "hermes_window_apply_full_f64": [c_void_p, c_int, c_void_p, ctypes.POINTER(RadialProfile), c_int, c_int, c_double,
+                                     c_void_p, c_void_p],
     "hermes_multipole_window_ifft_profiles_f32": [c_void_p, c_int, c_void_p, c_void_p, ctypes.POINTER(RadialProfile),
                                                   c_int, c_int, ctypes.POINTER(c_int), c_int, c_double, c_void_p],
     "hermes_pair_reduce_noalloc": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, ctypes.POINTER(WindowDesc),

@@ -82,15 +82,6 @@ __device__ __forceinline__ double octant_power(const C* __restrict__ F1, const C
     return p;
 }
 
-// sum_k (-h/2)^k / (k! (2l+3)(2l+5)...(2l+2k+1)), h = x^2: j_l(x) (2l+1)!! / x^l.
-template <int LO, int TERMS>
-__device__ __forceinline__ double jl_series(double h) {
-    double s = 1.0;
-#pragma unroll
-    for (int k = TERMS; k >= 1; --k) s = fma(s, h * (-1.0 / (2.0 * k * (2.0 * LO + 2.0 * k + 1.0))), 1.0);
-    return s;
-}
-
 template <int N>
 __device__ __forceinline__ double ipow(double x) {
     if constexpr (N == 0) return 1.0;

@@ -2,8 +2,7 @@
 //
 // *_f64: faithful FP64 restatements of the reference algorithms
 //   spherical_jn_numba      special_functions.py:49-128
-//   assoc_legendre_numba    special_functions.py:273-304
-//   spherical_harmonic_numba special_functions.py:307-334
+//   assoc_legendre_numba, spherical_harmonic_numba  special_functions.py:273-334 (without angles)
 //   window transfer kernels window_functions.py:29-129, :426-438
 // *_f32: the FP32 fast path used by the batched kernels (no acos/atan2: Y_lm is
 //   evaluated from ((kx + i ky)/|k|)^m and the Legendre polynomial part, j_l from
@@ -92,32 +91,41 @@ __device__ inline double los_perp_f64(bool ring, double t) {
     return t == 0.0 ? 1.0 : bessel_j_f64<1>(t) / (HERMES_PI * t);
 }
 
-__device__ inline double jl_f64(int l, double x) {
+// sum_k (-h/2)^k / (k! (2l+3)(2l+5)...(2l+2k+1)), h = x^2: j_l(x) (2l+1)!! / x^l.
+template <int LO, int TERMS>
+__device__ __forceinline__ double jl_series(double h) {
+    double s = 1.0;
+#pragma unroll
+    for (int k = TERMS; k >= 1; --k) s = fma(s, h * (-1.0 / (2.0 * k * (2.0 * LO + 2.0 * k + 1.0))), 1.0);
+    return s;
+}
+
+// sin and cos of 2 pi t from the exact turn fraction.
+__device__ __forceinline__ void sincos_turns(double t, double* s, double* c) { sincospi(2.0 * (t - floor(t)), s, c); }
+
+// j_l(2 pi t)
+__device__ inline double jl_f64(int l, double t) {
     if (l < 0) return __builtin_nan("");
-    if (x == 0.0) return l == 0 ? 1.0 : 0.0;
-    double ax = fabs(x);
-    if (ax <= 5.0e-2) {
-        if (l == 0) {
-            double x2 = x * x;
-            return 1.0 - x2 / 6.0 + x2 * x2 / 120.0;
-        }
-        double denom = 1.0;
-        for (int n = 1; n <= l; ++n) denom *= 2.0 * n + 1.0;
-        double x2 = x * x;
-        return (pow(x, (double)l) / denom) *
-               (1.0 - x2 / (2.0 * (2.0 * l + 3.0)) + x2 * x2 / (8.0 * (2.0 * l + 3.0) * (2.0 * l + 5.0)));
+    if (t == 0.0) return l == 0 ? 1.0 : 0.0;
+    const double x = 2.0 * HERMES_PI * t, ax = fabs(x);
+    if (ax <= 5.0e-2) {  // the reference's truncated series
+        double lead = 1.0;
+        for (int n = 1; n <= l; ++n) lead *= x / (2.0 * n + 1.0);
+        const double x2 = x * x;
+        return lead * (1.0 - x2 / (2.0 * (2.0 * l + 3.0)) + x2 * x2 / (8.0 * (2.0 * l + 3.0) * (2.0 * l + 5.0)));
     }
+    const double ix = 1.0 / x;
     double sx, cx;
-    sincos(x, &sx, &cx);
-    double j0 = sx / x;
+    sincos_turns(t, &sx, &cx);
+    const double j0 = sx * ix;
     if (l == 0) return j0;
-    double j1 = sx / (x * x) - cx / x;
+    const double j1 = (j0 - cx) * ix;
     if (l == 1) return j1;
     if (ax < l + 1.0) {
         int n_stop = l + 40;
         double jp1 = 0.0, jcur = 1.0, jt = 0.0, jd0 = 0.0, jd1 = 0.0;
         for (int n = n_stop; n > 0; --n) {
-            double jm1 = ((2.0 * n + 1.0) / x) * jcur - jp1;
+            double jm1 = fma((2.0 * n + 1.0) * ix, jcur, -jp1);
             if (n - 1 == l) jt = jm1;
             if (n - 1 == 1) jd1 = jm1;
             if (n - 1 == 0) jd0 = jm1;
@@ -134,72 +142,65 @@ __device__ inline double jl_f64(int l, double x) {
     }
     double jm1 = j0, jcur = j1;
     for (int ell = 1; ell < l; ++ell) {
-        double jn = ((2.0 * ell + 1.0) / x) * jcur - jm1;
+        const double jn = fma((2.0 * ell + 1.0) * ix, jcur, -jm1);
         jm1 = jcur;
         jcur = jn;
     }
     return jcur;
 }
 
-__device__ inline double plm_f64(int l, int m, double x) {
-    double pmm = 1.0;
-    if (m > 0) {
-        double t = 1.0 - x * x;
-        double somx2 = sqrt(t > 0.0 ? t : 0.0);
-        double fact = 1.0;
-        for (int i = 0; i < m; ++i) {
-            pmm *= -fact * somx2;
-            fact += 2.0;
-        }
+// Y_l^m of a fixed (l, m) without angles: norm poly(mu) ((kx + i ky) / k)^|m| with poly the part of P_l^|m|
+// free of (1 - mu^2)^(|m|/2), by its recurrence in l with coefficients tabulated on the host.
+struct YlmTable {
+    int l, m;
+    double norm;           // N_l|m| (-1)^|m| (2|m| - 1)!!
+    double a[41], b[41];   // poly_n = a[n] mu poly_{n-1} - b[n] poly_{n-2}, |m| + 2 <= n <= l
+};
+
+// ik = 1 / |k|, 0 for k = 0 (where Y_00 is its constant and every other order 0).
+__device__ inline double2 ylm_f64(const YlmTable& Y, double kx, double ky, double kz, double ik) {
+    const int am = Y.m < 0 ? -Y.m : Y.m;
+    const double mu = kz * ik, ur = kx * ik, ui = ky * ik;
+    double p = 1.0, q = (2.0 * am + 1.0) * mu;
+    if (Y.l == am) q = 1.0;
+    for (int n = am + 2; n <= Y.l; ++n) {
+        const double r = fma(Y.a[n] * mu, q, -Y.b[n] * p);
+        p = q;
+        q = r;
     }
-    if (l == m) return pmm;
-    double pmmp1 = x * (2.0 * m + 1.0) * pmm;
-    if (l == m + 1) return pmmp1;
-    double a = pmm, b = pmmp1, pll = 0.0;
-    for (int ell = m + 2; ell <= l; ++ell) {
-        pll = ((2.0 * ell - 1.0) * x * b - (ell + m - 1.0) * a) / (ell - m);
-        a = b;
-        b = pll;
+    double pr = Y.norm * q, pi = 0.0;
+    for (int i = 0; i < am; ++i) {
+        const double t = pr * ur - pi * ui;
+        pi = pr * ui + pi * ur;
+        pr = t;
     }
-    return pll;
+    if (ik == 0.0 && Y.l > 0) pr = pi = 0.0;
+    if (Y.m < 0) {  // Y_{l,-m} = (-1)^m conj(Y_{l,m})
+        const double sg = (am & 1) ? -1.0 : 1.0;
+        return make_double2(sg * pr, -sg * pi);
+    }
+    return make_double2(pr, pi);
 }
 
-__device__ inline double factorial_small_f64(int n) {
-    double out = 1.0;
-    for (int i = 2; i <= n; ++i) out *= i;
-    return out;
-}
-
-__device__ inline double2 ylm_f64(int l, int m, double ki, double kj, double kk) {
-    if (l < 0) return make_double2(__builtin_nan(""), 0.0);
-    int am = m < 0 ? -m : m;
-    if (am > l) return make_double2(0.0, 0.0);
-    double k = sqrt(ki * ki + kj * kj + kk * kk);
-    if (k == 0.0) {
-        if (l == 0 && m == 0) return make_double2(1.0 / sqrt(4.0 * HERMES_PI), 0.0);
-        return make_double2(0.0, 0.0);
+// N_l0 P_l(mu), the real spherical harmonic of m = 0 (0 at k = 0 unless l = 0: mu is then 0 and ik 0).
+__device__ inline double yl0_f64(int l, double mu) {
+    double p = 1.0, q = mu;
+    if (l == 0) q = 1.0;
+    for (int n = 2; n <= l; ++n) {
+        const double r = ((2.0 * n - 1.0) * mu * q - (n - 1.0) * p) / n;
+        p = q;
+        q = r;
     }
-    double mu = kk / k;
-    if (mu > 1.0) mu = 1.0;
-    else if (mu < -1.0) mu = -1.0;
-    double theta = acos(mu);
-    double ph = atan2(kj, ki);
-    double x = cos(theta);
-    double P = plm_f64(l, am, x);
-    double norm = sqrt((2.0 * l + 1.0) / (4.0 * HERMES_PI) * factorial_small_f64(l - am) / factorial_small_f64(l + am));
-    double s = norm * P;
-    double re = s * cos(am * ph), im = s * sin(am * ph);
-    if (m >= 0) return make_double2(re, im);
-    double sign = (am % 2 == 1) ? -1.0 : 1.0;
-    return make_double2(sign * re, -sign * im);
+    return sqrt((2.0 * l + 1.0) / (4.0 * HERMES_PI)) * q;
 }
 
 __device__ inline double win_sphere_f64(double k, double R) {
-    double q = 2 * HERMES_PI * k * R;
-    if (q == 0.0) return 1.0;
+    // 3 j_1(q) / q; below q = 1 by its series (s - q c cancels)
+    const double q = 2 * HERMES_PI * (k * R), q2 = q * q;
+    if (q2 < 1.0) return jl_series<1, 9>(q2);
     double s, c;
-    sincos(q, &s, &c);
-    return 3 * (s - q * c) / (q * q * q);
+    sincos_turns(k * R, &s, &c);
+    return 3 * (s - q * c) / (q2 * q);
 }
 
 // Line-of-sight windows (window_functions.py:164-319).  Along a coordinate axis they are even in every
@@ -225,27 +226,20 @@ __device__ inline double los_window_f64(int type, double ki, double kj, double k
     return perp * par;
 }
 
-// Transfer function of one real, even window at k (cycles per grid cell): the isotropic ones and the
-// line-of-sight ones.
-__device__ inline double iso_window_f64(int type, double ki, double kj, double kk, double a0, double a1,
-                                        int axis = 2, const double* los = nullptr) {
-    if (type >= HERMES_WIN_RING && type <= HERMES_WIN_CYLINDER)
-        return los_window_f64(type, ki, kj, kk, a0, a1, axis, los);
+// Transfer function of one isotropic window at |k| = k cycles per grid cell.
+__device__ inline double isotropic_f64(int type, double k, double a0, double a1) {
     switch (type) {
-    case HERMES_WIN_SPHERE: return win_sphere_f64(sqrt(ki * ki + kj * kj + kk * kk), a0);
+    case HERMES_WIN_SPHERE: return win_sphere_f64(k, a0);
     case HERMES_WIN_GAUSSIAN: {
-        double k = sqrt(ki * ki + kj * kj + kk * kk);
         double q = 2 * HERMES_PI * k * a0;
         return exp(-(q * q) / 2);
     }
     case HERMES_WIN_SHELL: {
-        double k = sqrt(ki * ki + kj * kj + kk * kk);
-        double q = 2 * HERMES_PI * k * a0;
+        const double q = 2 * HERMES_PI * (k * a0);
         if (q == 0.0) return 1.0;
-        return sin(q) / q;
+        return sinpi(2.0 * (k * a0 - floor(k * a0))) / q;
     }
     case HERMES_WIN_THICK_SHELL: {
-        double k = sqrt(ki * ki + kj * kj + kk * kk);
         double ri = a0 - 0.5 * a1;
         if (ri < 0.0) ri = 0.0;
         double ro = a0 + 0.5 * a1;
@@ -254,22 +248,30 @@ __device__ inline double iso_window_f64(int type, double ki, double kj, double k
         return (ro * ro * ro * win_sphere_f64(k, ro) - ri * ri * ri * win_sphere_f64(k, ri)) / den;
     }
     case HERMES_WIN_GAUSSIAN_SHELL: {
-        double k = sqrt(ki * ki + kj * kj + kk * kk);
         if (k == 0) return 1.0;
-        double qs = 2 * HERMES_PI * k * a0;
+        double qs = 2 * HERMES_PI * (k * a0);
         double qm = 2 * HERMES_PI * k * a1;
         double den = a0 * a0 + a1 * a1;
         if (den == 0.0) return 1.0;
-        double sinc = (qs == 0.0) ? 1.0 : sin(qs) / qs;
-        return (a1 * a1 * cos(qs) + a0 * a0 * sinc) / den * exp(-(qm * qm) / 2);
+        double sn, cs;
+        sincos_turns(k * a0, &sn, &cs);
+        double sinc = (qs == 0.0) ? 1.0 : sn / qs;
+        return (a1 * a1 * cs + a0 * a0 * sinc) / den * exp(-(qm * qm) / 2);
     }
-    case HERMES_WIN_INVERSE_LAPLACIAN: {
-        double k2 = ki * ki + kj * kj + kk * kk;
-        if (k2 == 0.0) return 0.0;
-        return -1.0 / (((2.0 * HERMES_PI) * (2.0 * HERMES_PI)) * k2);
-    }
+    case HERMES_WIN_INVERSE_LAPLACIAN:
+        if (k == 0.0) return 0.0;
+        return -1.0 / (((2.0 * HERMES_PI) * (2.0 * HERMES_PI)) * (k * k));
     }
     return __builtin_nan("");
+}
+
+// The same for any real, even window at k: the isotropic ones and, unless LOS is false, the line-of-sight ones.
+template <bool LOS = true>
+__device__ inline double iso_window_f64(int type, double ki, double kj, double kk, double a0, double a1,
+                                        int axis = 2, const double* los = nullptr) {
+    if (LOS && type >= HERMES_WIN_RING && type <= HERMES_WIN_CYLINDER)
+        return los_window_f64(type, ki, kj, kk, a0, a1, axis, los);
+    return isotropic_f64(type, sqrt(ki * ki + kj * kj + kk * kk), a0, a1);
 }
 
 // U_l(k) of a radial profile at k cycles per grid cell (hermes_radial_profile; FP64).
@@ -286,27 +288,26 @@ __device__ inline double radial_table_f64(const double* __restrict__ tab, int n,
 
 __device__ inline double radial_profile_f64(const hermes_radial_profile& p, int l, double k) {
     switch (p.kind) {
-    case HERMES_RADIAL_SHELL: return jl_f64(l, 2.0 * HERMES_PI * k * p.a0);
+    case HERMES_RADIAL_SHELL: return jl_f64(l, k * p.a0);
     case HERMES_RADIAL_TABLE: return radial_table_f64(p.table, p.n_table, k * p.k_scale);
-    case HERMES_RADIAL_SPHERE: return iso_window_f64(HERMES_WIN_SPHERE, k, 0.0, 0.0, p.a0, p.a1);
-    case HERMES_RADIAL_GAUSSIAN: return iso_window_f64(HERMES_WIN_GAUSSIAN, k, 0.0, 0.0, p.a0, p.a1);
-    case HERMES_RADIAL_THICK_SHELL: return iso_window_f64(HERMES_WIN_THICK_SHELL, k, 0.0, 0.0, p.a0, p.a1);
-    case HERMES_RADIAL_GAUSSIAN_SHELL: return iso_window_f64(HERMES_WIN_GAUSSIAN_SHELL, k, 0.0, 0.0, p.a0, p.a1);
+    case HERMES_RADIAL_SPHERE: return isotropic_f64(HERMES_WIN_SPHERE, k, p.a0, p.a1);
+    case HERMES_RADIAL_GAUSSIAN: return isotropic_f64(HERMES_WIN_GAUSSIAN, k, p.a0, p.a1);
+    case HERMES_RADIAL_THICK_SHELL: return isotropic_f64(HERMES_WIN_THICK_SHELL, k, p.a0, p.a1);
+    case HERMES_RADIAL_GAUSSIAN_SHELL: return isotropic_f64(HERMES_WIN_GAUSSIAN_SHELL, k, p.a0, p.a1);
     }
     return __builtin_nan("");
 }
 
-// Complex transfer function of a window at signed k (isotropic windows are real).  general = false
-// compiles out the non-axis line-of-sight branch (for callers that never see axis-3 descriptors).
-__device__ inline double2 window_value_f64(const hermes_window_desc& d, double ki, double kj, double kk,
-                                           bool general = true) {
+// Transfer function of a real window at signed k: the isotropic and line-of-sight ones and the m = 0 multipoles.
+// general = false compiles out the non-axis line-of-sight branch (for callers that never see axis-3 descriptors).
+__device__ inline double real_window_f64(const hermes_window_desc& d, double ki, double kj, double kk,
+                                         bool general = true) {
     if (d.type == HERMES_WIN_SHELL_MULTIPOLE) {
-        double k = sqrt(ki * ki + kj * kj + kk * kk);
-        double radial = jl_f64(d.l, 2.0 * HERMES_PI * k * d.a0);
-        double2 y = ylm_f64(d.l, d.m, ki, kj, kk);
-        return make_double2(radial * y.x, radial * y.y);
+        const double k = sqrt(ki * ki + kj * kj + kk * kk);
+        if (k == 0.0) return d.l == 0 ? sqrt(0.25 / HERMES_PI) : 0.0;
+        return jl_f64(d.l, k * d.a0) * yl0_f64(d.l, kk / k);
     }
-    return make_double2(iso_window_f64(d.type, ki, kj, kk, d.a0, d.a1, d.axis, general ? d.los : nullptr), 0.0);
+    return iso_window_f64(d.type, ki, kj, kk, d.a0, d.a1, d.axis, general ? d.los : nullptr);
 }
 
 // ------------------------------------------------------------------ FP32 fast path

@@ -24,93 +24,138 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // ---------------------------------------------------------------- kernel builders
+// Every built-in window has a definite symmetry under the reversal of a k component, and the alias sum of an
+// octant position (x, y, z) in [0, L/2]^3 keeps it: the kernel at a mirrored position (L - x for x, ...) is
+//   x: (-1)^m conj K,   y: conj K,   z: (-1)^(l+m) K      (real windows: l = m = 0),
+// so one evaluation serves up to 8 positions.  (A zero component is its own mirror; its aliases are 0 and -L.)
+// Only a line of sight off the axes lacks the symmetry: k_build_rfft_general and k_build_full_general.
+// Window sums are FP64 VALU work: for a thin-shell multipole about 8 (sin, cos, recurrences) per position, the
+// store of 8 positions otherwise.  One evaluation per position and Y_lm through acos, atan2, cos and sin took
+// 7.50 ms (l <= 2, FP64, L = 256) before the product with the spectrum (0.14 ms); this takes 0.12 ms with it.
+
+// Aliases of an octant position in the fold's order, (0,0,0) (1,0,0) (0,1,0) (0,0,1) (1,1,0) (1,0,1) (0,1,1)
+// (1,1,1) of convolution.py:263-281; bit 2: x, bit 1: y, bit 0: z.
+__device__ constexpr int FOLD_ORDER[8] = {0, 4, 2, 1, 6, 5, 3, 7};
+
 // convolution.py:14-38 + :263-281: K[x,y,z] = sum over the 8 mirrors {x, L-x} x ... of
-// P[i]P[j]P[k] W(i/L, j/L, k/L), in the fold's summation order.
+// P[i]P[j]P[k] W(i/L, j/L, k/L), for windows even in every component.
+// LOS false compiles the line-of-sight windows out: their Bessel series double the registers.
+template <typename T, bool LOS>
+__global__ __launch_bounds__(256, 2) void k_build_rfft(int L, const double* __restrict__ P, hermes_window_desc d,
+                                                    T* __restrict__ out) {
+    const int Lh = L / 2 + 1;
+    const int64_t n = (int64_t)Lh * Lh * Lh;
+    const double inv_L = 1.0 / L;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int z = (int)(i % Lh), y = (int)((i / Lh) % Lh), x = (int)(i / ((int64_t)Lh * Lh));
+        double t = 0.0;
+        for (int a = 0; a < 8; ++a) {
+            const int o = FOLD_ORDER[a];
+            const int ii = (o & 4) ? L - x : x, jj = (o & 2) ? L - y : y, kk = (o & 1) ? L - z : z;
+            t += P[ii] * P[jj] * P[kk] *
+                 iso_window_f64<LOS>(d.type, ii * inv_L, jj * inv_L, kk * inv_L, d.a0, d.a1, d.axis, nullptr);
+        }
+        if (d.type == HERMES_WIN_INVERSE_LAPLACIAN && i == 0) t = 0.0;
+        const int xm = (L - x) & (L - 1), ym = (L - y) & (L - 1);
+        out[((int64_t)x * L + y) * Lh + z] = (T)t;
+        if (xm != x) out[((int64_t)xm * L + y) * Lh + z] = (T)t;
+        if (ym != y) out[((int64_t)x * L + ym) * Lh + z] = (T)t;
+        if (xm != x && ym != y) out[((int64_t)xm * L + ym) * Lh + z] = (T)t;
+    }
+}
+
+// The same for a line of sight off the axes (descriptor axis 3), even only under k -> -k: every position sums its
+// signed aliases (the mirror alias L - x sits at k = -(L - x) / L).
 template <typename T>
-__global__ void k_build_rfft(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
+__global__ __launch_bounds__(256, 2) void k_build_rfft_general(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
     const int Lh = L / 2 + 1;
     const int64_t n = (int64_t)L * L * Lh;
     const double inv_L = 1.0 / L;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int z = (int)(i % Lh);
-        int y = (int)((i / Lh) % L);
-        int x = (int)(i / ((int64_t)Lh * L));
-        int xs[2] = {x, L - x}, ys[2] = {y, L - y}, zs[2] = {z, L - z};
-        // fold order: (0,0,0) (1,0,0) (0,1,0) (0,0,1) (1,1,0) (1,0,1) (0,1,1) (1,1,1)
-        const int ord[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 0}, {1, 0, 1}, {0, 1, 1}, {1, 1, 1}};
+        const int z = (int)(i % Lh), y = (int)((i / Lh) % L), x = (int)(i / ((int64_t)Lh * L));
         double t = 0.0;
-#pragma unroll
         for (int a = 0; a < 8; ++a) {
-            int ii = xs[ord[a][0]], jj = ys[ord[a][1]], kk = zs[ord[a][2]];
-            double wa = 0.0;
-            // the mirror alias L - x sits at k = -(L - x) / L (the sign matters for a non-axis line of sight)
-            const double sx = ord[a][0] ? -1.0 : 1.0, sy = ord[a][1] ? -1.0 : 1.0, sz = ord[a][2] ? -1.0 : 1.0;
-            wa += P[ii] * P[jj] * P[kk] *
-                  iso_window_f64(d.type, sx * ii * inv_L, sy * jj * inv_L, sz * kk * inv_L, d.a0, d.a1, d.axis, d.los);
-            t = (a == 0) ? wa : t + wa;
+            const int o = FOLD_ORDER[a];
+            const int ii = (o & 4) ? x - L : x, jj = (o & 2) ? y - L : y, kk = (o & 1) ? z - L : z;
+            t += P[ii < 0 ? -ii : ii] * P[jj < 0 ? -jj : jj] * P[kk < 0 ? -kk : kk] *
+                 iso_window_f64(d.type, ii * inv_L, jj * inv_L, kk * inv_L, d.a0, d.a1, d.axis, d.los);
         }
-        if (d.type == HERMES_WIN_INVERSE_LAPLACIAN && i == 0) t = 0.0;
         out[i] = (T)t;
     }
 }
 
-// radial_multipole_windows.py:147-183 order: aliases (x-L | x) per axis, "0" first.
-template <typename T>
-__global__ void k_build_full(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
-    const int64_t n = (int64_t)L * L * L;
+// Full-grid complex kernels in the alias order of radial_multipole_windows.py:147-183 ((x-L | x) per axis, "0"
+// first), one octant position per thread.  KIND 0: a real window of desc (isotropic, line of sight along an
+// axis); 1: j_l(2 pi |k| R) Y_lm with R = prof.a0; 2: U_l(|k|) Y_lm of a radial profile
+// (radial_multipole_windows.py:186-264).  APPLY: writes spec * K * scale instead of K (FP64; the product of
+// convolution.py:291-295 without storing K).
+template <typename T, int KIND, bool APPLY>
+__global__ __launch_bounds__(256, 2) void k_build_full(int L, const double* __restrict__ P, hermes_window_desc d,
+                                                    hermes_radial_profile prof, YlmTable Y, double scale,
+                                                    const double2* __restrict__ spec, T* __restrict__ out) {
+    const int Lh = L / 2 + 1;
+    const int64_t n = (int64_t)Lh * Lh * Lh;
     const double inv_L = 1.0 / L;
+    const int am = Y.m < 0 ? -Y.m : Y.m;
+    const double sx = KIND && (am & 1) ? -1.0 : 1.0, sz = KIND && ((Y.l + am) & 1) ? -1.0 : 1.0;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int z = (int)(i % L);
-        int y = (int)((i / L) % L);
-        int x = (int)(i / ((int64_t)L * L));
-        double pi[2] = {P[L - x], P[x]}, pj[2] = {P[L - y], P[y]}, pk[2] = {P[L - z], P[z]};
-        double ki[2] = {(x - L) * inv_L, x * inv_L}, kj[2] = {(y - L) * inv_L, y * inv_L},
-               kk[2] = {(z - L) * inv_L, z * inv_L};
+        const int z = (int)(i % Lh), y = (int)((i / Lh) % Lh), x = (int)(i / ((int64_t)Lh * Lh));
         double re = 0.0, im = 0.0;
-#pragma unroll
         for (int a = 0; a < 8; ++a) {
-            int u = (a >> 2) & 1, v = (a >> 1) & 1, w = a & 1;
-            double p = pi[u] * pj[v] * pk[w];
-            double2 wv = window_value_f64(d, ki[u], kj[v], kk[w]);
-            if (a == 0) {
-                re = p * wv.x;
-                im = p * wv.y;
+            const int ax = (a & 4) ? x : x - L, ay = (a & 2) ? y : y - L, az = (a & 1) ? z : z - L;
+            const double p = P[ax < 0 ? -ax : ax] * P[ay < 0 ? -ay : ay] * P[az < 0 ? -az : az];
+            const double kx = ax * inv_L, ky = ay * inv_L, kz = az * inv_L;
+            if (KIND == 0) {
+                re += p * iso_window_f64(d.type, kx, ky, kz, d.a0, d.a1, d.axis, nullptr);
             } else {
-                re += p * wv.x;
-                im += p * wv.y;
+                const double k = sqrt(kx * kx + ky * ky + kz * kz);
+                const double rad = p * (KIND == 1 ? jl_f64(Y.l, k * prof.a0) : radial_profile_f64(prof, Y.l, k));
+                const double2 yv = ylm_f64(Y, kx, ky, kz, k == 0.0 ? 0.0 : 1.0 / k);
+                re += rad * yv.x;
+                im += rad * yv.y;
             }
         }
-        if (d.type == HERMES_WIN_INVERSE_LAPLACIAN && i == 0) re = im = 0.0;
-        out[2 * i] = (T)re;
-        out[2 * i + 1] = (T)im;
+        if (KIND == 0 && d.type == HERMES_WIN_INVERSE_LAPLACIAN && i == 0) re = 0.0;
+        if (APPLY) {
+            re *= scale;
+            im *= scale;
+        }
+#pragma unroll
+        for (int mode = 0; mode < 8; ++mode) {
+            const bool fx = mode & 4, fy = mode & 2, fz = mode & 1;
+            const int xx = fx ? (L - x) & (L - 1) : x, yy = fy ? (L - y) & (L - 1) : y,
+                      zz = fz ? (L - z) & (L - 1) : z;
+            if ((fx && xx == x) || (fy && yy == y) || (fz && zz == z)) continue;
+            const double sg = (fx ? sx : 1.0) * (fz ? sz : 1.0);
+            double kr = sg * re, ki = (fx != fy) ? -sg * im : sg * im;
+            const int64_t o = ((int64_t)xx * L + yy) * L + zz;
+            if (APPLY) {
+                const double2 f = spec[o];
+                const double t = f.x * kr - f.y * ki;
+                ki = f.x * ki + f.y * kr;
+                kr = t;
+            }
+            if constexpr (sizeof(T) == 8) *(double2*)(out + 2 * o) = make_double2(kr, ki);
+            else *(float2*)(out + 2 * o) = make_float2((float)kr, (float)ki);
+        }
     }
 }
 
-// radial_multipole_windows.py:147-183 and :186-264: K[x,y,z] = sum over the 8 signed aliases of
-// P P P U_l(|k|) Y_lm(k-hat), U_l from a radial profile (closed form or table).
+// A real window along a line of sight off the axes (descriptor axis 3), position by position.
 template <typename T>
-__global__ void k_build_full_profile(int L, const double* __restrict__ P, hermes_radial_profile prof, int l, int m,
-                                     T* __restrict__ out) {
+__global__ __launch_bounds__(256, 2) void k_build_full_general(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
     const int64_t n = (int64_t)L * L * L;
     const double inv_L = 1.0 / L;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int z = (int)(i % L), y = (int)((i / L) % L), x = (int)(i / ((int64_t)L * L));
-        const double pi[2] = {P[L - x], P[x]}, pj[2] = {P[L - y], P[y]}, pk[2] = {P[L - z], P[z]};
-        const double ki[2] = {(x - L) * inv_L, x * inv_L}, kj[2] = {(y - L) * inv_L, y * inv_L},
-                     kk[2] = {(z - L) * inv_L, z * inv_L};
-        double re = 0.0, im = 0.0;
-#pragma unroll
+        double re = 0.0;
         for (int a = 0; a < 8; ++a) {
-            const int u = (a >> 2) & 1, v = (a >> 1) & 1, w = a & 1;
-            const double p = pi[u] * pj[v] * pk[w];
-            const double k = sqrt(ki[u] * ki[u] + kj[v] * kj[v] + kk[w] * kk[w]);
-            const double rad = radial_profile_f64(prof, l, k);
-            const double2 yv = ylm_f64(l, m, ki[u], kj[v], kk[w]);
-            re += p * rad * yv.x;
-            im += p * rad * yv.y;
+            const int ax = (a & 4) ? x : x - L, ay = (a & 2) ? y : y - L, az = (a & 1) ? z : z - L;
+            re += P[ax < 0 ? -ax : ax] * P[ay < 0 ? -ay : ay] * P[az < 0 ? -az : az] *
+                  iso_window_f64(d.type, ax * inv_L, ay * inv_L, az * inv_L, d.a0, d.a1, d.axis, d.los);
         }
         out[2 * i] = (T)re;
-        out[2 * i + 1] = (T)im;
+        out[2 * i + 1] = (T)0;
     }
 }
 
@@ -212,7 +257,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __r
                             int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
                             int ix = ax < 0 ? -ax : ax, iy = ay < 0 ? -ay : ay, iz = az < 0 ? -az : az;
                             double p = P[ix] * P[iy] * P[iz];
-                            const double w = window_value_f64(d, sx * ax * inv_L, sy * ay * inv_L, az * inv_L).x;
+                            const double w = real_window_f64(d, sx * ax * inv_L, sy * ay * inv_L, az * inv_L);
                             km += FP64 ? p * w : (double)((float)p * (float)w);
                         }
                         kb += pm * km;
@@ -224,7 +269,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __r
                         double p = P[ix] * P[iy] * P[iz];
                         if (FP64) {
                             double inv_L = 1.0 / L;
-                            kb += p * window_value_f64(d, ax * inv_L, ay * inv_L, az * inv_L, GEN).x;
+                            kb += p * real_window_f64(d, ax * inv_L, ay * inv_L, az * inv_L, GEN);
                         } else {
                             kb += (double)((float)p * window_value_f32(d, ax, ay, az, L, cnorms[b]));
                         }
@@ -664,12 +709,55 @@ int hermes_window_build_rfft(hermes_ctx* ctx, int J, const double* P, const herm
     HERMES_REQUIRE(desc->type != HERMES_WIN_SHELL_MULTIPOLE, "multipole windows need the full complex layout");
     if (int rc = check_desc(*desc)) return rc;
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
-    int L = 1 << J;
-    int64_t n = (int64_t)L * L * (L / 2 + 1);
-    if (dbl) k_build_rfft<double><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
-    else k_build_rfft<float><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
+    const int L = 1 << J, Lh = L / 2 + 1;
+    if (desc->type >= HERMES_WIN_RING && desc->axis == 3) {
+        const unsigned nb = hermes_blocks((int64_t)L * L * Lh, 256, 65536);
+        if (dbl) k_build_rfft_general<double><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
+        else k_build_rfft_general<float><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
+    } else {
+        const unsigned nb = hermes_blocks((int64_t)Lh * Lh * Lh, 256, 65536);
+        const bool los = desc->type >= HERMES_WIN_RING;
+        if (dbl && los) k_build_rfft<double, true><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
+        else if (dbl) k_build_rfft<double, false><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
+        else if (los) k_build_rfft<float, true><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
+        else k_build_rfft<float, false><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
+    }
     HERMES_LAUNCH_CHECK();
     return 0;
+}
+
+static YlmTable ylm_table(int l, int m) {
+    YlmTable Y{};
+    const int am = m < 0 ? -m : m;
+    Y.l = l;
+    Y.m = m;
+    Y.norm = hermes_ylm_cnorm(l, am);
+    for (int n = am + 2; n <= l; ++n) {
+        Y.a[n] = (2.0 * n - 1.0) / (n - am);
+        Y.b[n] = (n + am - 1.0) / (n - am);
+    }
+    return Y;
+}
+
+// One launch of k_build_full: kind as its KIND; spec != nullptr applies it (FP64).
+static hipError_t launch_build_full(hermes_ctx* ctx, int J, int kind, const double* P, const hermes_window_desc& d,
+                                    const hermes_radial_profile& prof, int l, int m, int dbl, double scale,
+                                    const double2* spec, void* out) {
+    const int L = 1 << J, Lh = L / 2 + 1;
+    const unsigned nb = hermes_blocks((int64_t)Lh * Lh * Lh, 256, 65536);
+    const YlmTable Y = ylm_table(l, m);
+#define HERMES_BUILD(T, KIND, APPLY) \
+    k_build_full<T, KIND, APPLY><<<nb, 256, 0, ctx->stream>>>(L, P, d, prof, Y, scale, spec, (T*)out)
+    if (spec && kind == 1) HERMES_BUILD(double, 1, true);
+    else if (spec) HERMES_BUILD(double, 2, true);
+    else if (dbl && kind == 0) HERMES_BUILD(double, 0, false);
+    else if (dbl && kind == 1) HERMES_BUILD(double, 1, false);
+    else if (dbl) HERMES_BUILD(double, 2, false);
+    else if (kind == 0) HERMES_BUILD(float, 0, false);
+    else if (kind == 1) HERMES_BUILD(float, 1, false);
+    else HERMES_BUILD(float, 2, false);
+#undef HERMES_BUILD
+    return hipGetLastError();
 }
 
 int hermes_window_build_full(hermes_ctx* ctx, int J, const double* P, const hermes_window_desc* desc, int dbl,
@@ -678,11 +766,19 @@ int hermes_window_build_full(hermes_ctx* ctx, int J, const double* P, const herm
     HERMES_REQUIRE(J >= 1 && J <= 10, "J=%d unsupported", J);
     if (int rc = check_desc(*desc)) return rc;
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
-    int L = 1 << J;
-    int64_t n = (int64_t)L * L * L;
-    if (dbl) k_build_full<double><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
-    else k_build_full<float><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
-    HERMES_LAUNCH_CHECK();
+    hermes_radial_profile prof{};
+    if (desc->type == HERMES_WIN_SHELL_MULTIPOLE) {
+        prof.a0 = desc->a0;
+        HERMES_CHECK_HIP(launch_build_full(ctx, J, 1, P, *desc, prof, desc->l, desc->m, dbl, 1.0, nullptr, out));
+    } else if (desc->type >= HERMES_WIN_RING && desc->axis == 3) {
+        const int L = 1 << J;
+        const unsigned nb = hermes_blocks((int64_t)L * L * L, 256, 65536);
+        if (dbl) k_build_full_general<double><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (double*)out);
+        else k_build_full_general<float><<<nb, 256, 0, ctx->stream>>>(L, P, *desc, (float*)out);
+        HERMES_LAUNCH_CHECK();
+    } else {
+        HERMES_CHECK_HIP(launch_build_full(ctx, J, 0, P, *desc, prof, 0, 0, dbl, 1.0, nullptr, out));
+    }
     return 0;
 }
 
@@ -705,15 +801,20 @@ int hermes_window_build_full_profile(hermes_ctx* ctx, int J, const double* P, co
     HERMES_REQUIRE(l >= 0 && l <= 40 && m >= -l && m <= l, "invalid multipole (l=%d, m=%d)", l, m);
     if (int rc = check_profile(*prof, l, "hermes_window_build_full_profile")) return rc;
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
-    const int L = 1 << J;
-    const int64_t n = (int64_t)L * L * L;
-    if (dbl)
-        k_build_full_profile<double><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *prof, l, m,
-                                                                                              (double*)out);
-    else
-        k_build_full_profile<float><<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(L, P, *prof, l, m,
-                                                                                             (float*)out);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(launch_build_full(ctx, J, prof->kind == HERMES_RADIAL_SHELL ? 1 : 2, P, hermes_window_desc{}, *prof,
+                                       l, m, dbl, 1.0, nullptr, out));
+    return 0;
+}
+
+int hermes_window_apply_full_f64(hermes_ctx* ctx, int J, const double* P, const hermes_radial_profile* prof, int l,
+                                 int m, double scale, const void* spec, void* out) {
+    HERMES_REQUIRE(ctx && P && prof && spec && out && spec != out, "hermes_window_apply_full_f64: invalid argument");
+    HERMES_REQUIRE(J >= 1 && J <= 10, "J=%d unsupported", J);
+    HERMES_REQUIRE(l >= 0 && l <= 40 && m >= -l && m <= l, "invalid multipole (l=%d, m=%d)", l, m);
+    if (int rc = check_profile(*prof, l, "hermes_window_apply_full_f64")) return rc;
+    HERMES_CHECK_HIP(hipSetDevice(ctx->device));
+    HERMES_CHECK_HIP(launch_build_full(ctx, J, prof->kind == HERMES_RADIAL_SHELL ? 1 : 2, P, hermes_window_desc{}, *prof,
+                                       l, m, 1, scale, (const double2*)spec, out));
     return 0;
 }
 

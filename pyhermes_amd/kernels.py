@@ -200,6 +200,17 @@ def window_build_full_profile(J, P, prof, l, m, dbl=True):
     return out
 
 
+def window_apply_full_f64(spec, P, prof, l, m, scale, out):
+    """out = spec * K * scale for the window of window_build_full_profile, K not stored (complex128 spectra)."""
+    L = spec.shape[0]
+    for t in (spec, out):
+        if t.dtype != torch.complex128 or tuple(t.shape) != (L, L, L) or not t.is_contiguous():
+            raise ValueError("window_apply_full_f64 needs contiguous complex128 (L, L, L) tensors")
+    _lib.call("hermes_window_apply_full_f64", _lib.context(), _J_of(L), ptr(P), ctypes_byref(prof), int(l), int(m),
+              float(scale), ptr(spec), ptr(out))
+    return out
+
+
 def multipole_window_ifft_profiles_f32(H, P, profiles, l, ms, scale, out):
     """multipole_window_ifft_multi_f32 with a radial profile per shell (``profiles``: RadialProfile list)."""
     S = len(profiles)

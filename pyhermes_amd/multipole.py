@@ -4,8 +4,8 @@ Two paths compute ``ddd_l`` for shell pairs (r12, r13):
 
 * ``ddd_multipole_plain_f64`` -- a per-set restatement of calc_DDD_multipole
   (corr3pcf_multipoles.py:460-579) on the GPU in FP64: for every (l, m >= 0) two
-  window builds, two forward and two inverse complex FFTs and the FP64
-  contraction, exactly as the reference sequences them.
+  windows applied to the field's transform, two inverse complex FFTs and the FP64
+  contraction, in the reference's order.
 * ``ddd_multipole_batched_f32`` -- all shell pairs at once: one real FFT per
   field, then per (l, m) one fused window + inverse-FFT call producing every
   shell's field (window, z pass, y and x passes) and one MFMA Gram contraction
@@ -49,36 +49,36 @@ def combine_m_terms(v_re_by_m, l):
 
 
 # ---------------------------------------------------------------- plain FP64
-def _multipole_field_f64(geo, delta_c, edge, l, m):
-    """field @ radial_multipole window (complex_full_fft), FP64: fftn -> x K -> ifftn.  ``edge``: a thin-shell
-    radius in grid units or an EdgeProfile."""
-    if isinstance(edge, EdgeProfile):
-        K = edge.window_full(geo.J, geo.P, l, m, dbl=True)
-    else:
-        K = kernels.window_build_full(geo.J, geo.P, kernels.window_desc("shell_multipole", edge, l=l, m=m), dbl=True)
-    spec = kernels.fftn_c2c(delta_c)
-    kernels.spectrum_mul(spec, K, 1.0 / geo.L ** 3)
-    del K
-    kernels.fftn_c2c(spec, inverse=True, out=spec)
-    return spec
+def _multipole_field_f64(geo, spec, edge, l, m, out):
+    """ifftn(spec x K) of the radial_multipole window K, FP64, in ``out``.  ``edge``: a thin-shell radius in grid
+    units or an EdgeProfile."""
+    prof = edge.profile(l) if isinstance(edge, EdgeProfile) else kernels.radial_profile("shell", edge)
+    kernels.window_apply_full_f64(spec, geo.P, prof, l, m, 1.0 / geo.L ** 3, out)
+    return kernels.fftn_c2c(out, inverse=True, out=out)
+
+
+def _full_spectrum_f64(d):
+    c = torch.complex(d, torch.zeros_like(d))
+    return kernels.fftn_c2c(c, out=c)
 
 
 def ddd_multipole_plain_f64(geo, d1, d2, d3, R12_grid, R13_grid, l_min, l_max, return_m_values=False,
                             progress=None):
-    """One (r12, r13) set, every (l, m) recomputed from scratch as the reference does.  d*: (L,L,L) float64."""
+    """One (r12, r13) set in FP64, term by term as the reference sequences it; the fields are transformed once per
+    call.  d*: (L,L,L) float64."""
     N = geo.L ** 3
-    d2c = torch.complex(d2, torch.zeros_like(d2))
-    d3c = d2c if d3 is d2 else torch.complex(d3, torch.zeros_like(d3))
+    spec2 = _full_spectrum_f64(d2)
+    spec3 = spec2 if d3 is d2 else _full_spectrum_f64(d3)
+    F1, F2 = torch.empty_like(spec2), torch.empty_like(spec2)
     out = []
     mvals = {}
     for l in range(l_min, l_max + 1):
         vm = np.empty(l + 1, dtype=np.complex128)
         for m in range(l + 1):
-            F1 = _multipole_field_f64(geo, d2c, R12_grid, l, m)
-            F2 = _multipole_field_f64(geo, d3c, R13_grid, l, -m)
+            _multipole_field_f64(geo, spec2, R12_grid, l, m, F1)
+            _multipole_field_f64(geo, spec3, R13_grid, l, -m, F2)
             raw = kernels.multipole_summand_f64(d1, F1, F2, geo.gamma)
             vm[m] = 4.0 * np.pi * raw / N
-            del F1, F2
         mvals[l] = vm
         out.append(combine_m_terms([v.real for v in vm], l))
         if progress is not None:
