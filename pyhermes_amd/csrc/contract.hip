@@ -15,6 +15,7 @@
 // given as (V.re, -V.im).
 #include "../../include/hermes_amd.h"
 #include "hermes_common.h"
+#include "reduce.h"
 
 namespace {
 
@@ -176,45 +177,6 @@ __global__ __launch_bounds__(SUM_THREADS, 2) void k_summand_f64(int L, int tz, i
         for (int w = 0; w < SUM_THREADS / 64; ++w) t += sh[threadIdx.x][w];
         partial[2 * (blockIdx.y * gridDim.x + blockIdx.x) + threadIdx.x] = t;
     }
-}
-
-// Column sums of a row-major (nb x width) FP64 array, width a divisor of RED_THREADS.  Block b
-// sums rows [b * rows_per_block, (b + 1) * rows_per_block) in a fixed order (thread phase p takes
-// rows p, p + phases, ...; phases are then added in index order), so results are run-to-run identical.
-constexpr int RED_THREADS = 256;
-
-__global__ __launch_bounds__(RED_THREADS) void k_sum_rows(const double* __restrict__ in, int64_t nb, int width,
-                                                          int64_t stride, int64_t rows_per_block,
-                                                          double* __restrict__ out) {
-    __shared__ double sh[RED_THREADS];
-    const int phases = RED_THREADS / width;
-    const int j = threadIdx.x % width, ph = threadIdx.x / width;
-    const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
-    const int64_t r1 = r0 + rows_per_block < nb ? r0 + rows_per_block : nb;
-    double t = 0.0;
-    if (ph < phases)
-        for (int64_t r = r0 + ph; r < r1; r += phases) t += in[r * stride + j];
-    sh[threadIdx.x] = t;
-    __syncthreads();
-    if (threadIdx.x < width) {
-        double s = 0.0;
-        for (int p = 0; p < phases; ++p) s += sh[p * width + threadIdx.x];
-        out[(int64_t)blockIdx.x * width + threadIdx.x] = s;
-    }
-}
-
-constexpr int RED_MAX_BLOCKS = 1024;
-
-// Two launches: <= RED_MAX_BLOCKS partial rows, then one row.  tmp holds RED_MAX_BLOCKS * width doubles.
-// Column sums of nb rows (width <= RED_THREADS columns, rows stride apart) in a fixed order.
-static void sum_rows(hipStream_t st, const double* in, int64_t nb, int width, double* tmp, double* out,
-                     int64_t stride = 0) {
-    if (stride == 0) stride = width;
-    int64_t rpb = (nb + RED_MAX_BLOCKS - 1) / RED_MAX_BLOCKS;
-    if (rpb < 16) rpb = 16;
-    const int64_t nblk = (nb + rpb - 1) / rpb;
-    k_sum_rows<<<(unsigned)nblk, RED_THREADS, 0, st>>>(in, nb, width, stride, rpb, tmp);
-    k_sum_rows<<<1, RED_THREADS, 0, st>>>(tmp, nblk, width, width, nblk, out);
 }
 
 // ---------------------------------------------------------------- batched FP32 MFMA Gram
@@ -684,15 +646,14 @@ int hermes_multipole_summand_f64(hermes_ctx* ctx, int J, const double* d1, const
     int xseg = L < 64 ? L : 64;
     while (xseg > 4 && nyz * (L / xseg) < 1024) xseg /= 2;
     const int nb = nyz * (L / xseg);
-    double* ws = (double*)hermes_workspace(ctx, WS_CONTRACT, sizeof(double) * (2 * (size_t)nb + 2 + 2 * RED_MAX_BLOCKS));
+    double* ws = (double*)hermes_workspace(ctx, WS_CONTRACT, sizeof(double) * (2 * (size_t)nb + 2 + 2 * (size_t)hermes_reduce::sum_scratch_rows(nb)));
     HERMES_REQUIRE(ws, "%s", hermes_last_error());
     Gamma3 G;
     for (int i = 0; i < 9; ++i) G.g[i] = gamma3x3_host[i];
     k_summand_f64<<<dim3(nyz, L / xseg), SUM_THREADS, 0, ctx->stream>>>(L, tz, ty, xseg, d1, (const double2*)F1,
                                                                        (const double2*)F2, G, ws);
     HERMES_LAUNCH_CHECK();
-    sum_rows(ctx->stream, ws, nb, 2, ws + 2 * nb + 2, ws + 2 * nb);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, 2, nb, 2, ws + 2 * nb + 2, ws + 2 * nb));
     HERMES_CHECK_HIP(hipMemcpyAsync(out_host, ws + 2 * nb, sizeof(double) * 2, hipMemcpyDeviceToHost, ctx->stream));
     HERMES_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     return 0;
@@ -767,7 +728,7 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
     HERMES_REQUIRE(!split || !g.cross, "hermes_multipole_gram_f32: split sums are for the auto Gram");
     const int row = split ? 512 : 256;
     double* ws = (double*)hermes_workspace(
-        ctx, WS_CONTRACT, sizeof(double) * ((size_t)nblocks * row + row + (size_t)RED_MAX_BLOCKS * row));
+        ctx, WS_CONTRACT, sizeof(double) * ((size_t)nblocks * row + (size_t)hermes_reduce::sum_scratch_rows(nblocks) * row));
     HERMES_REQUIRE(ws, "%s", hermes_last_error());
     const bool timed = ctx->time_gram && !ctx->capturing;
     size_t slot = 0;
@@ -799,10 +760,7 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
         HERMES_CHECK_HIP(hipEventRecord(ctx->gram_ev[slot + 1], ctx->stream));
         ctx->gram_pending += 1;
     }
-    double* tmp = ws + (size_t)nblocks * row + row;
-    sum_rows(ctx->stream, ws, nblocks, 256, tmp, out_dev, row);
-    if (split) sum_rows(ctx->stream, ws + 256, nblocks, 256, tmp, out_dev + 256, row);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, row, nblocks, row, ws + (size_t)nblocks * row, out_dev));
     if (gout) *gout = g;
     return 0;
 }

@@ -15,6 +15,7 @@
 //   the stable per-bucket list of sub-cells the sampler draws from.
 #include "../../include/hermes_amd.h"
 #include "hermes_common.h"
+#include "reduce.h"
 
 #include <cmath>
 
@@ -121,14 +122,6 @@ __global__ __launch_bounds__(MC_THREADS) void k_triplet_box(double R1, double R2
         double t = 0.0;
         for (int w = 0; w < MC_THREADS / 64; ++w) t += sh[w];
         partial[blockIdx.x] = t;
-    }
-}
-
-__global__ void k_sum_1(const double* __restrict__ partial, int nb, double* __restrict__ out) {
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < nb; ++i) t += partial[i];
-        out[0] = t;
     }
 }
 
@@ -533,8 +526,7 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     k_triplet_box<<<nb, MC_THREADS, 0, ctx->stream>>>(R1, R2, mu, spos, n1, n, n_rot, d_abc, g2, g3, phi, 1 << J,
                                                       phi_res, ws);
     HERMES_LAUNCH_CHECK();
-    k_sum_1<<<1, 64, 0, ctx->stream>>>(ws, nb, ws + nb);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, 1, nb, 1, nullptr, ws + nb));
     double s = 0.0;
     HERMES_CHECK_HIP(hipMemcpyAsync(&s, ws + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HERMES_CHECK_HIP(hipStreamSynchronize(ctx->stream));

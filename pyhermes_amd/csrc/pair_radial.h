@@ -304,27 +304,4 @@ __global__ __launch_bounds__(radial_threads<BT>()) void k_pair_radial(int L, con
     }
 }
 
-// Column sums of `rows` rows of n doubles in a fixed order: 8 columns and 32 phases (rows ph, ph + 32, ...)
-// per workgroup, the phases added in order.  (One thread per group of 64 rows and then one per column took
-// 20 + 6 us for 1073 rows of 20: a serial chain of loads.)
-constexpr int SUM_COLS = 8, SUM_PHASES = 32;
-__global__ __launch_bounds__(SUM_COLS* SUM_PHASES) void k_sum_columns(const double* __restrict__ partial, int rows,
-                                                                      int n, double* __restrict__ out) {
-    __shared__ double sh[SUM_COLS * SUM_PHASES];
-    const int c = blockIdx.x * SUM_COLS + threadIdx.x % SUM_COLS, ph = threadIdx.x / SUM_COLS;
-    double s = 0.0;
-    if (c < n) {
-#pragma unroll 8
-        for (int r = ph; r < rows; r += SUM_PHASES) s += partial[(int64_t)r * n + c];
-    }
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < SUM_COLS && c < n) {
-        double t = 0.0;
-#pragma unroll
-        for (int p = 0; p < SUM_PHASES; ++p) t += sh[p * SUM_COLS + threadIdx.x];
-        out[c] = t;
-    }
-}
-
 }  // namespace hermes_pair

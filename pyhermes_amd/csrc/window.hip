@@ -7,6 +7,7 @@
 #include "hermes_common.h"
 #include "pair_los.h"
 #include "pair_radial.h"
+#include "reduce.h"
 #include "special.h"
 
 #include <algorithm>
@@ -653,14 +654,6 @@ __global__ __launch_bounds__(RED_THREADS) void k_reduce_sum(const T* __restrict_
     }
 }
 
-__global__ void k_reduce_final(const double* __restrict__ partial, int nb, double* __restrict__ out) {
-    if (threadIdx.x < 2) {
-        double t = 0.0;
-        for (int i = 0; i < nb; ++i) t += partial[2 * i + threadIdx.x];
-        out[threadIdx.x] = t;
-    }
-}
-
 int check_desc(const hermes_window_desc& d) {
     if (d.type < 0 || d.type > HERMES_WIN_CYLINDER) {
         hermes_set_error("unknown window type %d", d.type);
@@ -940,10 +933,9 @@ static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int rows
     return e != hipSuccess ? e : hipGetLastError();
 }
 
+// Pair reductions have at most 2048 rows of partial sums: one launch, no scratch.
 static hipError_t sum_columns(hipStream_t st, const double* partial, int rows, int n, double* out) {
-    using namespace hermes_pair;
-    k_sum_columns<<<(n + SUM_COLS - 1) / SUM_COLS, SUM_COLS * SUM_PHASES, 0, st>>>(partial, rows, n, out);
-    return hipGetLastError();
+    return hermes_reduce::sum_columns(st, partial, n, rows, n, nullptr, out);
 }
 
 // Scratch of the pair reduction: the context's grow-only slot, or, for the allocation-free entry point, a
@@ -1447,8 +1439,7 @@ int hermes_reduce_sum(hermes_ctx* ctx, const void* x, int64_t n, int ncomp, int 
     if (dbl) k_reduce_sum<double><<<nb, RED_THREADS, 0, ctx->stream>>>((const double*)x, n, ncomp, ws);
     else k_reduce_sum<float><<<nb, RED_THREADS, 0, ctx->stream>>>((const float*)x, n, ncomp, ws);
     HERMES_LAUNCH_CHECK();
-    k_reduce_final<<<1, 64, 0, ctx->stream>>>(ws, nb, ws + 2 * nb);
-    HERMES_LAUNCH_CHECK();
+    HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, 2, nb, 2, nullptr, ws + 2 * nb));
     double h[2];
     HERMES_CHECK_HIP(hipMemcpyAsync(h, ws + 2 * nb, sizeof(double) * 2, hipMemcpyDeviceToHost, ctx->stream));
     HERMES_CHECK_HIP(hipStreamSynchronize(ctx->stream));
