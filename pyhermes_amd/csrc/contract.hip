@@ -5,14 +5,12 @@
 //   S = sum_x d1[x] sum_{l1} F1[x-l1] sum_{l2} G3(l1,l2) F2[x-l2]   (complex128)
 // fused with a deterministic FP64 reduction.
 //
-// Batched FP32 path (MFMA): with Gamma = Q diag(lam) Q^T,
-//   sum_{l1,l2} G3(l1,l2) U[x-l1] V[x-l2] = sum_{abc} lam_abc U~_abc[x] V~_abc[x],
-// U~_abc = separable 3-tap filter of U with Q's columns.  For 16 shells at once
-//   G[s1][s2] = sum_x d1[x] sum_{abc,comp} lam_abc U~_{s1,abc,comp}[x] V~_{s2,abc,comp}[x]
-// is a 16 x 16 Gram matrix accumulated with v_mfma_f32_16x16x4f32 (lane = shell
-// x cell), flushed to FP64 after every x plane; per-workgroup FP64 partials are
-// summed in fixed order.  comp runs over (re, im) so G = Re(U V) sums when V is
-// given as (V.re, -V.im).
+// Batched FP32 path (MFMA): for up to 16 x 16 shells at once
+//   G[s1][s2] = sum_x d1[x] sum_{l1,l2} G3(l1,l2) Re(U_s1[x-l1] W_s2[x-l2])
+// as a 16 x 16 Gram matrix accumulated with v_mfma_f32_16x16x4f32 (lane = shell x cell); with
+// Gamma = Q diag(lam) Q^T the y stencil is an eigen-filter on the fields, the x and z stencils sit on d1 (see
+// k_gram_auto, k_gram_cross).  FP32 sums go to FP64 every few planes; per-workgroup FP64 partials are summed in
+// fixed order.
 #include "../../include/hermes_amd.h"
 #include "hermes_common.h"
 #include "reduce.h"
@@ -184,155 +182,11 @@ struct GramArgs {
     int L, S1, S2, cross, xseg;
     int xs, ys;       // element strides of x and y in the fields U, V (x-major: L^2, L; y-major: L, L^2)
     float vsign;      // sign applied to V's imaginary part in the cross case (-1: Re(U V))
-    float Q[9];       // Q[tap * 3 + col]
-    float lam[27];    // lam_a lam_b lam_c, index (a * 3 + b) * 3 + c
-    float lamyz[9];   // lam_b lam_c, index b * 3 + c (auto kernel)
-    float gx[9];      // Gamma[l1 * 3 + l2] = sum_a Q[l1][a] lam_a Q[l2][a] (auto kernel)
-    float Qs[9];      // auto kernel: Q[tap][col] sqrt|lam_col|, columns sorted by ascending lam
+    float gx[9];      // Gamma[l1 * 3 + l2] = sum_a Q[l1][a] lam_a Q[l2][a]
+    float Qs[9];      // Q[tap][col] sqrt|lam_col|, columns sorted by ascending lam
 };
 
-constexpr int GRAM_WAVES = 4;
-
 typedef float float4_t __attribute__((ext_vector_type(4)));
-
-// Raw values of field f at plane x around cell (y, z): raw[ly * 3 + lz] = f[x, y-ly, z-lz].
-__device__ __forceinline__ void load_plane(const float2* __restrict__ f, const GramArgs& g, int x, int y, int z,
-                                           float2 raw[9]) {
-    const int m = g.L - 1;
-#pragma unroll
-    for (int ly = 0; ly < 3; ++ly) {
-        const float2* row = f + (int64_t)x * g.xs + (int64_t)((y - ly) & m) * g.ys;
-#pragma unroll
-        for (int lz = 0; lz < 3; ++lz) raw[ly * 3 + lz] = row[(z - lz) & m];
-    }
-}
-
-// yz-filter: Y[b * 3 + c] = sum_{ly, lz} Q[ly][b] Q[lz][c] raw[ly * 3 + lz].
-__device__ __forceinline__ void filter_plane(const float2 raw[9], const float* Q, float2 Y[9]) {
-    float2 Z[3][3];  // Z[ly][c]
-#pragma unroll
-    for (int ly = 0; ly < 3; ++ly)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const float q0 = Q[0 * 3 + c], q1 = Q[1 * 3 + c], q2 = Q[2 * 3 + c];
-            const float2 u0 = raw[ly * 3 + 0], u1 = raw[ly * 3 + 1], u2 = raw[ly * 3 + 2];
-            Z[ly][c] = make_float2(q0 * u0.x + q1 * u1.x + q2 * u2.x, q0 * u0.y + q1 * u1.y + q2 * u2.y);
-        }
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        const float q0 = Q[0 * 3 + b], q1 = Q[1 * 3 + b], q2 = Q[2 * 3 + b];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            Y[b * 3 + c] = make_float2(q0 * Z[0][c].x + q1 * Z[1][c].x + q2 * Z[2][c].x,
-                                       q0 * Z[0][c].y + q1 * Z[1][c].y + q2 * Z[2][c].y);
-    }
-}
-
-// One x plane: x-filter of the three yz-filtered planes and 54 MFMA updates.
-template <bool CROSS>
-__device__ __forceinline__ void gram_plane(const float2 Yc[9], const float2 Y1[9], const float2 Y2[9],
-                                           const float2 Vc[9], const float2 V1[9], const float2 V2[9],
-                                           const float* Q, const float* lam, float dval, float vsign,
-                                           float4_t& accr, float4_t& acci) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float q0 = Q[0 * 3 + a], q1 = Q[1 * 3 + a], q2 = Q[2 * 3 + a];
-#pragma unroll
-        for (int bc = 0; bc < 9; ++bc) {
-            const float2 ut = make_float2(q0 * Yc[bc].x + q1 * Y1[bc].x + q2 * Y2[bc].x,
-                                          q0 * Yc[bc].y + q1 * Y1[bc].y + q2 * Y2[bc].y);
-            float2 vt;
-            if (CROSS)
-                vt = make_float2(q0 * Vc[bc].x + q1 * V1[bc].x + q2 * V2[bc].x,
-                                 vsign * (q0 * Vc[bc].y + q1 * V1[bc].y + q2 * V2[bc].y));
-            else
-                vt = ut;
-            const float dl = dval * lam[a * 9 + bc];
-            accr = __builtin_amdgcn_mfma_f32_16x16x4f32(dl * ut.x, vt.x, accr, 0, 0, 0);
-            acci = __builtin_amdgcn_mfma_f32_16x16x4f32(dl * ut.y, vt.y, acci, 0, 0, 0);
-        }
-    }
-}
-
-template <bool CROSS>
-__global__ __launch_bounds__(64 * GRAM_WAVES) void k_gram_f32(const float* __restrict__ d1,
-                                                              const float2* __restrict__ U,
-                                                              const float2* __restrict__ V, GramArgs g,
-                                                              double* __restrict__ partial) {
-    __shared__ double red[GRAM_WAVES][256];
-    const int L = g.L;
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    const int s = lane % 16, k = lane / 16;
-    const int nzg = L / 4, nyg = L / GRAM_WAVES;
-    const int zg = blockIdx.x % nzg;
-    const int yg = (blockIdx.x / nzg) % nyg;
-    const int xs = blockIdx.x / (nzg * nyg);
-    const int y = yg * GRAM_WAVES + wave;
-    const int z = zg * 4 + k;
-    const int x0 = xs * g.xseg, xend = x0 + g.xseg;
-    const int64_t N = (int64_t)L * L * L;
-    const bool ua = s < g.S1;
-    const bool vb = s < g.S2;
-    const float2* fu = U + (int64_t)(ua ? s : 0) * N;
-    const float2* fv = (CROSS ? V : U) + (int64_t)(vb ? s : 0) * N;
-    float Q[9], lam[27];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Q[i] = g.Q[i];
-#pragma unroll
-    for (int i = 0; i < 27; ++i) lam[i] = g.lam[i];
-    const float2 zero = make_float2(0.f, 0.f);
-
-    float2 rawU[9], rawV[9];
-    float2 P0[9], P1[9], P2[9], W0[9], W1[9], W2[9];
-    // warm-up: P1 = Y(x0-2), P2 = Y(x0-1)
-#pragma unroll
-    for (int i = 0; i < 9; ++i) { rawU[i] = zero; rawV[i] = zero; }
-    if (ua) load_plane(fu, g, (x0 - 2) & (L - 1), y, z, rawU);
-    if (CROSS && vb) load_plane(fv, g, (x0 - 2) & (L - 1), y, z, rawV);
-    filter_plane(rawU, Q, P1);
-    if (CROSS) filter_plane(rawV, Q, W1);
-    if (ua) load_plane(fu, g, (x0 - 1) & (L - 1), y, z, rawU);
-    if (CROSS && vb) load_plane(fv, g, (x0 - 1) & (L - 1), y, z, rawV);
-    filter_plane(rawU, Q, P2);
-    if (CROSS) filter_plane(rawV, Q, W2);
-    if (ua) load_plane(fu, g, x0, y, z, rawU);
-    if (CROSS && vb) load_plane(fv, g, x0, y, z, rawV);
-    float dnext = d1[((int64_t)x0 * L + y) * L + z];  // d at plane x, loaded one step ahead
-
-    double acc64[4] = {0.0, 0.0, 0.0, 0.0};
-    // each step: filter the prefetched plane x, prefetch plane x+1, then the MFMA work of plane x
-#define GRAM_STEP(CUR, PREV1, PREV2, WCUR, WPREV1, WPREV2)                                           \
-    if (x < xend) {                                                                                  \
-        filter_plane(rawU, Q, CUR);                                                                  \
-        if (CROSS) filter_plane(rawV, Q, WCUR);                                                      \
-        const float dval = dnext;                                                                    \
-        if (x + 1 < xend) {                                                                          \
-            if (ua) load_plane(fu, g, x + 1, y, z, rawU);                                            \
-            if (CROSS && vb) load_plane(fv, g, x + 1, y, z, rawV);                                   \
-            dnext = d1[((int64_t)(x + 1) * L + y) * L + z];                                          \
-        }                                                                                            \
-        float4_t accr = {0.f, 0.f, 0.f, 0.f}, acci = {0.f, 0.f, 0.f, 0.f};                           \
-        gram_plane<CROSS>(CUR, PREV1, PREV2, WCUR, WPREV1, WPREV2, Q, lam, dval, g.vsign, accr, acci); \
-        _Pragma("unroll") for (int j = 0; j < 4; ++j) acc64[j] += (double)accr[j] + (double)acci[j];  \
-        ++x;                                                                                         \
-    }
-    for (int x = x0; x < xend;) {
-        GRAM_STEP(P0, P2, P1, W0, W2, W1)
-        GRAM_STEP(P1, P0, P2, W1, W0, W2)
-        GRAM_STEP(P2, P1, P0, W2, W1, W0)
-    }
-#undef GRAM_STEP
-    // lane holds G[4*(lane/16) + j][lane % 16]
-#pragma unroll
-    for (int j = 0; j < 4; ++j) red[wave][(4 * (lane / 16) + j) * 16 + (lane % 16)] = acc64[j];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-        double t = 0.0;
-#pragma unroll
-        for (int w = 0; w < GRAM_WAVES; ++w) t += red[w][i];
-        partial[(int64_t)blockIdx.x * 256 + i] = t;
-    }
-}
 
 // Auto Gram with the z-direction Gamma stencil also moved onto d1 (the y stencil stays on the fields as
 // the eigen-filter T_b(y) = sum_ly Qs[ly][b] F(y - ly), column b scaled by sqrt|lam_b|, sign s_b).  For the
@@ -354,13 +208,13 @@ __global__ __launch_bounds__(64 * GRAM_WAVES) void k_gram_f32(const float* __res
 // (and the MFMAs of plane p), y taps of plane p+3 from raw buffer (p+3)&1, store of staged plane p+4 into
 // raw buffer (p+4)&1, load of plane p+5 into registers.  A workgroup of 8 waves owns 2 (y) x 16 (z) cells
 // and 50 KB of LDS.
-// Tile geometry with TY rows of 16 cells: 4 TY waves (4 along z with 4 cells each, times TY rows).  The raw
+// Tile geometry with TY rows of TZ cells: a wave takes 4 cells along z.  The raw
 // tile keeps 16 shells per (row, z) position, the shell slot XOR-swizzled by z & 15 so that both the
 // z-fastest staging stores and the shell-fastest y-tap reads spread over the banks.
-template <int TY>
+template <int TY, int TZ_>
 struct D2Geom {
-    static constexpr int WAVES = 4 * TY, NROW = TY, TZ = 16;
-    static constexpr int RY = TY + 2, RZ = TZ + 4;   // raw rows y0-2 .. y0+TY-1, z z0-2 .. z0+17
+    static constexpr int NROW = TY, TZ = TZ_, WAVES = TY * TZ / 4;
+    static constexpr int RY = TY + 2, RZ = TZ + 4;   // raw rows y0-2 .. y0+TY-1, z z0-2 .. z0+TZ+1
     static constexpr int RP = 16;
     static constexpr int TILE = RY * RZ * RP;        // float2 per raw buffer
     static constexpr int TB = TY * RZ * 16;          // float2 per channel of a T buffer
@@ -373,7 +227,11 @@ struct D2Geom {
     static_assert((2 * TILE + 2 * TBUF) * 8 + WAVES * 256 * 8 <= 80 * 1024, "LDS of two workgroups per CU");
 };
 // 2 rows per workgroup: 8 waves and at most 66 KB of LDS, so two workgroups and four waves per SIMD
-using D2 = D2Geom<2>;
+using D2 = D2Geom<2, 16>;
+// the cross kernel: 4 waves and 39 KB; its 160 registers allow three waves per SIMD, so three workgroups per CU
+// (with 8 waves two per SIMD and one barrier for all: 540 us instead of 388 for 11 x 15 shells at L = 128; held to
+// 128 registers it spills 32: 874 us)
+using D2X = D2Geom<2, 8>;
 
 template <int NNEG, bool SPLIT = false>
 __global__ __launch_bounds__(64 * D2::WAVES, 4) void k_gram_auto(const float* __restrict__ d1,
@@ -620,6 +478,251 @@ __global__ __launch_bounds__(64 * D2::WAVES, 4) void k_gram_auto(const float* __
     }
 }
 
+// Cross Gram (U and V different fields, or different blocks of 16 shells of one field): the same form without the
+// symmetry, so the right operand of a cell has all 25 offsets delta = (dx, dz), |dx|, |dz| <= 2,
+//   G[a][b] = sum_{p, r} T^a(p, r) B^b(p, r),  B(p, r) = sum_delta C_delta(p, r) T_V(p + dx, r + dz),
+// and a y-filtered plane q of V serves the operands of five planes, q - 2 (dx = 2, then complete) .. q + 2.  The
+// left operand T^a needs the cell's own z only: each lane filters it from the raw U tile (no halo in z) when its
+// plane is complete.  250 VALU instructions and 6 matrix instructions per wave and plane, where the eigen form in
+// all three directions took 54 matrix instructions, about 600 VALU instructions and uncoalesced loads (each lane
+// read its shell's taps from memory).  Bound by VALU and LDS.  11 x 15 shells at L = 128: 1417 us before, 388 us now.
+// Step p (W = V): planes of V: p+2 into the operands, y taps of p+3, staged store of p+4, load of p+5; planes of U:
+// p finished, staged store of p+1, load of p+2.
+template <int NNEG>
+__global__ __launch_bounds__(64 * D2X::WAVES, 3) void k_gram_cross(const float* __restrict__ d1,
+                                                                  const float2* __restrict__ U,
+                                                                  const float2* __restrict__ V, GramArgs g,
+                                                                  double* __restrict__ partial) {
+    using GM = D2X;
+    constexpr int UT = GM::RY * GM::TZ * 16;  // raw U values per plane
+    __shared__ __align__(16) float2 smem[2 * GM::TILE + 2 * GM::TBUF];
+    __shared__ __align__(16) float2 useg[2][UT];
+    auto raw = [&](int q) -> float2* { return smem + (q & 1) * GM::TILE; };
+    auto tb = [&](int q) -> float2* { return smem + 2 * GM::TILE + (q & 1) * GM::TBUF; };
+    const int L = g.L, m = L - 1;
+    const int tid = threadIdx.x;
+    const int lane = tid % 64, wave = tid / 64;
+    const int s = lane % 16, k = lane / 16;
+    const int zw = wave % (GM::TZ / 4), yw = wave / (GM::TZ / 4);
+    const int nzb = L / GM::TZ, nyb = L / GM::NROW;
+    const int nb = nzb * nyb * (L / g.xseg);
+    const int q = (nb % 8 == 0) ? (int)(blockIdx.x % 8) * (nb / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    const int xs = q / (nzb * nyb);
+    const int rr = q % (nzb * nyb);
+    const int PZ = nzb < 16 ? nzb : 16;
+    const int zb = (rr / (PZ * nyb)) * PZ + (rr % (PZ * nyb)) % PZ;
+    const int yb = (rr % (PZ * nyb)) / PZ;
+    const int z0 = zb * GM::TZ, y0 = yb * GM::NROW;
+    const int x0 = xs * g.xseg, xend = x0 + g.xseg;
+    const int64_t N = (int64_t)L * L * L;
+    const int64_t LL = (int64_t)L * L;
+    const float* Q = g.Qs;
+    const float G00 = g.gx[0], G11 = g.gx[4], G22 = g.gx[8], G10 = g.gx[3], G21 = g.gx[7], G20 = g.gx[6];
+    const int cz = 4 * zw + k;
+    const int yrow = (y0 + yw) * L, zc = z0 + cz;
+
+    // staging: SHT threads per shell, positions z fastest
+    constexpr int SHT = 4 * GM::WAVES;
+    constexpr int VP = GM::RY * GM::RZ, UP = GM::RY * GM::TZ;  // positions per shell
+    constexpr int VPT = (VP + SHT - 1) / SHT, UPT = UP / SHT;
+    const int sh = tid / SHT, sj = tid % SHT;
+    const float2* vbase = V + (int64_t)(sh < g.S2 ? sh : 0) * N;
+    const float2* ubase = U + (int64_t)(sh < g.S1 ? sh : 0) * N;
+    int voff[VPT], uoff[UPT];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int e = sj + SHT * i < VP ? sj + SHT * i : 0, ry = e / GM::RZ, rz = e % GM::RZ;
+        voff[i] = ((y0 - 2 + ry) & m) * g.ys + ((z0 - 2 + rz) & m);
+    }
+#pragma unroll
+    for (int i = 0; i < UPT; ++i) {
+        const int e = sj + SHT * i;
+        uoff[i] = ((y0 - 2 + e / GM::TZ) & m) * g.ys + ((z0 + e % GM::TZ) & m);
+    }
+    float2 vst[VPT], ust[UPT];
+    auto vload = [&](int plane) {
+        const float2* p = vbase + (int64_t)(plane & m) * g.xs;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i)
+            if (sj + SHT * i < VP) vst[i] = p[voff[i]];
+    };
+    auto vstore = [&](int plane) {
+        float2* t = raw(plane);
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int e = sj + SHT * i, rz = e % GM::RZ;
+            if (e < VP) t[e * GM::RP + (sh ^ (rz & 15))] = vst[i];
+        }
+    };
+    auto uload = [&](int plane) {
+        const float2* p = ubase + (int64_t)(plane & m) * g.xs;
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) ust[i] = p[uoff[i]];
+    };
+    auto ustore = [&](int plane) {
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) {
+            const int e = sj + SHT * i;
+            useg[plane & 1][e * 16 + (sh ^ (e % GM::TZ))] = ust[i];
+        }
+    };
+    int traw[GM::TPT];
+    bool tact[GM::TPT];
+#pragma unroll
+    for (int i = 0; i < GM::TPT; ++i) {
+        const int u = tid + i * 64 * GM::WAVES;
+        tact[i] = u < GM::TB;
+        const int uu = tact[i] ? u : 0;
+        const int ts = uu % 16, zp = (uu / 16) % GM::RZ, row = uu / (16 * GM::RZ);
+        traw[i] = ((row + 2) * GM::RZ + zp) * GM::RP + (ts ^ (zp & 15));
+    }
+    auto tphase = [&](int plane) {
+        const float2* rw = raw(plane);
+        float2* t = tb(plane);
+#pragma unroll
+        for (int i = 0; i < GM::TPT; ++i) {
+            if (!tact[i]) continue;
+            const float2 r0 = rw[traw[i]];
+            const float2 r1 = rw[traw[i] - GM::RZ * GM::RP];
+            const float2 r2 = rw[traw[i] - 2 * GM::RZ * GM::RP];
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                const float q0 = Q[0 * 3 + b], q1 = Q[1 * 3 + b], q2 = Q[2 * 3 + b];
+                t[b * GM::TB + tid + i * 64 * GM::WAVES] =
+                    make_float2(q0 * r0.x + q1 * r1.x + q2 * r2.x, q0 * r0.y + q1 * r1.y + q2 * r2.y);
+            }
+        }
+    };
+    auto efun = [&](const float dd[3], float E[5]) {
+        E[0] = G20 * dd[0];
+        E[1] = G10 * dd[0] + G21 * dd[1];
+        E[2] = G00 * dd[0] + G11 * dd[1] + G22 * dd[2];
+        E[3] = G10 * dd[1] + G21 * dd[2];
+        E[4] = G20 * dd[2];
+    };
+    auto dload = [&](int plane, float dd[3]) {
+        const float* dp = d1 + (int64_t)(plane & m) * LL;
+        dd[0] = dp[yrow + (zc & m)];
+        dd[1] = dp[yrow + ((zc + 1) & m)];
+        dd[2] = dp[yrow + ((zc + 2) & m)];
+    };
+    const int tme = (yw * GM::RZ + cz + 2) * 16 + s;  // this lane's T index at dz = 0 (channel 0)
+    const int ume = ((yw + 2) * GM::TZ + cz) * 16 + (s ^ cz);
+
+    double acc_slot[4] = {0.0, 0.0, 0.0, 0.0};
+    // warm-up: T of plane x0 - 2, raw plane x0 - 1, staged plane x0 of V (the loop starts at p = x0 - 4; its first
+    // four steps only fill operands); E of planes x0 - 2, x0 - 1, d of plane x0
+    float E0[5], E1[5], E2[5], dn[3];
+    float2 B0[3], B1[3], B2[3], B3[3], B4[3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) B0[b] = B1[b] = B2[b] = B3[b] = B4[b] = make_float2(0.f, 0.f);
+    vload(x0 - 2);
+    vstore(x0 - 2);
+    vload(x0 - 1);
+    dload(x0 - 2, dn);
+    efun(dn, E0);
+    dload(x0 - 1, dn);
+    efun(dn, E1);
+    dload(x0, dn);
+    __syncthreads();
+    tphase(x0 - 2);
+    vstore(x0 - 1);
+    vload(x0);
+    uload(x0 - 3);
+    float4_t accr = {0.f, 0.f, 0.f, 0.f};
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const bool lead = ((wv >> 2) ^ wv) & 1;
+    // step p: slots S0 .. S4 hold planes p .. p+4; EA = E(p+2), EB = E(p+3), EF = E(p+4) (computed now)
+#define CROSS_STEP(S0, S1, S2, S3, S4, EA, EB, EF)                                                  \
+    if (p < xend) {                                                                                 \
+        __syncthreads();                                                                            \
+        efun(dn, EF);                                                                               \
+        dload(p + 5, dn);                                                                           \
+        if (lead) {                                                                                 \
+            tphase(p + 3);                                                                          \
+            vstore(p + 4);                                                                          \
+            vload(p + 5);                                                                           \
+            ustore(p + 1);                                                                          \
+            uload(p + 2);                                                                           \
+        }                                                                                           \
+        const float2* t = tb(p + 2) + tme;                                                          \
+        _Pragma("unroll") for (int j = 0; j < 5; ++j) {                                             \
+            const float c2 = G20 * EA[j], c1 = G10 * EA[j] + G21 * EB[j];                           \
+            const float c0 = G00 * EA[j] + G11 * EB[j] + G22 * EF[j];                               \
+            const float m1 = G10 * EB[j] + G21 * EF[j], m2 = G20 * EF[j];                           \
+            _Pragma("unroll") for (int b = 0; b < 3; ++b) {                                         \
+                const float2 w = t[b * GM::TB + (j - 2) * 16];                                      \
+                const float sg = b < NNEG ? -1.0f : 1.0f;                                           \
+                S0[b].x = (sg * c2) * w.x + S0[b].x;                                          \
+                S0[b].y = (sg * c2) * w.y + S0[b].y;                                          \
+                S1[b].x = (sg * c1) * w.x + S1[b].x;                                          \
+                S1[b].y = (sg * c1) * w.y + S1[b].y;                                          \
+                S2[b].x = (sg * c0) * w.x + S2[b].x;                                          \
+                S2[b].y = (sg * c0) * w.y + S2[b].y;                                          \
+                S3[b].x = (sg * m1) * w.x + S3[b].x;                                          \
+                S3[b].y = (sg * m1) * w.y + S3[b].y;                                          \
+                S4[b].x = j ? (sg * m2) * w.x + S4[b].x : (sg * m2) * w.x;              \
+                S4[b].y = j ? (sg * m2) * w.y + S4[b].y : (sg * m2) * w.y;              \
+            }                                                                                       \
+        }                                                                                           \
+        if (p >= x0) {                                                                              \
+            const float2 r0 = useg[p & 1][ume], r1 = useg[p & 1][ume - GM::TZ * 16];                \
+            const float2 r2 = useg[p & 1][ume - 2 * GM::TZ * 16];                                   \
+            _Pragma("unroll") for (int b = 0; b < 3; ++b) {                                         \
+                const float q0 = Q[0 * 3 + b], q1 = Q[1 * 3 + b], q2 = Q[2 * 3 + b];                \
+                const float ax = q0 * r0.x + q1 * r1.x + q2 * r2.x;                                 \
+                const float ay = g.vsign * (q0 * r0.y + q1 * r1.y + q2 * r2.y);                     \
+                accr = __builtin_amdgcn_mfma_f32_16x16x4f32(ax, S0[b].x, accr, 0, 0, 0);            \
+                accr = __builtin_amdgcn_mfma_f32_16x16x4f32(ay, S0[b].y, accr, 0, 0, 0);            \
+            }                                                                                       \
+        }                                                                                           \
+        if (!lead) {                                                                                \
+            tphase(p + 3);                                                                          \
+            vstore(p + 4);                                                                          \
+            vload(p + 5);                                                                           \
+            ustore(p + 1);                                                                          \
+            uload(p + 2);                                                                           \
+        }                                                                                           \
+        if ((p - x0) % 6 == 5 || p + 1 >= xend) { /* at most six planes in FP32 */                  \
+            _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                         \
+                acc_slot[j] += (double)accr[j];                                                     \
+                accr[j] = 0.f;                                                                      \
+            }                                                                                       \
+        }                                                                                           \
+        ++p;                                                                                        \
+    }
+    int p = x0 - 4;
+    while (p < xend) {  // 15 steps: the operand slots turn by five, the E planes by three
+        CROSS_STEP(B0, B1, B2, B3, B4, E0, E1, E2)
+        CROSS_STEP(B1, B2, B3, B4, B0, E1, E2, E0)
+        CROSS_STEP(B2, B3, B4, B0, B1, E2, E0, E1)
+        CROSS_STEP(B3, B4, B0, B1, B2, E0, E1, E2)
+        CROSS_STEP(B4, B0, B1, B2, B3, E1, E2, E0)
+        CROSS_STEP(B0, B1, B2, B3, B4, E2, E0, E1)
+        CROSS_STEP(B1, B2, B3, B4, B0, E0, E1, E2)
+        CROSS_STEP(B2, B3, B4, B0, B1, E1, E2, E0)
+        CROSS_STEP(B3, B4, B0, B1, B2, E2, E0, E1)
+        CROSS_STEP(B4, B0, B1, B2, B3, E0, E1, E2)
+        CROSS_STEP(B0, B1, B2, B3, B4, E1, E2, E0)
+        CROSS_STEP(B1, B2, B3, B4, B0, E2, E0, E1)
+        CROSS_STEP(B2, B3, B4, B0, B1, E0, E1, E2)
+        CROSS_STEP(B3, B4, B0, B1, B2, E1, E2, E0)
+        CROSS_STEP(B4, B0, B1, B2, B3, E2, E0, E1)
+    }
+#undef CROSS_STEP
+    double* red = (double*)smem;  // [GM::WAVES][256]
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) red[wave * 256 + (4 * (lane / 16) + j) * 16 + (lane % 16)] = acc_slot[j];
+    __syncthreads();
+    for (int i = tid; i < 256; i += 64 * GM::WAVES) {
+        double tsum = 0.0;
+#pragma unroll
+        for (int w = 0; w < GM::WAVES; ++w) tsum += red[w * 256 + i];
+        partial[(int64_t)blockIdx.x * 256 + i] = tsum;
+    }
+}
+
 // Lane-layout self check of the 16x16x4 FP32 MFMA: C = A B for A[m][k] = m + 16 k,
 // B[k][n] = (k + 1) * (n - 7).
 __global__ void k_mfma_selftest(float* out) {
@@ -692,17 +795,14 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
     g.cross = V != nullptr;
     g.S2 = g.cross ? n_v : n_u;
     g.vsign = v_conj ? 1.0f : -1.0f;  // Re(U V) needs -V.im, Re(U conj V) needs +V.im
-    // planes per workgroup: the auto kernel's warm-up (two planes filtered ahead) and its final reduction
-    // are paid once per segment, so it takes 512 planes (8192 workgroups at L = 512, 16 per workgroup slot;
-    // 256- and 128-plane segments measured 2% and 3% slower)
-    const int seg = g.cross ? 64 : 512;
-    g.xseg = L < seg ? L : seg;
-    for (int i = 0; i < 9; ++i) g.Q[i] = (float)Q3x3_host[i];
-    for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b)
-            for (int c = 0; c < 3; ++c) g.lam[(a * 3 + b) * 3 + c] = (float)(lam3_host[a] * lam3_host[b] * lam3_host[c]);
-    for (int b = 0; b < 3; ++b)
-        for (int c = 0; c < 3; ++c) g.lamyz[b * 3 + c] = (float)(lam3_host[b] * lam3_host[c]);
+    // planes per workgroup: each segment pays a warm-up of two (auto) or four (cross) planes and a final reduction,
+    // so it takes 512 planes (8192 workgroups at L = 512, 16 per workgroup slot; 256- and 128-plane segments
+    // measured 2% and 3% slower), and shorter ones, down to 8, where the columns alone do not give the 512
+    // workgroups that fill the chip (L = 64: 65 us with whole columns, 128 workgroups; 34 us with 16 planes)
+    const int ncol = g.cross ? (L / D2X::TZ) * (L / D2X::NROW) : (L / D2::TZ) * (L / D2::NROW);
+    const int fill = g.cross ? 2 * 768 : 512;  // cross: 768 slots, at least two rounds of them
+    g.xseg = L < 512 ? L : 512;
+    while (g.xseg > 8 && ncol * (L / g.xseg) < fill) g.xseg /= 2;
     for (int l1 = 0; l1 < 3; ++l1)
         for (int l2 = 0; l2 < 3; ++l2) {
             double t = 0.0;
@@ -721,10 +821,8 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
         if (lc < 0.0) ++nneg;
         for (int tap = 0; tap < 3; ++tap) g.Qs[tap * 3 + c] = (float)(Q3x3_host[tap * 3 + order[c]] * sqrt(fabs(lc)));
     }
-    // auto kernel: 16 z x 4 y cells per workgroup (needs L >= 16); cross kernel: 4 z x 4 y
     HERMES_REQUIRE(g.cross || J >= 4, "hermes_multipole_gram_f32: J=%d, the auto Gram needs J >= 4", J);
-    const int nblocks = g.cross ? (L / 4) * (L / GRAM_WAVES) * (L / g.xseg)
-                                : (L / D2::TZ) * (L / D2::NROW) * (L / g.xseg);
+    const int nblocks = ncol * (L / g.xseg);
     HERMES_REQUIRE(!split || !g.cross, "hermes_multipole_gram_f32: split sums are for the auto Gram");
     const int row = split ? 512 : 256;
     double* ws = (double*)hermes_workspace(
@@ -742,8 +840,14 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
         }
         HERMES_CHECK_HIP(hipEventRecord(ctx->gram_ev[slot], ctx->stream));
     }
+    const float2 *u = (const float2*)U, *v = (const float2*)V;
     if (g.cross)
-        k_gram_f32<true><<<nblocks, 64 * GRAM_WAVES, 0, ctx->stream>>>(d1, (const float2*)U, (const float2*)V, g, ws);
+        switch (nneg) {
+            case 0: k_gram_cross<0><<<nblocks, 64 * D2X::WAVES, 0, ctx->stream>>>(d1, u, v, g, ws); break;
+            case 1: k_gram_cross<1><<<nblocks, 64 * D2X::WAVES, 0, ctx->stream>>>(d1, u, v, g, ws); break;
+            case 2: k_gram_cross<2><<<nblocks, 64 * D2X::WAVES, 0, ctx->stream>>>(d1, u, v, g, ws); break;
+            default: k_gram_cross<3><<<nblocks, 64 * D2X::WAVES, 0, ctx->stream>>>(d1, u, v, g, ws); break;
+        }
     else
         switch (nneg + (split ? 4 : 0)) {
             case 0: k_gram_auto<0><<<nblocks, 64 * D2::WAVES, 0, ctx->stream>>>(d1, (const float2*)U, g, ws); break;
