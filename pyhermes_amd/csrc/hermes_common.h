@@ -16,7 +16,7 @@ enum hermes_ws_slot {
     WS_PROJ_TILE = 0,   // projection: per-tile counters / offsets
     WS_PROJ_REC = 1,    // projection: bucketed particle records
     WS_REDUCE = 2,      // reductions: per-block partial sums
-    WS_SPEC = 3,        // window / FFT staging
+    WS_SPEC = 3,        // Monte-Carlo sampler: bricked copies of the grids
     WS_MISC = 4,
     WS_MC = 5,
     WS_MLP = 6,

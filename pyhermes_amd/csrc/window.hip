@@ -304,6 +304,7 @@ constexpr int SHELL_CHUNK = 16;
 
 struct ApplyArgs {
     int L, l, m, n_shell;
+    int group;  // shells per workgroup of the fused window kernel
     float cnorm, scale;
     float sx, sy, sz;  // sign factors for x-, y- (1) and z-mirrors: (-1)^m, (-1)^(l+m)
     double radii_over_L[MAX_SHELLS];
@@ -322,7 +323,7 @@ struct MultiM {
 __device__ __forceinline__ float2 cmulf(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.y); }
 
-__global__ __launch_bounds__(256) void k_multipole_apply(const float2* __restrict__ H, const float* __restrict__ Pf,
+__global__ __launch_bounds__(256) void k_multipole_apply(const float2* __restrict__ H, const double* __restrict__ P,
                                                          ApplyArgs A, float2* __restrict__ out) {
     const int L = A.L, Lh = L / 2 + 1;
     const int64_t nrep = (int64_t)Lh * Lh * Lh;
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(256) void k_multipole_apply(const float2* __restric
 #pragma unroll
         for (int a = 0; a < 8; ++a) {
             int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
-            pw[a] = Pf[ax < 0 ? -ax : ax] * Pf[ay < 0 ? -ay : ay] * Pf[az < 0 ? -az : az];
+            pw[a] = (float)P[ax < 0 ? -ax : ax] * (float)P[ay < 0 ? -ay : ay] * (float)P[az < 0 ? -az : az];
             nrm[a] = sqrt((double)ax * ax + (double)ay * ay + (double)az * az);
             float2 yy = ylm_f32(A.l, A.m < 0 ? -A.m : A.m, (float)ax, (float)ay, (float)az, A.cnorm);
             if (A.m < 0) {  // Y_{l,-m} = (-1)^m conj(Y_{l,m})
@@ -395,7 +396,9 @@ __global__ __launch_bounds__(256) void k_multipole_apply(const float2* __restric
 // Fused multipole window and inverse z-FFT (FP32).  Workgroup (x, y), 0 <= x, y <= L/2, evaluates
 // K_{R_s,l,m} at its octant representatives (x, y, z <= L/2) exactly as k_multipole_apply does, forms
 // the four mirror lines (x, y), (xm, y), (x, ym), (xm, ym) of H_full * K * scale in LDS with the same
-// mirror rules, transforms them along z and writes each distinct line once.  Loops over shells.
+// mirror rules, transforms them along z and writes each distinct line once.  Loops over the shells of its group:
+// blockIdx.y splits them on small grids, where one workgroup per (x, y) leaves the SIMDs with a wave or less
+// (mpwin_groups; each group evaluates the alias weights again).
 
 // MP orders m of one l per launch: the radial factors j_l(2 pi |a| R_s) of the 8 aliases are
 // evaluated once per (representative, shell) and shared by the MP windows; the weights
@@ -416,7 +419,7 @@ constexpr int mpwin_threads() {
 // monopole) instead of j_l(2 pi |a| R_s / L); prof is unused otherwise.
 template <int LOG2L, int MP, bool PACK = false, bool PROF = false>
 __global__ __launch_bounds__(mpwin_threads<LOG2L>()) void k_mpwin_zfft_multi(
-    const float2* __restrict__ H, const float* __restrict__ Pf, ApplyArgs A, MultiM M,
+    const float2* __restrict__ H, const double* __restrict__ P, ApplyArgs A, MultiM M,
     const float2* __restrict__ twg, float2* __restrict__ out, const hermes_radial_profile* __restrict__ prof) {
     static_assert(!PACK || MP == 2, "packing needs two orders");
     static_assert(!(PACK && PROF), "packed pairs take thin shells only");
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(mpwin_threads<LOG2L>()) void k_mpwin_zfft_multi(
     // helper lanes, alias tid of the Nyquist plane
     auto weights = [&](int z, int a, float2* w, double& nrm, bool& live) {
         const int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
-        const float pw = Pf[ax < 0 ? -ax : ax] * Pf[ay < 0 ? -ay : ay] * Pf[az < 0 ? -az : az];
+        const float pw = (float)P[ax < 0 ? -ax : ax] * (float)P[ay < 0 ? -ay : ay] * (float)P[az < 0 ? -az : az];
         live = pw != 0.0f;
         nrm = sqrt((double)ax * ax + (double)ay * ay + (double)az * az);
 #pragma unroll
@@ -534,7 +537,8 @@ __global__ __launch_bounds__(mpwin_threads<LOG2L>()) void k_mpwin_zfft_multi(
             for (int mi = 0; mi < MP; ++mi) j[mi] = jj;
         }
     };
-    for (int s = 0; s < A.n_shell; ++s) {
+    const int sb = blockIdx.y * A.group, se = min(A.n_shell, sb + A.group);
+    for (int s = sb; s < se; ++s) {
         const double rs = A.radii_over_L[s];
         if (PROF) pr = prof[s];
         if (zact) {
@@ -620,10 +624,6 @@ __global__ __launch_bounds__(mpwin_threads<LOG2L>()) void k_mpwin_zfft_multi(
         }
         hermes_fft::lds_barrier();
     }
-}
-
-__global__ void k_p_to_float(const double* __restrict__ P, int n, float* __restrict__ Pf) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) Pf[i] = (float)P[i];
 }
 
 // ---------------------------------------------------------------- FP64 sums
@@ -1224,16 +1224,22 @@ int hermes_pair_reduce(hermes_ctx* ctx, int J, int dbl, const void* F1, const vo
     return pair_reduce_impl(ctx, J, dbl, F1, F2, P, descs, n_desc, out_host, nullptr, 0);
 }
 
-static int make_apply_args(hermes_ctx* ctx, int J, const double* P, const double* radii, int n_shell, int l,
-                           int m, double scale, ApplyArgs* A, float** Pf_out) {
+// Grid of the fused window kernel: octant positions (x, y) by groups of shells.  At L = 64 a single group is 1089
+// waves, about one per SIMD; groups are added up to 8 waves per SIMD (8 shells, l <= 6, two orders: 44 us with one
+// group, 34 us with eight; 73 against 84 us at L = 128; from L = 256 one group always fills the chip).
+static dim3 mpwin_groups(int J, int threads, ApplyArgs* A) {
+    const int nblk = ((1 << J) / 2 + 1) * ((1 << J) / 2 + 1), waves = nblk * (threads / 64);
+    int groups = std::max(1, std::min(A->n_shell, (8192 + waves / 2) / waves));
+    A->group = (A->n_shell + groups - 1) / groups;
+    return dim3(nblk, (A->n_shell + A->group - 1) / A->group);
+}
+
+static int make_apply_args(hermes_ctx* ctx, int J, const double* radii, int n_shell, int l, int m, double scale,
+                           ApplyArgs* A) {
     HERMES_REQUIRE(n_shell >= 1 && n_shell <= MAX_SHELLS, "n_shell=%d outside 1..%d", n_shell, MAX_SHELLS);
     HERMES_REQUIRE(l >= 0 && l <= 40 && m >= -l && m <= l, "invalid multipole (l=%d, m=%d)", l, m);
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
     const int L = 1 << J;
-    float* Pf = (float*)hermes_workspace(ctx, WS_SPEC, sizeof(float) * (L + 1));
-    HERMES_REQUIRE(Pf, "%s", hermes_last_error());
-    k_p_to_float<<<hermes_blocks(L + 1, 256), 256, 0, ctx->stream>>>(P, L + 1, Pf);
-    HERMES_LAUNCH_CHECK();
     A->L = L;
     A->l = l;
     A->m = m;
@@ -1244,8 +1250,8 @@ static int make_apply_args(hermes_ctx* ctx, int J, const double* P, const double
     A->sx = (am & 1) ? -1.0f : 1.0f;
     A->sy = 1.0f;
     A->sz = ((l + am) & 1) ? -1.0f : 1.0f;
+    A->group = n_shell;
     for (int s = 0; s < MAX_SHELLS; ++s) A->radii_over_L[s] = s < n_shell ? radii[s] / L : 0.0;
-    *Pf_out = Pf;
     return 0;
 }
 
@@ -1254,12 +1260,11 @@ int hermes_multipole_apply_f32(hermes_ctx* ctx, int J, const void* H, const doub
     HERMES_REQUIRE(ctx && H && P && radii && out, "hermes_multipole_apply_f32: null argument");
     HERMES_REQUIRE(J >= 2 && J <= 10, "J=%d unsupported", J);
     ApplyArgs A;
-    float* Pf = nullptr;
-    int rc = make_apply_args(ctx, J, P, radii, n_shell, l, m, scale, &A, &Pf);
+    int rc = make_apply_args(ctx, J, radii, n_shell, l, m, scale, &A);
     if (rc) return rc;
     const int L = 1 << J;
     const int64_t nrep = (int64_t)(L / 2 + 1) * (L / 2 + 1) * (L / 2 + 1);
-    k_multipole_apply<<<hermes_blocks(nrep, 256, 1 << 20), 256, 0, ctx->stream>>>((const float2*)H, Pf, A,
+    k_multipole_apply<<<hermes_blocks(nrep, 256, 1 << 20), 256, 0, ctx->stream>>>((const float2*)H, P, A,
                                                                                    (float2*)out);
     HERMES_LAUNCH_CHECK();
     return 0;
@@ -1311,9 +1316,8 @@ static int mpwin_zpass(hermes_ctx* ctx, int J, const void* H, const double* P, c
     HERMES_REQUIRE(n_m >= 1 && n_m <= MAX_MP, "hermes_multipole_window_zpass_multi_f32: n_m=%d outside 1..%d", n_m,
                    MAX_MP);
     ApplyArgs A;
-    float* Pf = nullptr;
     const double zeros[MAX_SHELLS] = {0.0};
-    int rc = make_apply_args(ctx, J, P, radii ? radii : zeros, n_shell, l, ms_host[0], scale, &A, &Pf);
+    int rc = make_apply_args(ctx, J, radii ? radii : zeros, n_shell, l, ms_host[0], scale, &A);
     if (rc) return rc;
     MultiM M{};
     M.n = n_m;
@@ -1328,20 +1332,20 @@ static int mpwin_zpass(hermes_ctx* ctx, int J, const void* H, const double* P, c
     }
     const float2* twg = hermes_twiddles(ctx, J, 1);
     HERMES_REQUIRE(twg, "%s", hermes_last_error());
-    const unsigned nblk = (unsigned)(((1 << J) / 2 + 1) * ((1 << J) / 2 + 1));
+    const dim3 nblk = mpwin_groups(J, J <= 7 ? 64 : 64 << (J - 7), &A);
     const float2* h = (const float2*)H;
     float2* o = (float2*)out;
 #define HERMES_MPW(LG)                                                                                         \
     if (prof_dev && n_m == 1)                                                                                  \
-        k_mpwin_zfft_multi<LG, 1, false, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, Pf, A, M, twg, o, \
+        k_mpwin_zfft_multi<LG, 1, false, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, P, A, M, twg, o, \
                                                                                               prof_dev);       \
     else if (prof_dev)                                                                                         \
-        k_mpwin_zfft_multi<LG, 2, false, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, Pf, A, M, twg, o, \
+        k_mpwin_zfft_multi<LG, 2, false, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, P, A, M, twg, o, \
                                                                                               prof_dev);       \
     else if (n_m == 1)                                                                                         \
-        k_mpwin_zfft_multi<LG, 1><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, Pf, A, M, twg, o, nullptr);   \
+        k_mpwin_zfft_multi<LG, 1><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, P, A, M, twg, o, nullptr);   \
     else                                                                                                       \
-        k_mpwin_zfft_multi<LG, 2><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, Pf, A, M, twg, o, nullptr);
+        k_mpwin_zfft_multi<LG, 2><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, P, A, M, twg, o, nullptr);
     switch (J) {
         case 3: HERMES_MPW(3) break;
         case 4: HERMES_MPW(4) break;
@@ -1362,10 +1366,10 @@ static int mpwin_zpass(hermes_ctx* ctx, int J, const void* H, const double* P, c
                 Mi.sz[0] = M.sz[i];
                 if (prof_dev)
                     k_mpwin_zfft_multi<10, 1, false, true><<<nblk, mpwin_threads<10>(), 0, ctx->stream>>>(
-                        h, Pf, A, Mi, twg, o + (size_t)i * n_shell * ((size_t)1 << 30), prof_dev);
+                        h, P, A, Mi, twg, o + (size_t)i * n_shell * ((size_t)1 << 30), prof_dev);
                 else
                     k_mpwin_zfft_multi<10, 1><<<nblk, mpwin_threads<10>(), 0, ctx->stream>>>(
-                        h, Pf, A, Mi, twg, o + (size_t)i * n_shell * ((size_t)1 << 30), nullptr);
+                        h, P, A, Mi, twg, o + (size_t)i * n_shell * ((size_t)1 << 30), nullptr);
                 HERMES_LAUNCH_CHECK();
             }
             break;
@@ -1381,8 +1385,7 @@ int hermes_multipole_window_zpass_pack0_f32(hermes_ctx* ctx, int J, const void* 
     HERMES_REQUIRE(J >= 3 && J <= 9, "hermes_multipole_window_zpass_pack0_f32: J=%d outside 3..9", J);
     HERMES_REQUIRE(l >= 0 && l < 40, "hermes_multipole_window_zpass_pack0_f32: l=%d", l);
     ApplyArgs A;
-    float* Pf = nullptr;
-    int rc = make_apply_args(ctx, J, P, radii, n_shell, l, 0, scale, &A, &Pf);
+    int rc = make_apply_args(ctx, J, radii, n_shell, l, 0, scale, &A);
     if (rc) return rc;
     MultiM M{};
     M.n = 2;
@@ -1395,11 +1398,11 @@ int hermes_multipole_window_zpass_pack0_f32(hermes_ctx* ctx, int J, const void* 
     }
     const float2* twg = hermes_twiddles(ctx, J, 1);
     HERMES_REQUIRE(twg, "%s", hermes_last_error());
-    const unsigned nblk = (unsigned)(((1 << J) / 2 + 1) * ((1 << J) / 2 + 1));
+    const dim3 nblk = mpwin_groups(J, J <= 7 ? 64 : 64 << (J - 7), &A);
     const float2* h = (const float2*)H;
     float2* o = (float2*)out;
 #define HERMES_MPWP(LG) \
-    k_mpwin_zfft_multi<LG, 2, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, Pf, A, M, twg, o, nullptr);
+    k_mpwin_zfft_multi<LG, 2, true><<<nblk, mpwin_threads<LG>(), 0, ctx->stream>>>(h, P, A, M, twg, o, nullptr);
     switch (J) {
         case 3: HERMES_MPWP(3) break;
         case 4: HERMES_MPWP(4) break;
