@@ -17,44 +17,184 @@
 #include "hermes_common.h"
 #include "reduce.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace {
 
 constexpr double TWO_PI = 6.283185307179586476925286766559;
 
-__device__ __forceinline__ double interp_at(const double* __restrict__ g, const double* __restrict__ phi, int L,
-                                            int res, double sx, double sy, double sz) {
-    const int64_t mask = L - 1;
-    const int64_t xc = (int64_t)floor(sx), yc = (int64_t)floor(sy), zc = (int64_t)floor(sz);
+// Field layouts the interpolation reads (all FP64).
+//   GRID_PLAIN    (L, L, L) z fastest, one point per lane, 8-byte loads (any alignment)
+//   GRID_ALIGNED  the same on a 16-byte aligned grid: aligned pairs of z neighbours by one load
+//   GRID_BRICK    2 x 2 x 4 cells (x, y, z) to a 128-byte line (k_brick), eight lanes to a point: a lane holds one
+//                 16-byte pair of the line, so each of the 4 or 8 lines that a 3 x 3 x 3 neighbourhood meets (6 on
+//                 average; 9 * 1.125 in the plain layout) is requested once, by one instruction
+// Interpolation at random points is bound by the lines a CU can have outstanding, not by bytes or arithmetic: more
+// waves per SIMD or fewer lines read by one lane at a time do not help (2e7 triangles at L = 256: 11.1 ms with one
+// wave per SIMD, 11.8 with four, 13.9 with bricks read by one lane), fewer line requests do.
+enum GridLayout { GRID_PLAIN = 0, GRID_ALIGNED = 1, GRID_BRICK = 2 };
+
+template <int LAYOUT>
+__device__ __forceinline__ int off_x(int x, int lg) {
+    return LAYOUT == GRID_BRICK ? ((x >> 1) << (2 * lg + 1)) + ((x & 1) << 3) : x << (2 * lg);
+}
+template <int LAYOUT>
+__device__ __forceinline__ int off_y(int y, int lg) {
+    return LAYOUT == GRID_BRICK ? ((y >> 1) << (lg + 2)) + ((y & 1) << 2) : y << lg;
+}
+template <int LAYOUT>
+__device__ __forceinline__ int off_z(int z) {
+    return LAYOUT == GRID_BRICK ? ((z >> 2) << 4) + (z & 3) : z;
+}
+
+// Cell of a scaled coordinate reduced to [0, L) (exact for |s| < 2^53) and its fraction index.
+__device__ __forceinline__ void cell_of(double s, int L, int res, int& cell, int& frac) {
+    const double c = floor(s);
     // s in (-2^-54, 0) rounds s - floor(s) to 1.0; keep the phi index inside the table
-    const int64_t xf = min((int64_t)((sx - (double)xc) * res), (int64_t)res - 1);
-    const int64_t yf = min((int64_t)((sy - (double)yc) * res), (int64_t)res - 1);
-    const int64_t zf = min((int64_t)((sz - (double)zc) * res), (int64_t)res - 1);
+    frac = min((int)((s - c) * res), res - 1);
+    cell = (int)(c - L * floor(c * (1.0 / L)));
+}
+
+// n(s) = sum over the 27 cells c - (a, b, e) of g phi phi phi.  SPHI: phi holds the table interleaved,
+// phi[3 f + a] = phi(a + f / res) (LDS copies); otherwise phi[f + a res].  The three z taps are one aligned pair
+// and one single: two loads a row, with the weights put in their order.
+template <int LAYOUT, bool SPHI>
+__device__ __forceinline__ double interp_at(const double* __restrict__ g, const double* phi, int lg, int res,
+                                            double sx, double sy, double sz) {
+    const int L = 1 << lg, m = L - 1;
+    int cx, cy, cz, fx, fy, fz;
+    cell_of(sx, L, res, cx, fx);
+    cell_of(sy, L, res, cy, fy);
+    cell_of(sz, L, res, cz, fz);
+    auto tap = [&](int f, int a) { return SPHI ? phi[3 * f + a] : phi[f + a * res]; };
+    const int z0 = (cz - 2) & m;  // first cell of the row; taps 2, 1, 0 in ascending z
+    const bool odd = z0 & 1;
+    const int zp = odd ? (z0 + 1) & m : z0, zs = odd ? z0 : (z0 + 2) & m;
+    const double t0 = tap(fz, 0), t1 = tap(fz, 1), t2 = tap(fz, 2);
+    const double wa = odd ? t1 : t2, wb = odd ? t0 : t1, ws = odd ? t2 : t0;
+    const int op = off_z<LAYOUT>(zp), os = off_z<LAYOUT>(zs);
     double acc = 0.0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const int64_t xg = (xc - a) & mask;
-        const double px = phi[xf + a * res];
+        const int ox = off_x<LAYOUT>((cx - a) & m, lg);
+        const double px = tap(fx, a);
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
-            const int64_t yg = (yc - b) & mask;
-            const double py = phi[yf + b * res];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const int64_t zg = (zc - c) & mask;
-                acc += g[(xg * L + yg) * L + zg] * px * py * phi[zf + c * res];
+            const double* row = g + (int64_t)(ox + off_y<LAYOUT>((cy - b) & m, lg));
+            const double s1 = row[os];
+            double va, vb;
+            if (LAYOUT == GRID_PLAIN) {
+                va = row[op];
+                vb = row[op + 1];
+            } else {
+                const double2 v = *(const double2*)(row + op);
+                va = v.x;
+                vb = v.y;
             }
+            acc = fma(px * tap(fy, b), fma(va, wa, fma(vb, wb, s1 * ws)), acc);
         }
     }
     return acc;
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// interp_at on a bricked grid for the 64 points of a wave (all lanes must call; lane l gets the value of its own
+// point): in round r the lanes 8 k .. 8 k + 7 take the point of lane 8 r + k, one pair of cells of a line each.
+// Cells outside the neighbourhood are neither read nor added.
+__device__ __forceinline__ double interp_bricks(const double* __restrict__ g, const double* sphi, int lg, int res,
+                                                double sx, double sy, double sz) {
+    const int L = 1 << lg, m = L - 1, lane = threadIdx.x & 63;
+    int cx, cy, cz, fx, fy, fz;
+    cell_of(sx, L, res, cx, fx);
+    cell_of(sy, L, res, cy, fy);
+    cell_of(sz, L, res, cz, fz);
+    const int cells = ((cx - 2) & m) | ((cy - 2) & m) << 10 | ((cz - 2) & m) << 20;  // the neighbourhood's first cell
+    const int fracs = fx | fy << 10 | fz << 20;
+    const int ix = (lane >> 2) & 1, iy = (lane >> 1) & 1, iz = lane & 1;  // this lane's pair of a line
+    double mine = 0.0;
+#pragma unroll 2
+    for (int r = 0; r < 8; ++r) {
+        const int src = 8 * r + (lane >> 3);
+        const int c = __shfl(cells, src, 64), f = __shfl(fracs, src, 64);
+        const int x0 = c & 1023, y0 = (c >> 10) & 1023, z0 = (c >> 20) & 1023;
+        const double* tx = sphi + 3 * (f & 1023);
+        const double* ty = sphi + 3 * ((f >> 10) & 1023);
+        const double* tz = sphi + 3 * ((f >> 20) & 1023);
+        // cell o = 0, 1, 2 of the window has tap 2 - o
+        int ox[2], oy[2];
+        double wx[2], wy[2];
+        bool vx[2], vy[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int a = 2 * q + ix - (x0 & 1), b = 2 * q + iy - (y0 & 1);
+            vx[q] = a >= 0 && a <= 2;
+            vy[q] = b >= 0 && b <= 2;
+            wx[q] = tx[vx[q] ? 2 - a : 0];
+            wy[q] = ty[vy[q] ? 2 - b : 0];
+            ox[q] = off_x<GRID_BRICK>((x0 + a) & m, lg);
+            oy[q] = off_y<GRID_BRICK>((y0 + b) & m, lg);
+        }
+        double acc = 0.0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int e0 = 4 * q + 2 * iz - (z0 & 3), e1 = e0 + 1;
+            const bool v0 = e0 >= 0 && e0 <= 2, v1 = e1 >= 0 && e1 <= 2;
+            const double w0 = tz[v0 ? 2 - e0 : 0], w1 = tz[v1 ? 2 - e1 : 0];
+            const int oz = off_z<GRID_BRICK>((z0 + e0) & m);  // even: z0 + e0 = 4 k + 2 iz
+            const bool vz = v0 || v1;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (vz && vx[i >> 1] && vy[i & 1]) {
+                    const double2 v = *(const double2*)(g + (int64_t)(ox[i >> 1] + oy[i & 1] + oz));
+                    const double t = (v0 ? v.x * w0 : 0.0) + (v1 ? v.y * w1 : 0.0);
+                    acc = fma(wx[i >> 1] * wy[i & 1], t, acc);
+                }
+            }
+        }
+        acc += dpp_f64<0xB1>(acc);   // quad_perm 1 0 3 2
+        acc += dpp_f64<0x4E>(acc);   // quad_perm 2 3 0 1
+        acc += dpp_f64<0x141>(acc);  // row_half_mirror: the other four lanes of the eight
+        const double v = __shfl(acc, (lane & 7) * 8, 64);
+        if ((lane >> 3) == r) mine = v;
+    }
+    return mine;
+}
+
+template <int LAYOUT>
+__device__ __forceinline__ double interp(const double* __restrict__ g, const double* sphi, int lg, int res, double sx,
+                                         double sy, double sz) {
+    if constexpr (LAYOUT == GRID_BRICK) return interp_bricks(g, sphi, lg, res, sx, sy, sz);
+    else return interp_at<LAYOUT, true>(g, sphi, lg, res, sx, sy, sz);
+}
+
+// Bricked copy of a grid (GRID_BRICK), L >= 4.
+__global__ __launch_bounds__(256) void k_brick(const double* __restrict__ g, int lg, double* __restrict__ out) {
+    const int64_t n = (int64_t)1 << (3 * lg);
+    const int m = (1 << lg) - 1;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int z = (int)(i & m), y = (int)(i >> lg) & m, x = (int)(i >> (2 * lg));
+        out[off_x<GRID_BRICK>(x, lg) + off_y<GRID_BRICK>(y, lg) + off_z<GRID_BRICK>(z)] = g[i];
+    }
+}
+
+// The scaling function in LDS, tap-interleaved; res = 1024.
+__device__ __forceinline__ void load_phi(double* sphi, const double* __restrict__ phi, int tid, int nt) {
+    for (int i = tid; i < 3 * 1024; i += nt) sphi[3 * (i & 1023) + (i >> 10)] = phi[i];
+}
+
 __global__ void k_interpolate(const double* __restrict__ g, const double* __restrict__ spos, int64_t n,
-                              const double* __restrict__ phi, int L, int res, double dx, double dy, double dz,
+                              const double* __restrict__ phi, int lg, int res, double dx, double dy, double dz,
                               double* __restrict__ out) {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x)
-        out[p] = interp_at(g, phi, L, res, spos[3 * p] + dx, spos[3 * p + 1] + dy, spos[3 * p + 2] + dz);
+        out[p] = interp_at<GRID_PLAIN, false>(g, phi, lg, res, spos[3 * p] + dx, spos[3 * p + 1] + dy,
+                                              spos[3 * p + 2] + dz);
 }
 
 // corr3pcf_kernels.py:21-63
@@ -93,27 +233,42 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 constexpr int MC_THREADS = 256;
 
-// grid over (rotation, centre); per-block partial sums
-__global__ __launch_bounds__(MC_THREADS) void k_triplet_box(double R1, double R2, double mu,
-                                                            const double* __restrict__ spos,
-                                                            const double* __restrict__ n1, int64_t n, int n_rot,
-                                                            const double* __restrict__ abc,
-                                                            const double* __restrict__ g2,
-                                                            const double* __restrict__ g3,
-                                                            const double* __restrict__ phi, int L, int res,
-                                                            double* __restrict__ partial) {
+// The two edge vectors of every rotation (they depend on nothing else).
+__global__ void k_triplet_offsets(double R1, double R2, double mu, const double* __restrict__ abc, int n_rot,
+                                  double* __restrict__ off) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n_rot) return;
+    double o[6];
+    triangle_offsets(R1, R2, mu, TWO_PI * abc[3 * r], 2.0 * abc[3 * r + 1] - 1.0, TWO_PI * abc[3 * r + 2], o);
+    for (int i = 0; i < 6; ++i) off[6 * r + i] = o[i];
+}
+
+// blockIdx.y: rotation (strided); blockIdx.x: centres (strided); per-block partial sums.  Bound by random lines of
+// the grids and the latency of their loads.
+template <int LAYOUT>
+__global__ __launch_bounds__(MC_THREADS, 4) void k_triplet_box(const double* __restrict__ spos,
+                                                               const double* __restrict__ n1, int64_t n, int n_rot,
+                                                               const double* __restrict__ off,
+                                                               const double* __restrict__ g2,
+                                                               const double* __restrict__ g3,
+                                                               const double* __restrict__ phi, int lg, int res,
+                                                               double* __restrict__ partial) {
+    __shared__ double sphi[3 * 1024];
     __shared__ double sh[MC_THREADS / 64];
-    const int64_t total = n * (int64_t)n_rot;
+    load_phi(sphi, phi, threadIdx.x, MC_THREADS);
+    __syncthreads();
     double s = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / n);
-        const int64_t p = i - (int64_t)r * n;
-        double o[6];
-        triangle_offsets(R1, R2, mu, TWO_PI * abc[3 * r], 2.0 * abc[3 * r + 1] - 1.0, TWO_PI * abc[3 * r + 2], o);
-        const double x = spos[3 * p], y = spos[3 * p + 1], z = spos[3 * p + 2];
-        const double v2 = interp_at(g2, phi, L, res, x + o[0], y + o[1], z + o[2]);
-        const double v3 = interp_at(g3, phi, L, res, x + o[3], y + o[4], z + o[5]);
-        s += n1[p] * v2 * v3;
+    for (int r = blockIdx.y; r < n_rot; r += gridDim.y) {
+        const double* o = off + 6 * r;
+        // whole waves (the lanes of a bricked interpolation work together): lanes past the end repeat the last centre
+        for (int64_t q = blockIdx.x * (int64_t)MC_THREADS + (threadIdx.x & ~63); q < n;
+             q += (int64_t)gridDim.x * MC_THREADS) {
+            const int64_t mine = q + (threadIdx.x & 63), p = mine < n ? mine : n - 1;
+            const double x = spos[3 * p], y = spos[3 * p + 1], z = spos[3 * p + 2];
+            const double v2 = interp<LAYOUT>(g2, sphi, lg, res, x + o[0], y + o[1], z + o[2]);
+            const double v3 = interp<LAYOUT>(g3, sphi, lg, res, x + o[3], y + o[4], z + o[5]);
+            if (mine < n) s += n1[p] * v2 * v3;
+        }
     }
     s = wave_sum(s);
     if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
@@ -121,7 +276,7 @@ __global__ __launch_bounds__(MC_THREADS) void k_triplet_box(double R1, double R2
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int w = 0; w < MC_THREADS / 64; ++w) t += sh[w];
-        partial[blockIdx.x] = t;
+        partial[blockIdx.y * gridDim.x + blockIdx.x] = t;
     }
 }
 
@@ -150,7 +305,7 @@ __device__ __forceinline__ double u53(uint32_t a, uint32_t b) {
 }
 
 struct BinnedArgs {
-    int L, res, nr1, nr2, nmu;
+    int L, lg, res, nr1, nr2, nmu;
     double rmin1, rmax1, rmin2, rmax2;  // grid units, uniform (linear) bins
     double cap;                          // |w f| above cap goes to the overflow list (main pass)
     double scale_wf, scale_wf2;          // fixed-point scales for sum(w f) and sum((w f)^2)
@@ -215,19 +370,19 @@ struct Sample {
 // so the weight is w = 1 / (alpha + (1 - alpha) * mean_a R(k(v_a), b)) over the
 // vertices v_a of the drawn triangle (one anchor: the apex only).  The same i
 // always gives the same sample, whichever pass evaluates it.
+template <int LAYOUT>
 __device__ __forceinline__ void draw_sample(const BinnedArgs& A, const double* __restrict__ g1,
                                             const double* __restrict__ g2, const double* __restrict__ g3,
-                                            const double* __restrict__ phi, const ProposalTables& T, int64_t i,
-                                            Sample& S) {
+                                            const double* sphi, const ProposalTables& T, int64_t i, Sample& S) {
     const int L = A.L;
     const int B = A.nr1 * A.nr2 * A.nmu;
     const int Ls = L * A.sub;
     const double sub = (double)A.sub;
     const double dr1 = (A.rmax1 - A.rmin1) / A.nr1, dr2 = (A.rmax2 - A.rmin2) / A.nr2, dmu = 2.0 / A.nmu;
-    double ux, uy, uz, ubin, upick, umix, ubin2, w1, w2, w3, oph, oct, oal, uanc;
+    double ux, uy, uz, ubin, upick = 0.0, umix = 0.0, ubin2, w1, w2, w3, oph, oct, oal, uanc;
     uniforms2((uint64_t)i, A.seed, 0, ux, uy);
     uniforms2((uint64_t)i, A.seed, 1, uz, ubin);
-    uniforms2((uint64_t)i, A.seed, 2, upick, umix);
+    if (A.importance) uniforms2((uint64_t)i, A.seed, 2, upick, umix);
     uniforms2((uint64_t)i, A.seed, 3, ubin2, w1);
     uniforms2((uint64_t)i, A.seed, 4, w2, w3);
     uniforms2((uint64_t)i, A.seed, 5, oph, oct);
@@ -272,10 +427,16 @@ __device__ __forceinline__ void draw_sample(const BinnedArgs& A, const double* _
         cy = py - o[4];
         cz = pz - o[5];
     }
-    const double n1 = interp_at(g1, phi, L, A.res, cx, cy, cz);
-    const double n2 = interp_at(g2, phi, L, A.res, cx + o[0], cy + o[1], cz + o[2]);
-    const double n3 = interp_at(g3, phi, L, A.res, cx + o[3], cy + o[4], cz + o[5]);
-    const double f = n1 * n2 * n3;
+    // one vertex at a time, so that the registers allow several waves per SIMD
+    double f = 1.0;
+#pragma unroll 1
+    for (int v = 0; v < 3; ++v) {
+        const double* g = v == 0 ? g1 : (v == 1 ? g2 : g3);
+        const double x = v == 0 ? cx : (v == 1 ? cx + o[0] : cx + o[3]);
+        const double y = v == 0 ? cy : (v == 1 ? cy + o[1] : cy + o[4]);
+        const double z = v == 0 ? cz : (v == 1 ? cz + o[2] : cz + o[5]);
+        f *= interp<LAYOUT>(g, sphi, A.lg, A.res, x, y, z);
+    }
     double w = 1.0;
     S.k[0] = S.k[1] = S.k[2] = -1;
     if (T.cell_bucket) {
@@ -310,19 +471,29 @@ enum McPass { MC_PILOT = 0, MC_MAIN = 1, MC_FIXUP = 2 };
 // bit pattern of a non-negative double, whose integer order is the numeric order;
 // stats[1] counts overflow samples.  Fixed-point sums make the result
 // independent of the order of the atomics.
-template <int PASS>
-__global__ __launch_bounds__(MC_THREADS) void k_mc_binned(
+// Bound by the random lines of the grids (see GridLayout).  2e7 uniform triangles at L = 256: 10.4 ms with one lane
+// per triangle and 27 loads per vertex, 7.0 ms with bricks.
+template <int PASS, int LAYOUT>
+__global__ __launch_bounds__(MC_THREADS, 4) void k_mc_binned(
     const double* __restrict__ g1, const double* __restrict__ g2, const double* __restrict__ g3,
     const double* __restrict__ phi, BinnedArgs A, ProposalTables T, const int64_t* __restrict__ fix_list,
     unsigned long long* __restrict__ acc, unsigned long long* __restrict__ acc_hi,
     unsigned long long* __restrict__ stats, int64_t* __restrict__ over_list, float* __restrict__ rec) {
     __shared__ double red[MC_THREADS / 64];
+    __shared__ double sphi[3 * 1024];
+    load_phi(sphi, phi, threadIdx.x, MC_THREADS);
+    __syncthreads();
     const int B = A.nr1 * A.nr2 * A.nmu;
     double mx = 0.0;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < A.n; t += (int64_t)gridDim.x * blockDim.x) {
+    // whole waves (the lanes of a bricked interpolation work together): lanes past the end repeat the last sample
+    for (int64_t q = blockIdx.x * (int64_t)MC_THREADS + (threadIdx.x & ~63); q < A.n;
+         q += (int64_t)gridDim.x * MC_THREADS) {
+        const bool mine = q + (threadIdx.x & 63) < A.n;
+        const int64_t t = mine ? q + (threadIdx.x & 63) : A.n - 1;
         const int64_t i = PASS == MC_FIXUP ? fix_list[t] : t;
         Sample S;
-        draw_sample(A, g1, g2, g3, phi, T, i, S);
+        draw_sample<LAYOUT>(A, g1, g2, g3, sphi, T, i, S);
+        if (!mine) continue;
         const double a = fabs(S.wf);
         mx = (a == a) ? fmax(mx, a) : INFINITY;
         if (PASS == MC_FIXUP) {
@@ -370,7 +541,7 @@ constexpr int BK_PER_THREAD = 64;
 constexpr int BK_CHUNK = BK_THREADS * BK_PER_THREAD;
 
 __global__ __launch_bounds__(BK_THREADS) void k_bucket_assign(const double* __restrict__ g,
-                                                              const double* __restrict__ phi, int L, int res,
+                                                              const double* __restrict__ phi, int lg, int res,
                                                               int sub, const double* __restrict__ edges,
                                                               int nbucket, int64_t ncell,
                                                               unsigned char* __restrict__ cell_bucket,
@@ -378,14 +549,15 @@ __global__ __launch_bounds__(BK_THREADS) void k_bucket_assign(const double* __re
     __shared__ int h[256];
     for (int k = threadIdx.x; k < 256; k += BK_THREADS) h[k] = 0;
     __syncthreads();
-    const int64_t Ls = (int64_t)L * sub;
+    const int64_t Ls = (int64_t)sub << lg;
     const double inv = 1.0 / sub;
     const int64_t base = (int64_t)blockIdx.x * BK_CHUNK;
     for (int j = 0; j < BK_PER_THREAD; ++j) {
         const int64_t i = base + (int64_t)j * BK_THREADS + threadIdx.x;
         if (i < ncell) {
             const int64_t zs = i % Ls, ys = (i / Ls) % Ls, xs = i / (Ls * Ls);
-            const double v = interp_at(g, phi, L, res, (xs + 0.5) * inv, (ys + 0.5) * inv, (zs + 0.5) * inv);
+            const double v = interp_at<GRID_PLAIN, false>(g, phi, lg, res, (xs + 0.5) * inv, (ys + 0.5) * inv,
+                                                          (zs + 0.5) * inv);
             int lo = 0, hi = nbucket - 1;  // first edge > v
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
@@ -495,6 +667,37 @@ __global__ __launch_bounds__(BK_THREADS) void k_bucket_scatter(const unsigned ch
 
 }  // namespace
 
+// Layout for `points` interpolations on the n_grid grids g (replaced by their bricked copies where they are made).
+// A copy reads and writes the grid once, which pays from about one point per 8 cells on (L = 512, 4e6 triangles, one per 11:
+// 3.9 against 3.4 ms; L = 256, 1e6, one per 6: 0.94 against 1.22); below L = 128 the grid
+// stays in the L2 caches and a point per lane is the faster way (2e7 uniform triangles: L = 64 3.8 ms, with bricks
+// 4.4; L = 128 8.8 and 7.2; L = 256 11.8 and 7.6; L = 512 21.3 and 12.5).  The copies are kept within 4 GiB.  Grids
+// not aligned to 16 bytes are bricked under the same rule or read by 8 bytes.
+static int grid_layout(hermes_ctx* ctx, int J, double points, const double** g, int n_grid) {
+    const size_t n = (size_t)1 << (3 * J);
+    bool aligned = true;
+    for (int i = 0; i < n_grid; ++i) aligned = aligned && ((uintptr_t)g[i] & 15) == 0;
+    const int plain = aligned ? GRID_ALIGNED : GRID_PLAIN;
+    int copies = 0, of[3];
+    const double* distinct[3];
+    for (int i = 0; i < n_grid; ++i) {
+        int k = 0;
+        while (k < copies && distinct[k] != g[i]) ++k;
+        if (k == copies) distinct[copies++] = g[i];
+        of[i] = k;
+    }
+    if (J < 7 || points * 8.0 < (double)n * copies || copies * n * sizeof(double) > ((size_t)4 << 30)) return plain;
+    double* ws = (double*)hermes_workspace(ctx, WS_SPEC, copies * n * sizeof(double));
+    if (!ws) {
+        (void)hipGetLastError();
+        return plain;
+    }
+    for (int k = 0; k < copies; ++k)
+        k_brick<<<hermes_blocks((int64_t)n, 256, 16384), 256, 0, ctx->stream>>>(distinct[k], J, ws + k * n);
+    for (int i = 0; i < n_grid; ++i) g[i] = ws + of[i] * n;
+    return GRID_BRICK;
+}
+
 extern "C" {
 
 int hermes_interpolate(hermes_ctx* ctx, int J, const double* grid, const double* spos, int64_t n, const double* phi,
@@ -504,7 +707,7 @@ int hermes_interpolate(hermes_ctx* ctx, int J, const double* grid, const double*
     HERMES_REQUIRE(phi_res == 1024, "phi_res must be 1024");
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
     if (n == 0) return 0;
-    k_interpolate<<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(grid, spos, n, phi, 1 << J, phi_res, dx, dy,
+    k_interpolate<<<hermes_blocks(n, 256, 65536), 256, 0, ctx->stream>>>(grid, spos, n, phi, J, phi_res, dx, dy,
                                                                          dz, out);
     HERMES_LAUNCH_CHECK();
     return 0;
@@ -517,14 +720,24 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     HERMES_REQUIRE(J >= 2 && J <= 10, "J=%d unsupported", J);
     HERMES_REQUIRE(n > 0 && n_rot > 0, "need centres and rotations");
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
-    const int64_t total = n * (int64_t)n_rot;
-    const int nb = (int)hermes_blocks(total, MC_THREADS, 8192);
-    double* ws = (double*)hermes_workspace(ctx, WS_MC, sizeof(double) * ((size_t)nb + 8 + 3 * (size_t)n_rot));
+    // about 2048 workgroups: the centres by the rotations
+    const int nbx = (int)hermes_blocks(n, MC_THREADS, 2048);
+    const int nby = (int)std::min<int64_t>(n_rot, std::max(1, 2048 / nbx));
+    const int nb = nbx * nby;
+    double* ws = (double*)hermes_workspace(ctx, WS_MC, sizeof(double) * ((size_t)nb + 8 + 9 * (size_t)n_rot));
     HERMES_REQUIRE(ws, "%s", hermes_last_error());
-    double* d_abc = ws + nb + 8;
+    double *d_abc = ws + nb + 8, *d_off = d_abc + 3 * (size_t)n_rot;
     HERMES_CHECK_HIP(hipMemcpyAsync(d_abc, abc_host, sizeof(double) * 3 * n_rot, hipMemcpyHostToDevice, ctx->stream));
-    k_triplet_box<<<nb, MC_THREADS, 0, ctx->stream>>>(R1, R2, mu, spos, n1, n, n_rot, d_abc, g2, g3, phi, 1 << J,
-                                                      phi_res, ws);
+    k_triplet_offsets<<<hermes_blocks(n_rot, 64), 64, 0, ctx->stream>>>(R1, R2, mu, d_abc, n_rot, d_off);
+    HERMES_LAUNCH_CHECK();
+    const double* g[2] = {g2, g3};
+    const int layout = grid_layout(ctx, J, 2.0 * (double)n * n_rot, g, 2);
+    auto go = [&](auto kernel) {
+        kernel<<<dim3(nbx, nby), MC_THREADS, 0, ctx->stream>>>(spos, n1, n, n_rot, d_off, g[0], g[1], phi, J, phi_res, ws);
+    };
+    if (layout == GRID_BRICK) go(k_triplet_box<GRID_BRICK>);
+    else if (layout == GRID_ALIGNED) go(k_triplet_box<GRID_ALIGNED>);
+    else go(k_triplet_box<GRID_PLAIN>);
     HERMES_LAUNCH_CHECK();
     HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, 1, nb, 1, nullptr, ws + nb));
     double s = 0.0;
@@ -563,6 +776,7 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
     constexpr int64_t PILOT = 1 << 20;
     BinnedArgs A;
     A.L = 1 << J;
+    A.lg = J;
     A.res = phi_res;
     A.nr1 = nr1;
     A.nr2 = nr2;
@@ -592,6 +806,14 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
     unsigned long long* acc_hi = acc + 3 * (size_t)B;
     unsigned long long* stats = acc_hi + 2 * (size_t)B;
     int64_t* over_list = (int64_t*)(ws + sizeof(unsigned long long) * n_acc);
+    const double* g[3] = {g1, g2, g3};
+    const int layout = grid_layout(ctx, J, 3.0 * (double)n_samples, g, 3);
+    // workgroups load the scaling function once and loop over samples
+    auto launch = [&](auto brick, auto aligned, auto plain, const BinnedArgs& args, const int64_t* list, float* out) {
+        auto kernel = layout == GRID_BRICK ? brick : (layout == GRID_ALIGNED ? aligned : plain);
+        kernel<<<hermes_blocks(args.n, MC_THREADS, 2048), MC_THREADS, 0, ctx->stream>>>(
+            g[0], g[1], g[2], phi, args, T, list, acc, acc_hi, stats, over_list, out);
+    };
     unsigned long long st[2];
     auto read_stats = [&]() -> int {
         HERMES_CHECK_HIP(hipMemcpyAsync(st, stats, sizeof(st), hipMemcpyDeviceToHost, ctx->stream));
@@ -606,8 +828,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
     if (!(cap > 0.0)) {
         HERMES_CHECK_HIP(hipMemsetAsync(stats, 0, 2 * sizeof(unsigned long long), ctx->stream));
         A.n = n_samples < PILOT ? n_samples : PILOT;
-        k_mc_binned<MC_PILOT><<<hermes_blocks(A.n, MC_THREADS, 16384), MC_THREADS, 0, ctx->stream>>>(
-            g1, g2, g3, phi, A, T, nullptr, acc, acc_hi, stats, over_list, nullptr);
+        launch(k_mc_binned<MC_PILOT, GRID_BRICK>, k_mc_binned<MC_PILOT, GRID_ALIGNED>, k_mc_binned<MC_PILOT, GRID_PLAIN>, A,
+               nullptr, nullptr);
         HERMES_LAUNCH_CHECK();
         if (read_stats()) return 1;
         cap = max_of();
@@ -621,8 +843,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
         // |w f| <= cap for every accumulated sample: each bin sum stays below 2^62
         A.scale_wf = ldexp(1.0, 62) / ((double)n_samples * cap);
         A.scale_wf2 = ldexp(1.0, 62) / ((double)n_samples * cap * cap);
-        k_mc_binned<MC_MAIN><<<hermes_blocks(n_samples, MC_THREADS, 16384), MC_THREADS, 0, ctx->stream>>>(
-            g1, g2, g3, phi, A, T, nullptr, acc, acc_hi, stats, over_list, record);
+        launch(k_mc_binned<MC_MAIN, GRID_BRICK>, k_mc_binned<MC_MAIN, GRID_ALIGNED>, k_mc_binned<MC_MAIN, GRID_PLAIN>, A,
+               nullptr, record);
         HERMES_LAUNCH_CHECK();
         if (read_stats()) return 1;
         if (st[1] == 0) break;
@@ -641,8 +863,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
         F.record = 0;
         F.scale_wf = scale_hi = ldexp(1.0, 62) / ((double)n_over * mx);
         F.scale_wf2 = scale_hi2 = ldexp(1.0, 62) / ((double)n_over * mx * mx);
-        k_mc_binned<MC_FIXUP><<<hermes_blocks(n_over, MC_THREADS, 16384), MC_THREADS, 0, ctx->stream>>>(
-            g1, g2, g3, phi, F, T, over_list, acc, acc_hi, stats, over_list, nullptr);
+        launch(k_mc_binned<MC_FIXUP, GRID_BRICK>, k_mc_binned<MC_FIXUP, GRID_ALIGNED>, k_mc_binned<MC_FIXUP, GRID_PLAIN>, F,
+               over_list, nullptr);
         HERMES_LAUNCH_CHECK();
     }
     std::vector<long long> h(5 * (size_t)B);
@@ -687,7 +909,7 @@ int hermes_mc_bucketize(hermes_ctx* ctx, int J, const double* grid, const double
     if (nbucket > 1)
         HERMES_CHECK_HIP(hipMemcpyAsync(edges, edges_host, sizeof(double) * (nbucket - 1), hipMemcpyHostToDevice,
                                         ctx->stream));
-    k_bucket_assign<<<nblocks, BK_THREADS, 0, ctx->stream>>>(grid, phi, 1 << J, phi_res, sub, edges, nbucket, ncell,
+    k_bucket_assign<<<nblocks, BK_THREADS, 0, ctx->stream>>>(grid, phi, J, phi_res, sub, edges, nbucket, ncell,
                                                              cell_bucket, hist);
     HERMES_LAUNCH_CHECK();
     k_bucket_scan<<<nbucket, 1024, 0, ctx->stream>>>(hist, nblocks, tot);
