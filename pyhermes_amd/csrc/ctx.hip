@@ -58,14 +58,19 @@ void* hermes_workspace(hermes_ctx* ctx, int slot, size_t bytes) {
     return p;
 }
 
-int hermes_read_word(hermes_ctx* ctx, const int* dev, int* out) {
-    if (!ctx->host_word) HERMES_CHECK_HIP(hipHostMalloc((void**)&ctx->host_word, 64, hipHostMallocDefault));
-    HERMES_CHECK_HIP(hipMemcpyAsync(ctx->host_word, dev, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+int* hermes_host_word(hermes_ctx* ctx) {
+    if (!ctx->host_word && hipHostMalloc((void**)&ctx->host_word, 64, hipHostMallocDefault) != hipSuccess) {
+        ctx->host_word = nullptr;
+        hermes_set_error("hipHostMalloc of the host word failed");
+    }
+    return ctx->host_word;
+}
+
+int hermes_poll_stream(hermes_ctx* ctx) {
     hipError_t e;
     while ((e = hipStreamQuery(ctx->stream)) == hipErrorNotReady) {
     }
     HERMES_CHECK_HIP(e);
-    *out = *(volatile int*)ctx->host_word;
     return 0;
 }
 
@@ -100,6 +105,7 @@ int hermes_ctx_create(int device, hermes_ctx** out) {
     if (int rc = hermes_scratch_setup(device)) return rc;
     hermes_ctx* c = new hermes_ctx();
     c->device = device;
+    (void)hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device);
     c->stream = nullptr;
     *out = c;
     return 0;

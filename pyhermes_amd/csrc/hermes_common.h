@@ -22,8 +22,9 @@ enum hermes_ws_slot {
     WS_MLP = 6,
     WS_CONTRACT = 7,
     WS_PROFILE = 8,     // radial profiles of the fused window kernel
+    WS_PROJ_SLOT = 9,   // projection: slots of the particles in their tiles
 };
-constexpr int HERMES_WS_SLOTS = 9;
+constexpr int HERMES_WS_SLOTS = 10;
 
 // One library context per device: stream, grow-only workspaces and FFT plans.
 struct hermes_ctx {
@@ -48,7 +49,8 @@ struct hermes_ctx {
     // from the host, memset or synchronise; kernels report input errors into dev_err
     bool capturing = false;
     int* dev_err = nullptr;  // sticky device error word (see hermes_read_errors)
-    int* host_word = nullptr;  // pinned host word for hermes_read_word (allocated on first use)
+    int* host_word = nullptr;  // pinned host word (hermes_host_word)
+    int n_cu = 256;            // compute units of the device
 };
 
 
@@ -59,9 +61,11 @@ void* hermes_workspace(hermes_ctx* ctx, int slot, size_t bytes);
 // Resolves, on the current device, the device address of the allocation-free pair reduction's fixed
 // scratch array (window.hip); called once per device by hermes_ctx_create.
 int hermes_scratch_setup(int device);
-// Reads one device int after the stream's preceding work, waiting by polling the stream (a blocking
-// wait would add the host thread's wake-up latency to every eager call).  Not while capturing.
-int hermes_read_word(hermes_ctx* ctx, const int* dev, int* out);
+// Pinned host word that kernels of this context may store to (allocated on first use); nullptr with an error set.
+int* hermes_host_word(hermes_ctx* ctx);
+// Waits for the stream's work by polling it (a blocking wait would add the host thread's wake-up latency to every
+// eager call).  Not while capturing.
+int hermes_poll_stream(hermes_ctx* ctx);
 // Twiddle table e^{dir 2 pi i k / 2^log2L}, k < 2^log2L (device memory owned by ctx).
 const float2* hermes_twiddles(hermes_ctx* ctx, int log2L, int dir);
 // Inverse FFT along y and x of a batch of (L, L, L) complex64 grids already transformed along z.

@@ -3,7 +3,8 @@
 // Deterministic, atomics-free in floating point:
 //   1. count:  each particle is assigned to every output tile its 3x3x3 stencil
 //              touches (1..8 tiles; tiles are 4x8x64 cells, z fastest); integer
-//              counts per tile (wave-aggregated atomics).
+//              counts per tile (wave-aggregated atomics), whose returned values
+//              are the particle's slots in its tiles.
 //   2. scan:   exclusive scan of the tile counts.
 //   3. fill:   bucket 16-byte records {cell, frac, w} per tile.
 //   4. accumulate: one workgroup per tile sums the 27 FP64 contributions of its
@@ -13,6 +14,7 @@
 //              writes the tile once, coalesced, as FP32 and/or FP64.
 // Integer addition is associative, so the result is bit-identical whatever the
 // order in which records were bucketed or accumulated.
+#include <algorithm>
 #include <cmath>
 
 #include "../../include/hermes_amd.h"
@@ -22,9 +24,8 @@ namespace {
 
 constexpr int MAX_TX = 4, MAX_TY = 8, MAX_TZ = 64;
 constexpr int TILE_CELLS = MAX_TX * MAX_TY * MAX_TZ;
-constexpr int ACC_THREADS = 256;
+constexpr int ACC_THREADS = 256, ACC_THREADS_FEW = 1024;  // accumulation workgroups (see launch_accumulate)
 constexpr int SCAN_THREADS = 1024, SCAN_ITEMS = 4;  // counts per scan block: 4096
-constexpr int ACC_RCHUNK = 512;                      // records staged per LDS chunk
 constexpr int OFFCH = 128;                           // tile ranges staged per LDS block
 
 struct ProjRec {
@@ -106,9 +107,11 @@ __device__ __forceinline__ int replica_tile(const TileGeom& g, const int X[2], c
     return tile_id(g, X[a], Y[b], Z[d]);
 }
 
+// err: a word set on invalid positions (device memory, or pinned host memory that the host reads after the wait).
+// slots (may be NULL): slots[k n + p] = slot of particle p in the tile of its replica k.
 __global__ void k_proj_count(const double* __restrict__ pos, int64_t n, double sf, int res, TileGeom g,
                              int* __restrict__ tile_count, int32_t* __restrict__ cell_out,
-                             int32_t* __restrict__ frac_out, int* __restrict__ err) {
+                             int32_t* __restrict__ frac_out, int* err, int* __restrict__ slots) {
     const int m = g.L - 1;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int64_t nround = (n + stride - 1) / stride * stride;  // uniform trip count for the wave-wide ops
@@ -116,7 +119,8 @@ __global__ void k_proj_count(const double* __restrict__ pos, int64_t n, double s
         const bool act = p < n;
         int c[3] = {0, 0, 0}, f[3] = {0, 0, 0};
         if (act) {
-            if (!cell_frac(pos, p, sf, res, c, f)) atomicOr(err, 1);
+            if (!cell_frac(pos, p, sf, res, c, f))
+                __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (cell_out) { cell_out[3 * p] = c[0]; cell_out[3 * p + 1] = c[1]; cell_out[3 * p + 2] = c[2]; }
             if (frac_out) { frac_out[3 * p] = f[0]; frac_out[3 * p + 1] = f[1]; frac_out[3 * p + 2] = f[2]; }
         }
@@ -126,25 +130,92 @@ __global__ void k_proj_count(const double* __restrict__ pos, int64_t n, double s
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int t = act ? replica_tile(g, X, Y, Z, nx, ny, nz, k) : -1;
-            (void)wave_add(tile_count, t < 0 ? 0 : t, t >= 0);
+            const int slot = wave_add(tile_count, t < 0 ? 0 : t, t >= 0);
+            if (slots && t >= 0) slots[(int64_t)k * n + p] = slot;
         }
     }
 }
 
-// Exclusive scan of the tile counts in three launches: block sums, a scan of the block sums
-// (one workgroup; at most 2^19 tiles -> 128 blocks), then each block's local scan plus its offset.
-// The last launch also clears the fill cursors and writes the total to off[n].
+// The same for grids of at most LDS_TILES tiles (J <= 8), slots kept: a workgroup counts its PPT * 256 particles in
+// LDS, whose atomics return their ranks, adds one total per tile it met to the tile's counter, and the slots are
+// those bases plus the ranks.  On these grids the counters share a few cache lines (128 tiles: four), and one
+// global atomic per wave group and replica serialised on them: 500,000 shuffled particles at J = 6 took 0.69 ms in
+// this step and as much in the next, 21 us now.
+constexpr int LDS_TILES = 8192;
+
+template <int PPT>
+__global__ __launch_bounds__(256) void k_proj_count_lds(const double* __restrict__ pos, int64_t n, double sf, int res,
+                                                        TileGeom g, int ntiles, int* __restrict__ tile_count,
+                                                        int32_t* __restrict__ cell_out, int32_t* __restrict__ frac_out,
+                                                        int* err, int* __restrict__ slots) {
+    extern __shared__ int lcount[];  // [ntiles]
+    const int m = g.L - 1, tid = threadIdx.x;
+    for (int t = tid; t < ntiles; t += 256) lcount[t] = 0;
+    __syncthreads();
+    const int64_t p0 = (int64_t)blockIdx.x * (PPT * 256);
+    uint32_t home[PPT], rank[PPT][4];  // wrapped cell, and two 16-bit ranks a word, replicas 0 .. 7
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+        const int64_t p = p0 + i * 256 + tid;
+        if (p >= n) continue;
+        int c[3], f[3];
+        if (!cell_frac(pos, p, sf, res, c, f)) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (cell_out) { cell_out[3 * p] = c[0]; cell_out[3 * p + 1] = c[1]; cell_out[3 * p + 2] = c[2]; }
+        if (frac_out) { frac_out[3 * p] = f[0]; frac_out[3 * p + 1] = f[1]; frac_out[3 * p + 2] = f[2]; }
+        home[i] = (uint32_t)(c[0] & m) | ((uint32_t)(c[1] & m) << 10) | ((uint32_t)(c[2] & m) << 20);
+        int X[2], Y[2], Z[2];
+        const int nx = tiles_of(c[0], m, g.lgtx, X), ny = tiles_of(c[1], m, g.lgty, Y),
+                  nz = tiles_of(c[2], m, g.lgtz, Z);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int t = replica_tile(g, X, Y, Z, nx, ny, nz, k);
+            const uint32_t r = t >= 0 ? (uint32_t)atomicAdd(&lcount[t], 1) : 0u;
+            rank[i][k / 2] = k % 2 ? rank[i][k / 2] | r << 16 : r;
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < ntiles; t += 256) {
+        const int c = lcount[t];
+        if (c) lcount[t] = atomicAdd(&tile_count[t], c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+        const int64_t p = p0 + i * 256 + tid;
+        if (p >= n) continue;
+        const int c[3] = {(int)(home[i] & 1023), (int)((home[i] >> 10) & 1023), (int)(home[i] >> 20)};
+        int X[2], Y[2], Z[2];
+        const int nx = tiles_of(c[0], m, g.lgtx, X), ny = tiles_of(c[1], m, g.lgty, Y),
+                  nz = tiles_of(c[2], m, g.lgtz, Z);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int t = replica_tile(g, X, Y, Z, nx, ny, nz, k);
+            if (t >= 0) slots[(int64_t)k * n + p] = lcount[t] + (int)(k % 2 ? rank[i][k / 2] >> 16 : rank[i][k / 2] & 0xffff);
+        }
+    }
+}
+
+// Exclusive scan of the tile counts, SCAN_BLOCK per workgroup: one launch up to that many tiles (J <= 7), otherwise
+// a launch of block sums first, which every block of the second adds up to its own (at most 128 of them).  The
+// last launch also clears the fill cursors and writes the total to off[n].
+constexpr int SCAN_BLOCK = SCAN_THREADS * SCAN_ITEMS;
+
+__device__ __forceinline__ long long wave_sum_ll(long long s) {
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const int* __restrict__ count, int n,
                                                               long long* __restrict__ bsum) {
     __shared__ long long sh[SCAN_THREADS / 64];
-    const int base = blockIdx.x * SCAN_THREADS * SCAN_ITEMS;
+    const int base = blockIdx.x * SCAN_BLOCK;
     long long s = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         const int k = base + threadIdx.x * SCAN_ITEMS + i;
         if (k < n) s += count[k];
     }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    s = wave_sum_ll(s);
     if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -154,25 +225,13 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const int* __restr
     }
 }
 
-__global__ void k_scan_blocks(long long* __restrict__ bsum, int nb) {
-    // exclusive, in place; nb is small
-    if (threadIdx.x == 0) {
-        long long run = 0;
-        for (int i = 0; i < nb; ++i) {
-            const long long v = bsum[i];
-            bsum[i] = run;
-            run += v;
-        }
-        bsum[nb] = run;
-    }
-}
-
+// bsum: the block sums, or NULL when one block holds every tile.
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(const int* __restrict__ count, int n,
-                                                             const long long* __restrict__ bsum, int nb,
+                                                             const long long* __restrict__ bsum,
                                                              int* __restrict__ off, int* __restrict__ cursor) {
-    __shared__ long long part[SCAN_THREADS];
-    const int base = blockIdx.x * SCAN_THREADS * SCAN_ITEMS;
-    const int tid = threadIdx.x;
+    __shared__ long long wsum[SCAN_THREADS / 64], before;
+    const int base = blockIdx.x * SCAN_BLOCK;
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     int v[SCAN_ITEMS];
     long long s = 0;
 #pragma unroll
@@ -181,15 +240,22 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(const int* __restri
         v[i] = k < n ? count[k] : 0;
         s += v[i];
     }
-    part[tid] = s;
-    __syncthreads();
-    for (int o = 1; o < SCAN_THREADS; o <<= 1) {
-        const long long a = tid >= o ? part[tid - o] : 0;
-        __syncthreads();
-        part[tid] += a;
-        __syncthreads();
+    long long inc = s;  // inclusive scan within the wave
+    for (int o = 1; o < 64; o <<= 1) {
+        const long long up = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += up;
     }
-    long long run = bsum[blockIdx.x] + part[tid] - s;
+    if (lane == 63) wsum[wave] = inc;
+    if (wave == 0) {  // tiles of the blocks before this one
+        long long t = 0;
+        if (bsum)
+            for (int i = lane; i < (int)blockIdx.x; i += 64) t += bsum[i];
+        t = wave_sum_ll(t);
+        if (lane == 0) before = t;
+    }
+    __syncthreads();
+    long long run = before + inc - s;
+    for (int w = 0; w < wave; ++w) run += wsum[w];
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         const int k = base + tid * SCAN_ITEMS + i;
@@ -199,15 +265,17 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(const int* __restri
         }
         run += v[i];
     }
-    if (blockIdx.x == 0 && tid == 0) off[n] = (int)bsum[nb];
+    if (blockIdx.x == gridDim.x - 1 && tid == SCAN_THREADS - 1) off[n] = (int)run;
 }
 
 // Also reduces max |w| (as the bit pattern of a non-negative double: integer max of such patterns
-// orders them like the values, so the result is the same in any order) with one atomic per workgroup.
+// orders them like the values, so the result is the same in any order) with one atomic per workgroup.  SLOTS: the
+// slots were kept by the count; otherwise (catalogues too large to keep them) they are counted again.
+template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_proj_fill(const double* __restrict__ pos, const double* __restrict__ w,
                                                    int64_t n, double sf, int res, TileGeom g,
                                                    const int* __restrict__ off, int* __restrict__ cursor,
-                                                   ProjRec* __restrict__ rec, unsigned long long* __restrict__ wmax) {
+                                                   const int* __restrict__ slots, ProjRec* __restrict__ rec, unsigned long long* __restrict__ wmax) {
     __shared__ double wred[4];
     double mw = 0.0;
     const int m = g.L - 1;
@@ -233,8 +301,12 @@ __global__ __launch_bounds__(256) void k_proj_fill(const double* __restrict__ po
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int t = act ? replica_tile(g, X, Y, Z, nx, ny, nz, k) : -1;
-            const int slot = wave_add(cursor, t < 0 ? 0 : t, t >= 0);
-            if (t >= 0) rec[off[t] + slot] = r;
+            if (SLOTS) {
+                if (t >= 0) rec[off[t] + slots[(int64_t)k * n + p]] = r;
+            } else {
+                const int slot = wave_add(cursor, t < 0 ? 0 : t, t >= 0);
+                if (t >= 0) rec[off[t] + slot] = r;
+            }
         }
     }
     for (int o = 32; o > 0; o >>= 1) mw = fmax(mw, __shfl_xor(mw, o, 64));
@@ -287,8 +359,8 @@ __device__ __forceinline__ int acc_slot(int row, int lz, int lgtz) {
 // the tile loop (the next tile's first record chunk) are therefore issued unconditionally (clamped
 // index) before the current tile's stores, and every tile, empty or not, issues the same number of
 // stores; the wait at the top of the next tile then leaves this tile's stores in flight.
-template <bool COUNTS, bool FIXED, int OUTS>
-__global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
+template <bool COUNTS, bool FIXED, int OUTS, int NT>
+__global__ __launch_bounds__(NT) void k_proj_accumulate(
     const ProjRec* __restrict__ rec, const int* __restrict__ off, const double* __restrict__ phi, int res, TileGeom gg,
     const unsigned long long* __restrict__ wmax_bits, double phimax3, int ntiles, float* __restrict__ out32,
     double* __restrict__ out64, int32_t* __restrict__ counts_out) {
@@ -298,6 +370,7 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
         g.lgty = 3;
         g.lgtz = 6;
     }
+    constexpr int ACC_RCHUNK = 2 * NT;  // records staged per LDS chunk
     __shared__ __align__(16) long long acc[TILE_CELLS];
     __shared__ __align__(16) int cnt[COUNTS ? TILE_CELLS : 4];
     // the scaling function, resident for the workgroup's life, tap-interleaved: sphi[3 f + s] = phi[f + 1024 s],
@@ -311,35 +384,35 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
     const int ncell = tx * ty * tz;
     const int64_t L = g.L;
     // the host requires res == 1024 (3 * 1024 samples): all loads of the table in flight at once
-    static_assert((3 * 1024) % ACC_THREADS == 0, "phi table staging");
-    double ph[3 * 1024 / ACC_THREADS];
+    static_assert((3 * 1024) % NT == 0, "phi table staging");
+    double ph[3 * 1024 / NT];
 #pragma unroll
-    for (int j = 0; j < 3 * 1024 / ACC_THREADS; ++j) ph[j] = phi[tid + j * ACC_THREADS];
+    for (int j = 0; j < 3 * 1024 / NT; ++j) ph[j] = phi[tid + j * NT];
     const double unit = __longlong_as_double((long long)*wmax_bits) * phimax3;
 #pragma unroll
-    for (int j = 0; j < 3 * 1024 / ACC_THREADS; ++j) {
-        const int i = tid + j * ACC_THREADS;  // phi[i] = phi[f + 1024 s]
+    for (int j = 0; j < 3 * 1024 / NT; ++j) {
+        const int i = tid + j * NT;  // phi[i] = phi[f + 1024 s]
         sphi[3 * (i & 1023) + (i >> 10)] = ph[j];
     }
 
     // Software pipeline over this workgroup's tiles t, t+G, t+2G, ...: while tile t is processed, the
     // first record chunk of tile t+G is in flight into registers.
     const int G = gridDim.x;
-    constexpr int RPT = ACC_RCHUNK / ACC_THREADS;  // records per thread per chunk
+    constexpr int RPT = ACC_RCHUNK / NT;  // records per thread per chunk
     // This workgroup's tile ranges (begin, end) staged in LDS OFFCH tiles at a time: the loop then
     // issues no global loads for them (a refill, every OFFCH tiles, waits for the stores in flight).
     auto refill = [&](int k0) {
-        for (int i = tid; i < OFFCH; i += ACC_THREADS) {
+        for (int i = tid; i < OFFCH; i += NT) {
             const int tt = blockIdx.x + (k0 + i) * G;
             soff[i] = tt < ntiles ? make_int2(off[tt], off[tt + 1]) : make_int2(0, 0);
         }
     };
     // cell pairs per thread: a compile-time count, so the store count of the output phase is known to
     // the compiler and its waits can leave those stores in flight
-    constexpr int NPAIR = TILE_CELLS / (2 * ACC_THREADS);
+    constexpr int NPAIR = TILE_CELLS / (2 * NT);
 #pragma unroll
     for (int j = 0; j < NPAIR; ++j) {
-        const int i2 = tid * 2 + j * 2 * ACC_THREADS;
+        const int i2 = tid * 2 + j * 2 * NT;
         *(longlong2*)&acc[i2] = make_longlong2(0, 0);
         if (COUNTS) *(int2*)&cnt[i2] = make_int2(0, 0);
     }
@@ -352,15 +425,15 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
     const uint4* __restrict__ rec4 = (const uint4*)rec;
     uint4* srec4 = (uint4*)srec;
     {  // the first tile's first chunk, directly
-        const int i0 = beg + tid, i1 = beg + tid + ACC_THREADS;
+        const int i0 = beg + tid, i1 = beg + tid + NT;
         srec4[tid] = rec4[i0 < end ? i0 : 0];  // index 0 always exists; such entries are never read
-        srec4[tid + ACC_THREADS] = rec4[i1 < end ? i1 : 0];
+        srec4[tid + NT] = rec4[i1 < end ? i1 : 0];
     }
     // offset of each of this thread's cell pairs from its tile's first cell (the same for every tile)
     int loff[NPAIR];
 #pragma unroll
     for (int j = 0; j < NPAIR; ++j) {
-        const int i2 = tid * 2 + j * 2 * ACC_THREADS;
+        const int i2 = tid * 2 + j * 2 * NT;
         const int lz = i2 & (tz - 1), ly = (i2 >> g.lgtz) & (ty - 1), lx = i2 >> (g.lgtz + g.lgty);
         loff[j] = (lx * g.L + ly) * g.L + lz;
     }
@@ -381,7 +454,7 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
         // output stores (written at the end of the body, so the wait for it sees only in-loop paths)
         uint4 pref0, pref1;
         {
-            const int i0 = nbeg + tid, i1 = nbeg + tid + ACC_THREADS;
+            const int i0 = nbeg + tid, i1 = nbeg + tid + NT;
             pref0 = rec4[i0 < nend ? i0 : 0];
             pref1 = rec4[i1 < nend ? i1 : 0];
         }
@@ -398,12 +471,12 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
         for (int rb = beg; rb < end; rb += ACC_RCHUNK) {
             const int nr = end - rb < ACC_RCHUNK ? end - rb : ACC_RCHUNK;
             if (rb != beg) {
-                for (int r = tid; r < nr; r += ACC_THREADS) srec[r] = rec[rb + r];
+                for (int r = tid; r < nr; r += NT) srec[r] = rec[rb + r];
                 __syncthreads();
             }
             // items (record, x tap); y and z taps limited to the tile; 2^S folded into w (exact), so
             // each contribution is round((((w 2^S) phi_x) phi_y) phi_z)
-            for (int it = tid; it < nr * 3; it += ACC_THREADS) {
+            for (int it = tid; it < nr * 3; it += NT) {
                 const int r = it / 3, sx = it - 3 * r;
                 const ProjRec R = srec[r];
                 const int cx = R.cell & 1023;
@@ -429,7 +502,7 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
                 }
             }
             if (COUNTS) {
-                for (int r = tid; r < nr; r += ACC_THREADS) {
+                for (int r = tid; r < nr; r += NT) {
                     const ProjRec R = srec[r];
                     const int hx = (int)(R.cell & 1023) - ox, hy = (int)((R.cell >> 10) & 1023) - oy;
                     const int hz = (int)((R.cell >> 20) & 1023) - oz;
@@ -443,7 +516,7 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
         // cleared for the next tile as it is read
 #pragma unroll
         for (int j = 0; j < NPAIR; ++j) {
-            const int i2 = tid * 2 + j * 2 * ACC_THREADS;
+            const int i2 = tid * 2 + j * 2 * NT;
             if (!FIXED && i2 >= ncell) break;
             const int64_t gi = tbase + loff[j];
             const int ai = acc_slot<FIXED>(i2 >> g.lgtz, i2 & (tz - 1), g.lgtz);
@@ -463,23 +536,53 @@ __global__ __launch_bounds__(ACC_THREADS) void k_proj_accumulate(
         }
         // srec was last read by the tap loop, before the barrier that closed the last chunk
         srec4[tid] = pref0;
-        srec4[tid + ACC_THREADS] = pref1;
+        srec4[tid + NT] = pref1;
         beg = nbeg;
         end = nend;
     }
 }
 
+// 256 threads, three workgroups per CU; on grids with at most one tile per CU (J <= 6) 1024 threads, where a dense
+// catalogue puts thousands of records into each tile (500,000 particles at J = 6: 81 us with 256, 35 to 45 with 1024).
 template <bool COUNTS, bool FIXED>
-void launch_accumulate(int outs, int grid, hipStream_t st, const ProjRec* rec, const int* off, const double* phi,
+void launch_accumulate(int outs, int n_cu, hipStream_t st, const ProjRec* rec, const int* off, const double* phi,
                        int res, TileGeom g, const unsigned long long* wmax, double phimax3, int ntiles, float* out32,
                        double* out64, int32_t* counts) {
+    const bool few = ntiles <= n_cu;
+    const int grid = few ? ntiles : std::min(ntiles, 3 * n_cu);
+#define HERMES_ACC(OUTS)                                                                                              \
+    if (few)                                                                                                          \
+        k_proj_accumulate<COUNTS, FIXED, OUTS, ACC_THREADS_FEW><<<grid, ACC_THREADS_FEW, 0, st>>>(                     \
+            rec, off, phi, res, g, wmax, phimax3, ntiles, out32, out64, counts);                                      \
+    else                                                                                                              \
+        k_proj_accumulate<COUNTS, FIXED, OUTS, ACC_THREADS><<<grid, ACC_THREADS, 0, st>>>(rec, off, phi, res, g, wmax, \
+                                                                                          phimax3, ntiles, out32,     \
+                                                                                          out64, counts);             \
+    break;
     switch (outs) {
-        case 0: k_proj_accumulate<COUNTS, FIXED, 0><<<grid, ACC_THREADS, 0, st>>>(rec, off, phi, res, g, wmax, phimax3, ntiles, out32, out64, counts); break;
-        case 1: k_proj_accumulate<COUNTS, FIXED, 1><<<grid, ACC_THREADS, 0, st>>>(rec, off, phi, res, g, wmax, phimax3, ntiles, out32, out64, counts); break;
-        case 2: k_proj_accumulate<COUNTS, FIXED, 2><<<grid, ACC_THREADS, 0, st>>>(rec, off, phi, res, g, wmax, phimax3, ntiles, out32, out64, counts); break;
-        default: k_proj_accumulate<COUNTS, FIXED, 3><<<grid, ACC_THREADS, 0, st>>>(rec, off, phi, res, g, wmax, phimax3, ntiles, out32, out64, counts); break;
+        case 0: HERMES_ACC(0)
+        case 1: HERMES_ACC(1)
+        case 2: HERMES_ACC(2)
+        default: HERMES_ACC(3)
     }
+#undef HERMES_ACC
 }
+
+// Up to this worst case (8 records per particle) the records are reserved without a look at the count and the
+// slots of the count are kept.
+constexpr size_t RESERVE_BYTES = (size_t)2 << 30;
+
+// Tile workspace: max |w| (u64) | device error word and padding | count | off (ntiles + 1) | cursor | scan sums.
+struct TileWs {
+    size_t count, off, cursor, bsum, bytes;
+    explicit TileWs(int ntiles) {
+        count = 16;
+        off = count + sizeof(int) * (size_t)ntiles;
+        cursor = off + sizeof(int) * ((size_t)ntiles + 1);
+        bsum = (cursor + sizeof(int) * (size_t)ntiles + 15) / 16 * 16;
+        bytes = bsum + sizeof(long long) * (size_t)((ntiles + SCAN_BLOCK - 1) / SCAN_BLOCK);
+    }
+};
 
 int ilog2(int v) {
     int r = 0;
@@ -514,87 +617,96 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
     const double sf = (double)L / box;
     hipStream_t st = ctx->stream;
 
-    // tile workspace: (unused u64 slot) | count | off(ntiles+1) | cursor | err | scan block sums (i64)
-    const int nscan = (ntiles + SCAN_THREADS * SCAN_ITEMS - 1) / (SCAN_THREADS * SCAN_ITEMS);
-    size_t tile_bytes = (size_t)ntiles * 8 + (size_t)ntiles * 4 * 3 + 64 + (size_t)(nscan + 1) * 8 + 64;
-    char* tw = (char*)hermes_workspace(ctx, WS_PROJ_TILE, tile_bytes);
+    const TileWs tws(ntiles);
+    char* tw = (char*)hermes_workspace(ctx, WS_PROJ_TILE, tws.bytes);
     HERMES_REQUIRE(tw, "%s", hermes_last_error());
-    int* count = (int*)(tw + (size_t)ntiles * 8);
-    int* off = count + ntiles;
-    int* cursor = off + ntiles + 1;
-    int* err = cursor + ntiles;
-    long long* bsum = (long long*)(tw + (((size_t)ntiles * 8 + (size_t)ntiles * 4 * 3 + 16 + 15) / 16) * 16);
-    HERMES_CHECK_HIP(hermes_fill_u32(st, count, (size_t)ntiles, 0u));
-    unsigned long long* wmax = (unsigned long long*)tw;  // first 8 bytes of the u64 slot
-    HERMES_CHECK_HIP(hermes_fill_u32(st, wmax, 2, 0u));
+    unsigned long long* wmax = (unsigned long long*)tw;
+    int* count = (int*)(tw + tws.count);
+    int* off = (int*)(tw + tws.off);
+    int* cursor = (int*)(tw + tws.cursor);
+    long long* bsum = (long long*)(tw + tws.bsum);
+    const int nscan = (ntiles + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    HERMES_CHECK_HIP(hermes_fill_u32(st, tw, tws.count / 4 + (size_t)ntiles, 0u));
     // Invalid positions are projected at the origin (in bounds) and flagged: under stream capture in the
-    // context's sticky error word, eagerly in a word the call reads back before it returns (and fails).
-    int* errp = ctx->capturing ? ctx->dev_err : err;
+    // context's sticky error word, eagerly in a pinned host word read before the call returns (and fails).
+    int* errp = ctx->dev_err;
+    if (!ctx->capturing) {
+        errp = hermes_host_word(ctx);
+        HERMES_REQUIRE(errp, "%s", hermes_last_error());
+        *(volatile int*)errp = 0;
+    }
     HERMES_REQUIRE(errp, "hermes_project: no device error word");
-    if (!ctx->capturing) HERMES_CHECK_HIP(hermes_fill_u32(st, err, 1, 0u));
 
-    k_proj_count<<<hermes_blocks(n, 256, 4096), 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out,
-                                                              errp);
-    HERMES_LAUNCH_CHECK();
-    k_scan_reduce<<<nscan, SCAN_THREADS, 0, st>>>(count, ntiles, bsum);
-    HERMES_LAUNCH_CHECK();
-    k_scan_blocks<<<1, 64, 0, st>>>(bsum, nscan);
-    HERMES_LAUNCH_CHECK();
-    k_scan_apply<<<nscan, SCAN_THREADS, 0, st>>>(count, ntiles, bsum, nscan, off, cursor);
-    HERMES_LAUNCH_CHECK();
     // Records: a particle's 3-cell footprint meets at most 2 tiles per axis (tile sides >= 4), so 8n
     // records always suffice.  Up to RESERVE_BYTES that worst case is reserved and the kernels run back
     // to back, the positions checked once at the end; larger catalogues are sized exactly after the
     // count (a host synchronisation).  Capturing always uses the worst case (hermes_project_reserve).
-    constexpr size_t RESERVE_BYTES = (size_t)2 << 30;
     const size_t worst = (size_t)(n > 0 ? 8 * n : 1) * sizeof(ProjRec);
+    int* slots = nullptr;
+    if (n > 0 && worst <= RESERVE_BYTES) {
+        slots = (int*)hermes_workspace(ctx, WS_PROJ_SLOT, sizeof(int) * 8 * (size_t)n);
+        HERMES_REQUIRE(slots, "%s%s", hermes_last_error(), ctx->capturing ? " (hermes_project_reserve sizes it)" : "");
+    }
+    if (slots && ntiles <= LDS_TILES) {
+        // more particles per workgroup aggregate better, once there are workgroups enough to fill the chip
+        const size_t lds = sizeof(int) * ntiles;
+        if (n >= 4 * 256 * 256)
+            k_proj_count_lds<4><<<(unsigned)((n + 1023) / 1024), 256, lds, st>>>(pos, n, sf, phi_res, g, ntiles, count,
+                                                                                cell_out, frac_out, errp, slots);
+        else
+            k_proj_count_lds<1><<<(unsigned)((n + 255) / 256), 256, lds, st>>>(pos, n, sf, phi_res, g, ntiles, count,
+                                                                              cell_out, frac_out, errp, slots);
+    } else {
+        k_proj_count<<<hermes_blocks(n, 256, 4096), 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out,
+                                                                  errp, slots);
+    }
+    HERMES_LAUNCH_CHECK();
+    if (nscan > 1) {
+        k_scan_reduce<<<nscan, SCAN_THREADS, 0, st>>>(count, ntiles, bsum);
+        HERMES_LAUNCH_CHECK();
+    }
+    k_scan_apply<<<nscan, SCAN_THREADS, 0, st>>>(count, ntiles, nscan > 1 ? bsum : nullptr, off, cursor);
+    HERMES_LAUNCH_CHECK();
     ProjRec* rec = nullptr;
-    bool checked = false;
     if (ctx->capturing || worst <= RESERVE_BYTES) {
         rec = (ProjRec*)hermes_workspace(ctx, WS_PROJ_REC, worst);
         HERMES_REQUIRE(rec, "%s%s", hermes_last_error(), ctx->capturing ? " (hermes_project_reserve sizes it)" : "");
     } else {
-        int host[2] = {0, 0};
-        HERMES_CHECK_HIP(hipMemcpyAsync(&host[0], err, sizeof(int), hipMemcpyDeviceToHost, st));
-        HERMES_CHECK_HIP(hipMemcpyAsync(&host[1], off + ntiles, sizeof(int), hipMemcpyDeviceToHost, st));
+        int total = 0;
+        HERMES_CHECK_HIP(hipMemcpyAsync(&total, off + ntiles, sizeof(int), hipMemcpyDeviceToHost, st));
         HERMES_CHECK_HIP(hipStreamSynchronize(st));
-        HERMES_REQUIRE(host[0] == 0, "hermes_project: non-finite or out-of-range particle positions");
-        checked = true;
-        const int total = host[1];
+        HERMES_REQUIRE(*(volatile int*)errp == 0, "hermes_project: non-finite or out-of-range particle positions");
         rec = (ProjRec*)hermes_workspace(ctx, WS_PROJ_REC, (size_t)(total > 0 ? total : 1) * sizeof(ProjRec));
         HERMES_REQUIRE(rec, "%s", hermes_last_error());
     }
     if (n > 0) {
-        k_proj_fill<<<hermes_blocks(n, 256, 4096), 256, 0, st>>>(pos, w, n, sf, phi_res, g, off, cursor, rec,
-                                                                 wmax);
+        const unsigned nb = hermes_blocks(n, 256, 4096);
+        if (slots) k_proj_fill<true><<<nb, 256, 0, st>>>(pos, w, n, sf, phi_res, g, off, cursor, slots, rec, wmax);
+        else k_proj_fill<false><<<nb, 256, 0, st>>>(pos, w, n, sf, phi_res, g, off, cursor, slots, rec, wmax);
         HERMES_LAUNCH_CHECK();
     }
     const double phimax3 = phi_abs_max * phi_abs_max * phi_abs_max * (1.0 + 1e-12);
-    int n_cu = 256;
-    (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device);
-    const int acc_grid = ntiles < 3 * n_cu ? ntiles : 3 * n_cu;
     const bool full = g.lgtx == 2 && g.lgty == 3 && g.lgtz == 6;
     const int outs = (eps32 ? 1 : 0) | (eps64 ? 2 : 0);
     if (cell_counts) {
         if (full)
-            launch_accumulate<true, true>(outs, acc_grid, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
+            launch_accumulate<true, true>(outs, ctx->n_cu, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
                                           eps64, cell_counts);
         else
-            launch_accumulate<true, false>(outs, acc_grid, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
+            launch_accumulate<true, false>(outs, ctx->n_cu, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
                                            eps64, cell_counts);
     } else {
         if (full)
-            launch_accumulate<false, true>(outs, acc_grid, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
+            launch_accumulate<false, true>(outs, ctx->n_cu, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
                                            eps64, nullptr);
         else
-            launch_accumulate<false, false>(outs, acc_grid, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
+            launch_accumulate<false, false>(outs, ctx->n_cu, st, rec, off, phi, phi_res, g, wmax, phimax3, ntiles, eps32,
                                             eps64, nullptr);
     }
     HERMES_LAUNCH_CHECK();
-    if (!ctx->capturing && !checked) {  // invalid positions were projected at the origin (in bounds)
-        int host_err = 0;
-        if (hermes_read_word(ctx, err, &host_err)) return 1;
-        HERMES_REQUIRE(host_err == 0, "hermes_project: non-finite or out-of-range particle positions");
+    if (!ctx->capturing) {  // invalid positions were projected at the origin (in bounds)
+        if (hermes_poll_stream(ctx)) return 1;
+        HERMES_REQUIRE(*(volatile int*)errp == 0, "hermes_project: non-finite or out-of-range particle positions");
     }
     return 0;
 }
@@ -611,9 +723,10 @@ extern "C" int hermes_project_reserve(hermes_ctx* ctx, int J, int64_t n_max) {
     const int lgtx = ilog2(L < MAX_TX ? L : MAX_TX), lgty = ilog2(L < MAX_TY ? L : MAX_TY),
               lgtz = ilog2(L < MAX_TZ ? L : MAX_TZ);
     const int ntiles = 1 << (3 * J - lgtx - lgty - lgtz);
-    const int nscan = (ntiles + SCAN_THREADS * SCAN_ITEMS - 1) / (SCAN_THREADS * SCAN_ITEMS);
-    const size_t tile_bytes = (size_t)ntiles * 8 + (size_t)ntiles * 4 * 3 + 64 + (size_t)(nscan + 1) * 8 + 64;
-    HERMES_REQUIRE(hermes_workspace(ctx, WS_PROJ_TILE, tile_bytes), "%s", hermes_last_error());
+    HERMES_REQUIRE(hermes_workspace(ctx, WS_PROJ_TILE, TileWs(ntiles).bytes), "%s", hermes_last_error());
+    const int64_t n_slot = std::min<int64_t>(n_max, RESERVE_BYTES / (8 * sizeof(ProjRec)));
+    if (n_slot > 0)
+        HERMES_REQUIRE(hermes_workspace(ctx, WS_PROJ_SLOT, sizeof(int) * 8 * (size_t)n_slot), "%s", hermes_last_error());
     HERMES_REQUIRE(hermes_workspace(ctx, WS_PROJ_REC, (size_t)(n_max > 0 ? 8 * n_max : 1) * sizeof(ProjRec)), "%s",
                    hermes_last_error());
     return 0;
