@@ -89,7 +89,7 @@ int hermes_delta_f32(hermes_ctx *ctx, int64_t n, const float *eps, double a, dou
 int hermes_half_spectrum_f32(hermes_ctx *ctx, int J, const void *full, void *half);
 
 
-/* ---- 3-D FFTs (rocFFT), replacing scipy.fft rfftn / irfftn / fftn / ifftn in
+/* ---- 3-D FFTs (rocFFT plans; from 128^3 on the strided lines by own kernels), replacing scipy.fft rfftn / irfftn / fftn / ifftn in
  * convolution.py:284-295.  Unnormalised; batch transforms are contiguous
  * (batch, L, L, L).  c2r clobbers its input.  in == out selects in-place (c2c only). */
 int hermes_fft_r2c(hermes_ctx *ctx, int J, int batch, int dbl, const void *in_real, void *out_half);

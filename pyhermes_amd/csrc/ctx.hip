@@ -119,6 +119,7 @@ int hermes_ctx_destroy(hermes_ctx* ctx) {
         if (ctx->ws[i]) (void)hipFree(ctx->ws[i]);
     hermes_fft_cache_destroy(ctx->fft);
     if (ctx->twiddles) (void)hipFree(ctx->twiddles);
+    if (ctx->twiddles64) (void)hipFree(ctx->twiddles64);
     if (ctx->dev_err) (void)hipFree(ctx->dev_err);
     if (ctx->host_word) (void)hipHostFree(ctx->host_word);
     for (hipEvent_t e : ctx->gram_ev) (void)hipEventDestroy(e);

@@ -1,5 +1,7 @@
-// 3-D FFTs over (L, L, L) grids with rocFFT; plans cached per context.
+// 3-D FFTs over (L, L, L) grids; plans cached per context.
 // Replaces scipy.fft rfftn/irfftn/fftn/ifftn in convolution.py:284-295.
+// Grids of 128^3 and more: the contiguous z lines by a 1-D rocFFT plan (it runs at the rate of a copy), the strided y
+// and x lines by k_fft_lines.  Smaller ones: a 3-D rocFFT plan.
 // Transforms are unnormalised (the inverse is not divided by N); callers fold
 // 1/N into the spectral multiply.
 #include <rocfft/rocfft.h>
@@ -9,6 +11,7 @@
 #include <tuple>
 
 #include "../../include/hermes_amd.h"
+#include "fft_lds.h"
 #include "hermes_common.h"
 
 namespace {
@@ -21,8 +24,8 @@ struct Plan {
     void* work = nullptr;
 };
 
-// key: (L, kind, double, batch, inplace, interleaved batch)
-using PlanKey = std::tuple<int, int, int, int, int, int>;
+// key: (L, kind, double, batch, inplace, dimensions)
+using PlanKey = std::tuple<int, int, int, int64_t, int, int>;
 }  // namespace
 
 struct hermes_fft_cache {
@@ -41,12 +44,11 @@ void hermes_fft_cache_destroy(hermes_fft_cache* c) {
 
 namespace {
 // kind: 0 = r2c forward, 1 = c2r inverse, 2 = c2c forward, 3 = c2c inverse
-// ibatch != 0: complex transforms whose batch index is the fastest axis
-// (element stride = batch, batch distance = 1), i.e. data laid out (L, L, L, batch).
-int get_plan(hermes_ctx* ctx, int L, int kind, int dbl, int batch, int inplace, int ibatch, Plan** out) {
+// dims = 3: batch grids; dims = 1: batch contiguous lines of L values.
+int get_plan(hermes_ctx* ctx, int L, int kind, int dbl, int64_t batch, int inplace, int dims, Plan** out) {
     std::call_once(g_rocfft_once, []() { rocfft_setup(); });
     if (!ctx->fft) ctx->fft = new hermes_fft_cache();
-    PlanKey key{L, kind, dbl, batch, inplace, ibatch};
+    PlanKey key{L, kind, dbl, batch, inplace, dims};
     auto it = ctx->fft->plans.find(key);
     if (it != ctx->fft->plans.end()) {
         *out = &it->second;
@@ -60,19 +62,10 @@ int get_plan(hermes_ctx* ctx, int L, int kind, int dbl, int batch, int inplace, 
                                            : rocfft_transform_type_complex_inverse;
     rocfft_precision prec = dbl ? rocfft_precision_double : rocfft_precision_single;
     rocfft_result_placement pl = inplace ? rocfft_placement_inplace : rocfft_placement_notinplace;
-    rocfft_plan_description desc = nullptr;
-    if (ibatch) {
-        rocfft_plan_description_create(&desc);
-        size_t strides[3] = {(size_t)batch, (size_t)batch * L, (size_t)batch * L * L};
-        rocfft_plan_description_set_data_layout(desc, rocfft_array_type_complex_interleaved,
-                                                rocfft_array_type_complex_interleaved, nullptr, nullptr, 3, strides, 1,
-                                                3, strides, 1);
-    }
-    rocfft_status s = rocfft_plan_create(&p.plan, pl, tt, prec, 3, lengths, (size_t)batch, desc);
-    if (desc) rocfft_plan_description_destroy(desc);
+    rocfft_status s = rocfft_plan_create(&p.plan, pl, tt, prec, (size_t)dims, lengths, (size_t)batch, nullptr);
     if (s != rocfft_status_success) {
-        hermes_set_error("rocfft_plan_create failed (status %d) L=%d kind=%d dbl=%d batch=%d", (int)s, L, kind,
-                         dbl, batch);
+        hermes_set_error("rocfft_plan_create failed (status %d) L=%d kind=%d dbl=%d batch=%lld", (int)s, L, kind,
+                         dbl, (long long)batch);
         return 3;
     }
     rocfft_plan_get_work_buffer_size(p.plan, &p.work_bytes);
@@ -89,15 +82,10 @@ int get_plan(hermes_ctx* ctx, int L, int kind, int dbl, int batch, int inplace, 
     return 0;
 }
 
-int run(hermes_ctx* ctx, int J, int kind, int dbl, int batch, const void* in, void* out, int ibatch = 0) {
-    HERMES_REQUIRE(ctx, "null context");
-    HERMES_REQUIRE(J >= 1 && J <= 10, "FFT: J=%d unsupported", J);
-    HERMES_REQUIRE(batch >= 1, "FFT: batch must be >= 1");
-    HERMES_CHECK_HIP(hipSetDevice(ctx->device));
-    int inplace = (in == out) ? 1 : 0;
-    HERMES_REQUIRE(!(inplace && (kind == 0 || kind == 1)), "real<->complex FFTs must be out of place");
+int run_plan(hermes_ctx* ctx, int J, int kind, int dbl, int64_t batch, int dims, const void* in, void* out) {
+    const int inplace = (in == out) ? 1 : 0;
     Plan* p = nullptr;
-    int rc = get_plan(ctx, 1 << J, kind, dbl, batch, inplace, ibatch, &p);
+    int rc = get_plan(ctx, 1 << J, kind, dbl, batch, inplace, dims, &p);
     if (rc) return rc;
     rocfft_execution_info_set_stream(p->info, ctx->stream);
     void* ib[1] = {const_cast<void*>(in)};
@@ -108,6 +96,101 @@ int run(hermes_ctx* ctx, int J, int kind, int dbl, int batch, const void* in, vo
         return 3;
     }
     return 0;
+}
+
+// Strided lines of L = 2^LOG2L values, in place: element e of column c of block o is at o * outer + c + e * es, c < ncols
+// (y lines: a block is an x plane, its columns the z of a row; x lines: one block, its columns the positions of a
+// plane).  A workgroup stages TW columns in LDS, so every access is a run of TW values and each value is read and
+// written once; bound by HBM.  TW values are one 128-byte line (for half spectra the rows of y lines, L / 2 + 1 values
+// apart, start anywhere in a line: neighbouring tiles, on one XCD, share it in its L2).  Plain loads and stores: with
+// the streaming hint the shared lines and what the previous pass left in the last-level cache are lost (512^3 FP32,
+// y lines: 218 us plain, 446 streaming; 256^3 FP64, x lines: 40 and 80).  The library's strided kernels took 598 us
+// (512^3 FP32, half spectrum: 1.8 TB/s; now y 218, x 272) and 86 us (256^3 FP64: 3.1 TB/s; now 39 and 40).
+template <class C, int LOG2L, int TW, int NT, int DIR>
+__global__ __launch_bounds__(NT) void k_fft_lines(C* data, const C* __restrict__ twg, int64_t es, int64_t outer,
+                                                  int64_t ncols, int ntile) {
+    constexpr int L = 1 << LOG2L;
+    static_assert(NT % TW == 0 && TW * L % NT == 0, "a thread keeps one column of the tile");
+    using F = hermes_fft::LdsFft<LOG2L, TW, NT, DIR, true, C>;
+    extern __shared__ __align__(16) char lines_lds[];
+    C* tw = (C*)lines_lds;
+    C* lds = tw + L;
+    const int tid = threadIdx.x;
+    // workgroups are dealt to the 8 XCDs round-robin: each XCD takes a contiguous range of tiles
+    const int64_t nb = gridDim.x, xcd = blockIdx.x % 8, rem = nb % 8;
+    const int64_t b = xcd * (nb / 8) + (xcd < rem ? xcd : rem) + blockIdx.x / 8;
+    const int64_t col = (b % ntile) * TW + tid % TW;
+    const bool inside = col < ncols;  // the last tile of a block may be partly empty
+    C* p = data + (b / ntile) * outer + (inside ? col : 0) + (int64_t)(tid / TW) * es;
+    const int64_t step = (int64_t)(NT / TW) * es;
+    hermes_fft::load_twiddles<LOG2L>(tw, twg, tid, NT);
+    constexpr int PER = TW * L / NT;
+    C v[PER];  // the whole tile is in flight before the first store to LDS
+#pragma unroll
+    for (int k = 0; k < PER; ++k) v[k] = p[k * step];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) lds[tid + k * NT] = v[k];
+    __syncthreads();
+    F::run(lds, tw, tid);
+    if (!inside) return;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) p[k * step] = lds[tid + k * NT];
+}
+
+// y and x lines of `batch` grids of (L, L, M) values, in place.
+template <class C, int LOG2L, int DIR>
+int run_lines(hermes_ctx* ctx, int64_t batch, int64_t M, C* data, const C* twg) {
+    constexpr int L = 1 << LOG2L;
+    constexpr int TW = LOG2L == 7 ? 16 : 128 / (int)sizeof(C);  // 128^3: 16 in FP64 as well (21 us for 24 with 8)
+    constexpr int NT = TW * L > 4096 ? 512 : 256;
+    constexpr size_t lds = sizeof(C) * (size_t)(L + TW * L);
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    auto k = k_fft_lines<C, LOG2L, TW, NT, DIR>;
+    HERMES_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int64_t yt = (M + TW - 1) / TW, xt = (L * M + TW - 1) / TW;
+    k<<<(unsigned)(batch * L * yt), NT, lds, ctx->stream>>>(data, twg, M, L * M, M, (int)yt);
+    HERMES_LAUNCH_CHECK();
+    k<<<(unsigned)(batch * xt), NT, lds, ctx->stream>>>(data, twg, L * M, L * L * M, L * M, (int)xt);
+    HERMES_LAUNCH_CHECK();
+    return 0;
+}
+
+template <class C, int DIR>
+int lines(hermes_ctx* ctx, int J, int64_t batch, int64_t M, C* data, const C* twg) {
+    HERMES_REQUIRE(twg, "%s", hermes_last_error());
+    switch (J) {
+        case 7: return run_lines<C, 7, DIR>(ctx, batch, M, data, twg);
+        case 8: return run_lines<C, 8, DIR>(ctx, batch, M, data, twg);
+        case 9: return run_lines<C, 9, DIR>(ctx, batch, M, data, twg);
+        default: return run_lines<C, 10, DIR>(ctx, batch, M, data, twg);
+    }
+}
+
+int strided(hermes_ctx* ctx, int J, int dbl, int64_t batch, int64_t M, int dir, void* data) {
+    if (dbl)
+        return dir > 0 ? lines<double2, 1>(ctx, J, batch, M, (double2*)data, hermes_twiddles_f64(ctx, J, 1))
+                       : lines<double2, -1>(ctx, J, batch, M, (double2*)data, hermes_twiddles_f64(ctx, J, -1));
+    return dir > 0 ? lines<float2, 1>(ctx, J, batch, M, (float2*)data, hermes_twiddles(ctx, J, 1))
+                   : lines<float2, -1>(ctx, J, batch, M, (float2*)data, hermes_twiddles(ctx, J, -1));
+}
+
+// Own strided passes from 128^3 on.  Below, the 3-D plan takes two launches (64^3: 13 us) and this way three.
+constexpr int LINES_MIN_J = 7;
+
+int run(hermes_ctx* ctx, int J, int kind, int dbl, int batch, const void* in, void* out) {
+    HERMES_REQUIRE(ctx, "null context");
+    HERMES_REQUIRE(J >= 1 && J <= 10, "FFT: J=%d unsupported", J);
+    HERMES_REQUIRE(batch >= 1, "FFT: batch must be >= 1");
+    HERMES_CHECK_HIP(hipSetDevice(ctx->device));
+    HERMES_REQUIRE(!(in == out && (kind == 0 || kind == 1)), "real<->complex FFTs must be out of place");
+    if (J < LINES_MIN_J) return run_plan(ctx, J, kind, dbl, batch, 3, in, out);
+    const int64_t L = (int64_t)1 << J, nlines = batch * L * L;
+    if (kind == 1) {  // the real lines last
+        const int rc = strided(ctx, J, dbl, batch, L / 2 + 1, 1, const_cast<void*>(in));
+        return rc ? rc : run_plan(ctx, J, kind, dbl, nlines, 1, in, out);
+    }
+    const int rc = run_plan(ctx, J, kind, dbl, nlines, 1, in, out);
+    return rc ? rc : strided(ctx, J, dbl, batch, kind == 0 ? L / 2 + 1 : L, kind == 3 ? 1 : -1, out);
 }
 }  // namespace
 

@@ -16,35 +16,46 @@
 using namespace hermes_fft;
 
 // e^{dir 2 pi i k / 2^j} for j = 0..10, k < 2^j, computed in FP64 and rounded once.
-const float2* hermes_twiddles(hermes_ctx* ctx, int log2L, int dir) {
-    if (!ctx->twiddles && ctx->capturing) {
+template <class C, class T>
+static const C* twiddle_table(hermes_ctx* ctx, C*& table, int log2L, int dir) {
+    if (!table && ctx->capturing) {
         hermes_set_error("FFT twiddle tables are built on first use; run an FFT once before capturing");
         return nullptr;
     }
-    if (!ctx->twiddles) {
-        std::vector<float2> h((size_t)11 * 2 * 1024);
+    if (!table) {
+        std::vector<C> h((size_t)11 * 2 * 1024);
         for (int j = 0; j <= 10; ++j)
             for (int d = 0; d < 2; ++d) {
                 const int L = 1 << j;
                 const double sgn = d ? 1.0 : -1.0;
                 for (int k = 0; k < L; ++k) {
                     const double a = 2.0 * M_PI * (double)k / (double)L;
-                    h[(size_t)(j * 2 + d) * 1024 + k] = make_float2((float)cos(a), (float)(sgn * sin(a)));
+                    C& w = h[(size_t)(j * 2 + d) * 1024 + k];
+                    w.x = (T)cos(a);
+                    w.y = (T)(sgn * sin(a));
                 }
             }
-        float2* p = nullptr;
-        if (hipMalloc(&p, h.size() * sizeof(float2)) != hipSuccess) {
+        C* p = nullptr;
+        if (hipMalloc(&p, h.size() * sizeof(C)) != hipSuccess) {
             hermes_set_error("hipMalloc of the twiddle table failed");
             return nullptr;
         }
-        if (hipMemcpy(p, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
+        if (hipMemcpy(p, h.data(), h.size() * sizeof(C), hipMemcpyHostToDevice) != hipSuccess) {
             (void)hipFree(p);
             hermes_set_error("upload of the twiddle table failed");
             return nullptr;
         }
-        ctx->twiddles = p;
+        table = p;
     }
-    return ctx->twiddles + (size_t)(log2L * 2 + (dir > 0 ? 1 : 0)) * 1024;
+    return table + (size_t)(log2L * 2 + (dir > 0 ? 1 : 0)) * 1024;
+}
+
+const float2* hermes_twiddles(hermes_ctx* ctx, int log2L, int dir) {
+    return twiddle_table<float2, float>(ctx, ctx->twiddles, log2L, dir);
+}
+
+const double2* hermes_twiddles_f64(hermes_ctx* ctx, int log2L, int dir) {
+    return twiddle_table<double2, double>(ctx, ctx->twiddles64, log2L, dir);
 }
 
 namespace {

@@ -35,6 +35,7 @@ struct hermes_ctx {
     size_t ws_size[HERMES_WS_SLOTS] = {0};
     hermes_fft_cache* fft = nullptr;
     float2* twiddles = nullptr;  // e^{+-2 pi i k / 2^j} tables for the LDS FFTs (first use)
+    double2* twiddles64 = nullptr;
     // autotuned strided-pass tile per (log2 L, inverse, axis: 0 = y lines, 1 = x lines); 0 = not tuned
     int fft_cols_variant[11][2][2] = {};
     // layout of the FP32 fields the Gram contractions read (hermes_set_field_layout): 0 = x-major, 1 = y-major
@@ -68,6 +69,8 @@ int* hermes_host_word(hermes_ctx* ctx);
 int hermes_poll_stream(hermes_ctx* ctx);
 // Twiddle table e^{dir 2 pi i k / 2^log2L}, k < 2^log2L (device memory owned by ctx).
 const float2* hermes_twiddles(hermes_ctx* ctx, int log2L, int dir);
+// The same in FP64.
+const double2* hermes_twiddles_f64(hermes_ctx* ctx, int log2L, int dir);
 // Inverse FFT along y and x of a batch of (L, L, L) complex64 grids already transformed along z.
 int hermes_fft3_inverse_yx(hermes_ctx* ctx, int J, int batch, float2* data);
 
