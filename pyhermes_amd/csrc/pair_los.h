@@ -69,8 +69,10 @@ __global__ __launch_bounds__(LOS_THREADS, 2) void k_pair_los(int L, int axis, co
             const int r = axis == 2 ? e / LhP : e % LOS_ROWS, q = axis == 2 ? e % LhP : e / LOS_ROWS;
             const int p = pt * LOS_ROWS + r, u = p / Lh, v = p % Lh;
             double s = 0.0;
-            if (p < nperp && q <= half)
-                s = octant_power(F1, F2, L, axis == 0 ? q : u, axis == 0 ? u : (axis == 1 ? q : v), axis == 2 ? q : v);
+            if (p < nperp && q <= half) {
+                const int x = axis == 0 ? q : u, y = axis == 0 ? u : (axis == 1 ? q : v), z = axis == 2 ? q : v;
+                s = F1 == F2 ? octant_power<true>(F1, F2, L, x, y, z) : octant_power<false>(F1, F2, L, x, y, z);
+            }
             S[q * LOS_PITCH + r] = s;
         }
         __syncthreads();

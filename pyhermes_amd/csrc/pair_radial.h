@@ -14,11 +14,16 @@
 // follow by the upward recurrence for x >= XMIN (where the second solution, which amplifies rounding, is of
 // order one) and otherwise by the power series of the two top orders and the downward recurrence.
 //
-// Bound by FP64 VALU.  Thin shells and l = 0, 2, 4 at 30 radii: 5.70 ms per pass at L = 512 (FP32 spectra) and
-// 5.36 ms at L = 256 (FP64) with one thread per position, an FP32 sin/cos or an FP64 sincos and divisions per
-// (alias, radius), and a wave reduction per channel and position; now 1.23 ms and 0.20 ms.
+// Bound by FP64 VALU issue (about 0.6 ms of instructions at L = 512) with the gather of the powers, 0.3 ms, partly
+// beside it: 250 registers leave two waves per SIMD.  Thin shells and l = 0, 2, 4 at 30 radii: 5.70 ms per pass at
+// L = 512 (FP32 spectra) and 5.36 ms at L = 256 (FP64) with one thread per position, an FP32 sin/cos or an FP64
+// sincos and divisions per (alias, radius), and a wave reduction per channel and position; 1.23 ms and 0.20 ms with
+// this sharing; 0.93 and 0.18 with unconditional loads, one series test per radius and everything a step needs
+// fetched a step ahead.  Four aliases at a time and three waves per SIMD: 1.04 and 0.23 (twice the reductions).
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "special.h"
 
@@ -64,20 +69,27 @@ __device__ __forceinline__ double quad_sum(double v0, double v1, double v2, doub
 }
 __device__ __forceinline__ int quad_of_row(int row) { return ((row & 1) << 1) | (row >> 1); }
 
-// sum over the mirror modes (x | L-x, y | L-y, z | L-z) of Re F1 conj F2 from the half spectra.
-template <typename C>
+// sum over the mirror modes (x | L-x, y | L-y, z | L-z) of Re F1 conj F2 from the half spectra (SAME: F2 is F1).  The
+// four loads are unconditional, a mirror that is the mode itself is left out afterwards: a load under a condition is
+// waited for before the next one is issued.
+template <bool SAME, typename C>
 __device__ __forceinline__ double octant_power(const C* __restrict__ F1, const C* __restrict__ F2, int L, int x, int y,
                                                int z) {
     const int Lh = L / 2 + 1;
     const int xm = (L - x) & (L - 1), ym = (L - y) & (L - 1);
     const double wz = (z == 0 || z == L / 2) ? 1.0 : 2.0;
+    C f[4], g[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const int64_t i = ((int64_t)(a >> 1 ? xm : x) * L + ((a & 1) ? ym : y)) * Lh + z;
+        f[a] = F1[i];
+        g[a] = SAME ? f[a] : F2[i];
+    }
     double p = 0.0;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-        if ((a >> 1 && xm == x) || ((a & 1) && ym == y)) continue;
-        const int64_t i = ((int64_t)(a >> 1 ? xm : x) * L + ((a & 1) ? ym : y)) * Lh + z;
-        const C f = F1[i], g = F2[i];
-        p += wz * ((double)f.x * (double)g.x + (double)f.y * (double)g.y);
+        const double t = (double)f[a].x * (double)g[a].x + (double)f[a].y * (double)g[a].y;
+        p += ((a >> 1 && xm == x) || ((a & 1) && ym == y)) ? 0.0 : wz * t;
     }
     return p;
 }
@@ -132,8 +144,12 @@ constexpr int radial_threads() {
 
 __host__ __device__ inline int tetra(int n) { return n * (n + 1) * (n + 2) / 6; }
 
+// Aliases whose state (6 + LMAX / 2 doubles each) a thread holds at a time: all eight in 256 registers up to l = 4;
+// beyond, eight leave 160 registers in scratch, four 60.
+constexpr int radial_aliases(int lmax) { return lmax <= 4 ? 8 : 4; }
+
 template <int LMAX, bool ROT, int BT, typename C>
-__global__ __launch_bounds__(radial_threads<BT>()) void k_pair_radial(int L, const C* __restrict__ F1,
+__global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, const C* __restrict__ F1,
                                                                       const C* __restrict__ F2,
                                                                       const double* __restrict__ P,
                                                                       const double* __restrict__ radii, int nu,
@@ -143,6 +159,7 @@ __global__ __launch_bounds__(radial_threads<BT>()) void k_pair_radial(int L, con
     constexpr int NT = radial_threads<BT>(), NW = NT / 64, B3 = BT * BT * BT, PER = B3 / NT;
     constexpr int NE = LMAX / 2 + 1;         // even orders
     constexpr int UC = LMAX == 0 ? 4 : 1;    // radii per reduction
+    constexpr int NA = radial_aliases(LMAX);
     constexpr int NQ = (UC * NE + 3) / 4;    // groups of four wave sums
     constexpr double XMIN = radial_xmin(LMAX);
     extern __shared__ double wacc[];  // [waves][nch]
@@ -162,18 +179,23 @@ __global__ __launch_bounds__(radial_threads<BT>()) void k_pair_radial(int L, con
         while ((bj + 1) * (bj + 2) / 2 <= rem) ++bj;
         const int bk = rem - bj * (bj + 1) / 2;
         __syncthreads();  // the previous block's powers and list are consumed
+        auto gather = [&](auto same) {
 #pragma unroll
-        for (int o = 0; o < 6; ++o) {
-            const int X = (o == 0 || o == 2) ? bi : ((o == 1 || o == 4) ? bj : bk);
-            const int Y = (o == 1 || o == 3) ? bi : ((o == 0 || o == 5) ? bj : bk);
-            const int Z = (o >= 4) ? bi : (o >= 2 ? bj : bk);
+            for (int o = 0; o < 6; ++o) {
+                const int X = (o == 0 || o == 2) ? bi : ((o == 1 || o == 4) ? bj : bk);
+                const int Y = (o == 1 || o == 3) ? bi : ((o == 0 || o == 5) ? bj : bk);
+                const int Z = (o >= 4) ? bi : (o >= 2 ? bj : bk);
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const int r = tid + q * NT;
-                const int x = X * BT + r / (BT * BT), y = Y * BT + (r / BT) % BT, z = Z * BT + r % BT;
-                pw[o * B3 + r] = (x <= half && y <= half && z <= half) ? octant_power(F1, F2, L, x, y, z) : 0.0;
+                for (int q = 0; q < PER; ++q) {
+                    const int r = tid + q * NT;
+                    const int x = X * BT + r / (BT * BT), y = Y * BT + (r / BT) % BT, z = Z * BT + r % BT;
+                    const double p = octant_power<decltype(same)::value>(F1, F2, L, min(x, half), min(y, half), min(z, half));
+                    pw[o * B3 + r] = (x <= half && y <= half && z <= half) ? p : 0.0;
+                }
             }
-        }
+        };
+        if (F1 == F2) gather(std::true_type());
+        else gather(std::false_type());
         // the sorted triples of the block, in order
         bool val[PER];
         int rank[PER];
@@ -211,86 +233,118 @@ __global__ __launch_bounds__(radial_threads<BT>()) void k_pair_radial(int L, con
                 if (j != k) pi += at(5, c0, b0, a0);
             }
             if (!active) pk = pj = pi = 0.0;
-            double w[8][NE], iq[8];
-            double sn[8], cs[8], sd[8], cd[8], ra[8];
+#pragma unroll 1
+            for (int h = 0; h < 8; h += NA) {
+                double w[NA][NE], iq[NA];
+                double sn[NA], cs[NA], sd[NA], cd[NA], ra[NA];
 #pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                const int ax = (a & 4) ? i - L : i, ay = (a & 2) ? j - L : j, az = (a & 1) ? k - L : k;
-                const double p = P[ax < 0 ? -ax : ax] * P[ay < 0 ? -ay : ay] * P[az < 0 ? -az : az];
-                const int n2 = ax * ax + ay * ay + az * az;
-                ra[a] = sqrt((double)n2);
-                const double inv = n2 ? 1.0 / ra[a] : 0.0;
-                iq[a] = n2 ? inv * (0.5 / HERMES_PI) : __builtin_inf();
-                w[a][0] = p * (pi + pj + pk);
-                if constexpr (NE > 1) {
-                    const double mus[3] = {ax * inv, ay * inv, az * inv}, ps[3] = {pi, pj, pk};
+                for (int a = 0; a < NA; ++a) {
+                    const int ax = (a + h & 4) ? i - L : i, ay = (a + h & 2) ? j - L : j, az = (a + h & 1) ? k - L : k;
+                    const double p = P[ax < 0 ? -ax : ax] * P[ay < 0 ? -ay : ay] * P[az < 0 ? -az : az];
+                    const int n2 = ax * ax + ay * ay + az * az;
+                    const double rn = sqrt((double)n2), inv = n2 ? 1.0 / rn : 0.0;
+                    ra[a] = rn;
+                    iq[a] = n2 ? inv * (0.5 / HERMES_PI) : __builtin_inf();
+                    w[a][0] = p * (pi + pj + pk);
+                    if constexpr (NE > 1) {
+                        const double mus[3] = {ax * inv, ay * inv, az * inv}, ps[3] = {pi, pj, pk};
 #pragma unroll
-                    for (int e = 1; e < NE; ++e) w[a][e] = 0.0;
+                        for (int e = 1; e < NE; ++e) w[a][e] = 0.0;
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const double v = n2 ? p * ps[c] : 0.0;
-                        double pm = 1.0, pc = mus[c];
+                        for (int c = 0; c < 3; ++c) {
+                            const double v = n2 ? p * ps[c] : 0.0;
+                            double pm = 1.0, pc = mus[c];
 #pragma unroll
-                        for (int n = 1; n < LMAX; ++n) {
-                            const double pn = ((2.0 * n + 1.0) * mus[c] * pc - n * pm) * (1.0 / (n + 1.0));
-                            pm = pc;
-                            pc = pn;
-                            if (n % 2) w[a][(n + 1) / 2] += v * pn;
+                            for (int n = 1; n < LMAX; ++n) {
+                                const double pn = ((2.0 * n + 1.0) * mus[c] * pc - n * pm) * (1.0 / (n + 1.0));
+                                pm = pc;
+                                pc = pn;
+                                if (n % 2) w[a][(n + 1) / 2] += v * pn;
+                            }
                         }
                     }
+                    if constexpr (ROT) {
+                        const double t0 = rn * R0, td = rn * dR;
+                        sincospi(2.0 * (t0 - floor(t0)), &sn[a], &cs[a]);
+                        sincospi(2.0 * (td - floor(td)), &sd[a], &cd[a]);
+                    }
                 }
-                if constexpr (ROT) {
-                    const double t0 = ra[a] * R0, td = ra[a] * dR;
-                    sincospi(2.0 * (t0 - floor(t0)), &sn[a], &cs[a]);
-                    sincospi(2.0 * (td - floor(td)), &sd[a], &cd[a]);
-                }
-            }
-            for (int u0 = 0; u0 < nu; u0 += UC) {
-                double kb[NQ * 4];
+                // radii and channels of the next step are fetched a step ahead, and the channels' sums are read before the
+                // step's arithmetic: two waves per SIMD do not cover their latencies
+                double Rn[UC], iRn[UC];
+                int chn[NQ];
+                auto fetch = [&](int u0) {
 #pragma unroll
-                for (int v = 0; v < NQ * 4; ++v) kb[v] = 0.0;
+                    for (int q = 0; q < UC; ++q) {
+                        const int u = u0 + q < nu ? u0 + q : nu - 1;
+                        Rn[q] = radii[u];
+                        iRn[q] = radii[nu + u];
+                    }
 #pragma unroll
-                for (int q = 0; q < UC; ++q) {
-                    const int u = u0 + q;
-                    if (u < nu) {
-                        const double R = radii[u], iR = radii[nu + u];
+                    for (int g = 0; g < NQ; ++g) {
+                        const int n = 4 * g + quad_of_row(lane / 16), u = u0 + n / NE;
+                        chn[g] = (lane % 16 == 0 && n < UC * NE && u < nu) ? chan[u * (LMAX + 1) + 2 * (n % NE)] : -1;
+                    }
+                };
+                fetch(0);
+                for (int u0 = 0; u0 < nu; u0 += UC) {
+                    double kb[NQ * 4], Ru[UC], iRu[UC], sum[NQ];
+                    int ch[NQ];
 #pragma unroll
-                        for (int a = 0; a < 8; ++a) {
-                            double s = 0.0, c = 0.0;
-                            if constexpr (ROT) {
-                                s = sn[a];
-                                c = cs[a];
-                                sn[a] = fma(s, cd[a], c * sd[a]);  // for the next radius
-                                cs[a] = fma(c, cd[a], -(s * sd[a]));
-                            } else {
-                                const double t = ra[a] * R;
-                                sincospi(2.0 * (t - floor(t)), &s, &c);
-                            }
-                            double jv[LMAX + 1];
-                            const double ix = iq[a] * iR;
-                            if (R >= XMIN * iq[a]) {
-                                jv[0] = s * ix;
-                                if constexpr (LMAX >= 1) {
-                                    jv[1] = (jv[0] - c) * ix;
+                    for (int q = 0; q < UC; ++q) Ru[q] = Rn[q], iRu[q] = iRn[q];
 #pragma unroll
-                                    for (int n = 1; n < LMAX; ++n) jv[n + 1] = (2.0 * n + 1.0) * ix * jv[n] - jv[n - 1];
+                    for (int g = 0; g < NQ; ++g) {
+                        ch[g] = chn[g];
+                        sum[g] = ch[g] >= 0 ? wacc[wave * nch + ch[g]] : 0.0;
+                    }
+                    fetch(u0 + UC);
+#pragma unroll
+                    for (int v = 0; v < NQ * 4; ++v) kb[v] = 0.0;
+#pragma unroll
+                    for (int q = 0; q < UC; ++q) {
+                        const int u = u0 + q;
+                        if (u < nu) {
+                            const double R = Ru[q], iR = iRu[q];
+                            // One test for all of them (the first is the nearest to the origin): without a branch per
+                            // alias the eight serial chains of the recurrence overlap.
+                            auto add = [&](auto recurrence_only) {
+#pragma unroll
+                                for (int a = 0; a < NA; ++a) {
+                                    double s = 0.0, c = 0.0;
+                                    if constexpr (ROT) {
+                                        s = sn[a];
+                                        c = cs[a];
+                                        sn[a] = fma(s, cd[a], c * sd[a]);  // for the next radius
+                                        cs[a] = fma(c, cd[a], -(s * sd[a]));
+                                    } else {
+                                        const double t = ra[a] * R;
+                                        sincospi(2.0 * (t - floor(t)), &s, &c);
+                                    }
+                                    double jv[LMAX + 1];
+                                    const double ix = iq[a] * iR;
+                                    if (decltype(recurrence_only)::value || R >= XMIN * iq[a]) {
+                                        jv[0] = s * ix;
+                                        if constexpr (LMAX >= 1) {
+                                            jv[1] = (jv[0] - c) * ix;
+#pragma unroll
+                                            for (int n = 1; n < LMAX; ++n)
+                                                jv[n + 1] = (2.0 * n + 1.0) * ix * jv[n] - jv[n - 1];
+                                        }
+                                    } else {
+                                        radial_small<LMAX>(ROT ? 1.0 / ix : 2.0 * HERMES_PI * (ra[a] * R), ix, jv);
+                                    }
+#pragma unroll
+                                    for (int e = 0; e < NE; ++e) kb[q * NE + e] = fma(jv[2 * e], w[a][e], kb[q * NE + e]);
                                 }
-                            } else {
-                                radial_small<LMAX>(2.0 * HERMES_PI * (ra[a] * R), ix, jv);
-                            }
-#pragma unroll
-                            for (int e = 0; e < NE; ++e) kb[q * NE + e] = fma(jv[2 * e], w[a][e], kb[q * NE + e]);
+                            };
+                            if (__all(R >= XMIN * iq[0])) add(std::true_type());
+                            else add(std::false_type());
                         }
                     }
-                }
 #pragma unroll
-                for (int g = 0; g < NQ; ++g) {
-                    const double v = quad_sum(kb[4 * g], kb[4 * g + 1], kb[4 * g + 2], kb[4 * g + 3]);
-                    const int n = 4 * g + quad_of_row(lane / 16);
-                    const int u = u0 + n / NE;
-                    if (lane % 16 == 0 && n < UC * NE && u < nu) {
-                        const int ch = chan[u * (LMAX + 1) + 2 * (n % NE)];
-                        if (ch >= 0) wacc[wave * nch + ch] += v;
+                    for (int g = 0; g < NQ; ++g) {
+                        const double v = quad_sum(kb[4 * g], kb[4 * g + 1], kb[4 * g + 2], kb[4 * g + 3]);
+                        if (ch[g] >= 0) wacc[wave * nch + ch[g]] = sum[g] + v;
                     }
                 }
             }
