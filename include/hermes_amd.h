@@ -197,6 +197,10 @@ int hermes_window_build_full(hermes_ctx *ctx, int J, const double *P, const herm
  * convolution.py:284-295. */
 int hermes_spectrum_mul(hermes_ctx *ctx, int J, int half, int dbl, void *spec, const void *kernel,
                         int kernel_complex, double scale);
+/* out = real inverse transform of (transform of in) * kernel * scale, unnormalised, for a real kernel on the half
+ * spectrum (L, L, L/2+1).  spec: scratch of that many complex values; in is kept. */
+int hermes_convolve_real(hermes_ctx *ctx, int J, int dbl, const void *in_real, const void *kernel_half, double scale,
+                         void *spec, void *out_real);
 
 /* Fused multi-window pair product (Parseval form of pair_product_with_window,
  * corr2pcf.py:366-372): for every descriptor b,

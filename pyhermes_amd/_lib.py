@@ -67,6 +67,7 @@ _SIGNATURES.update({
     "hermes_window_build_rfft": [c_void_p, c_int, c_void_p, ctypes.POINTER(WindowDesc), c_int, c_void_p],
     "hermes_window_build_full": [c_void_p, c_int, c_void_p, ctypes.POINTER(WindowDesc), c_int, c_void_p],
     "hermes_spectrum_mul": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_double],
+    "hermes_convolve_real": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_double, c_void_p, c_void_p],
     "hermes_pair_reduce": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, ctypes.POINTER(WindowDesc), c_int,
                            _dpp],
     "hermes_window_build_full_profile": [c_void_p, c_int, c_void_p, ctypes.POINTER(RadialProfile), c_int, c_int,

@@ -98,7 +98,7 @@ int run_plan(hermes_ctx* ctx, int J, int kind, int dbl, int64_t batch, int dims,
     return 0;
 }
 
-// Strided lines of L = 2^LOG2L values, in place: element e of column c of block o is at o * outer + c + e * es, c < ncols
+// Strided lines of L = 2^LOG2L values, in place: element e of column c < ncols of block o is at o * outer + c + e * es
 // (y lines: a block is an x plane, its columns the z of a row; x lines: one block, its columns the positions of a
 // plane).  A workgroup stages TW columns in LDS, so every access is a run of TW values and each value is read and
 // written once; bound by HBM.  TW values are one 128-byte line (for half spectra the rows of y lines, L / 2 + 1 values
@@ -106,9 +106,14 @@ int run_plan(hermes_ctx* ctx, int J, int kind, int dbl, int64_t batch, int dims,
 // the streaming hint the shared lines and what the previous pass left in the last-level cache are lost (512^3 FP32,
 // y lines: 218 us plain, 446 streaming; 256^3 FP64, x lines: 40 and 80).  The library's strided kernels took 598 us
 // (512^3 FP32, half spectrum: 1.8 TB/s; now y 218, x 272) and 86 us (256^3 FP64: 3.1 TB/s; now 39 and 40).
-template <class C, int LOG2L, int TW, int NT, int DIR>
+// CONV (x lines of a convolution with a real kernel of the same layout, DIR = -1): the line is transformed, multiplied
+// by kernel * scale and transformed back while it is in LDS, which leaves out one pass over the spectrum and the
+// product's own (256^3 FP64: 40 + 51 + 40 us as three passes).
+template <class C, int LOG2L, int TW, int NT, int DIR, bool CONV = false>
 __global__ __launch_bounds__(NT) void k_fft_lines(C* data, const C* __restrict__ twg, int64_t es, int64_t outer,
-                                                  int64_t ncols, int ntile) {
+                                                  int64_t ncols, int ntile,
+                                                  const decltype(C::x)* __restrict__ kernel = nullptr,
+                                                  decltype(C::x) scale = 0) {
     constexpr int L = 1 << LOG2L;
     static_assert(NT % TW == 0 && TW * L % NT == 0, "a thread keeps one column of the tile");
     using F = hermes_fft::LdsFft<LOG2L, TW, NT, DIR, true, C>;
@@ -121,38 +126,96 @@ __global__ __launch_bounds__(NT) void k_fft_lines(C* data, const C* __restrict__
     const int64_t b = xcd * (nb / 8) + (xcd < rem ? xcd : rem) + blockIdx.x / 8;
     const int64_t col = (b % ntile) * TW + tid % TW;
     const bool inside = col < ncols;  // the last tile of a block may be partly empty
-    C* p = data + (b / ntile) * outer + (inside ? col : 0) + (int64_t)(tid / TW) * es;
+    const int64_t first = (b / ntile) * outer + (inside ? col : 0) + (int64_t)(tid / TW) * es;
+    C* p = data + first;
     const int64_t step = (int64_t)(NT / TW) * es;
     hermes_fft::load_twiddles<LOG2L>(tw, twg, tid, NT);
     constexpr int PER = TW * L / NT;
     C v[PER];  // the whole tile is in flight before the first store to LDS
 #pragma unroll
     for (int k = 0; k < PER; ++k) v[k] = p[k * step];
+    decltype(C::x) w[CONV ? PER : 1];
+    if constexpr (CONV) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) w[k] = kernel[first + k * step];
+    }
 #pragma unroll
     for (int k = 0; k < PER; ++k) lds[tid + k * NT] = v[k];
     __syncthreads();
     F::run(lds, tw, tid);
+    if constexpr (CONV) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const decltype(C::x) c = w[k] * scale;
+            C& z = lds[tid + k * NT];
+            z.x *= c;
+            z.y *= c;
+        }
+        for (int k = tid; k < L; k += NT) tw[k].y = -tw[k].y;
+        __syncthreads();
+        hermes_fft::LdsFft<LOG2L, TW, NT, -DIR, true, C>::run(lds, tw, tid);
+    }
     if (!inside) return;
 #pragma unroll
     for (int k = 0; k < PER; ++k) p[k * step] = lds[tid + k * NT];
 }
 
+// Tile of the strided passes: 128 bytes wide; 128^3 takes 16 values in FP64 as well (21 us for 24 with 8).
+template <class C, int LOG2L>
+struct LineTile {
+    static constexpr int L = 1 << LOG2L;
+    static constexpr int TW = LOG2L == 7 ? 16 : 128 / (int)sizeof(C);
+    static constexpr int NT = TW * L > 4096 ? 512 : 256;
+    static constexpr size_t lds = sizeof(C) * (size_t)(L + TW * L);
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+};
+
 // y and x lines of `batch` grids of (L, L, M) values, in place.
 template <class C, int LOG2L, int DIR>
 int run_lines(hermes_ctx* ctx, int64_t batch, int64_t M, C* data, const C* twg) {
-    constexpr int L = 1 << LOG2L;
-    constexpr int TW = LOG2L == 7 ? 16 : 128 / (int)sizeof(C);  // 128^3: 16 in FP64 as well (21 us for 24 with 8)
-    constexpr int NT = TW * L > 4096 ? 512 : 256;
-    constexpr size_t lds = sizeof(C) * (size_t)(L + TW * L);
-    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    using Tile = LineTile<C, LOG2L>;
+    constexpr int L = Tile::L, TW = Tile::TW, NT = Tile::NT;
     auto k = k_fft_lines<C, LOG2L, TW, NT, DIR>;
-    HERMES_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HERMES_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile::lds));
     const int64_t yt = (M + TW - 1) / TW, xt = (L * M + TW - 1) / TW;
-    k<<<(unsigned)(batch * L * yt), NT, lds, ctx->stream>>>(data, twg, M, L * M, M, (int)yt);
+    k<<<(unsigned)(batch * L * yt), NT, Tile::lds, ctx->stream>>>(data, twg, M, L * M, M, (int)yt, nullptr, 0);
     HERMES_LAUNCH_CHECK();
-    k<<<(unsigned)(batch * xt), NT, lds, ctx->stream>>>(data, twg, L * M, L * L * M, L * M, (int)xt);
+    k<<<(unsigned)(batch * xt), NT, Tile::lds, ctx->stream>>>(data, twg, L * M, L * L * M, L * M, (int)xt, nullptr, 0);
     HERMES_LAUNCH_CHECK();
     return 0;
+}
+
+// y lines forward, x lines forward times kernel * scale and back, y lines back, of one half spectrum, in place.
+template <class C, int LOG2L>
+int run_conv(hermes_ctx* ctx, C* data, const C* fwd, const C* inv, const decltype(C::x)* kernel, double scale) {
+    using Tile = LineTile<C, LOG2L>;
+    constexpr int L = Tile::L, TW = Tile::TW, NT = Tile::NT;
+    constexpr int64_t M = L / 2 + 1, yt = (M + TW - 1) / TW, xt = (L * M + TW - 1) / TW;
+    auto kf = k_fft_lines<C, LOG2L, TW, NT, -1>;
+    auto kb = k_fft_lines<C, LOG2L, TW, NT, 1>;
+    auto kx = k_fft_lines<C, LOG2L, TW, NT, -1, true>;
+    for (const void* k : {(const void*)kf, (const void*)kb, (const void*)kx})
+        HERMES_CHECK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile::lds));
+    kf<<<(unsigned)(L * yt), NT, Tile::lds, ctx->stream>>>(data, fwd, M, L * M, M, (int)yt, nullptr, 0);
+    HERMES_LAUNCH_CHECK();
+    kx<<<(unsigned)xt, NT, Tile::lds, ctx->stream>>>(data, fwd, L * M, L * L * M, L * M, (int)xt, kernel,
+                                                    (decltype(C::x))scale);
+    HERMES_LAUNCH_CHECK();
+    kb<<<(unsigned)(L * yt), NT, Tile::lds, ctx->stream>>>(data, inv, M, L * M, M, (int)yt, nullptr, 0);
+    HERMES_LAUNCH_CHECK();
+    return 0;
+}
+
+template <class C>
+int conv_lines(hermes_ctx* ctx, int J, C* data, const C* fwd, const C* inv, const void* kernel, double scale) {
+    HERMES_REQUIRE(fwd && inv, "%s", hermes_last_error());
+    auto w = (const decltype(C::x)*)kernel;
+    switch (J) {
+        case 7: return run_conv<C, 7>(ctx, data, fwd, inv, w, scale);
+        case 8: return run_conv<C, 8>(ctx, data, fwd, inv, w, scale);
+        case 9: return run_conv<C, 9>(ctx, data, fwd, inv, w, scale);
+        default: return run_conv<C, 10>(ctx, data, fwd, inv, w, scale);
+    }
 }
 
 template <class C, int DIR>
@@ -206,6 +269,25 @@ int hermes_fft_c2r(hermes_ctx* ctx, int J, int batch, int dbl, void* in_half, vo
 
 int hermes_fft_c2c(hermes_ctx* ctx, int J, int batch, int dbl, int inverse, const void* in, void* out) {
     return run(ctx, J, inverse ? 3 : 2, dbl, batch, in, out);
+}
+
+int hermes_convolve_real(hermes_ctx* ctx, int J, int dbl, const void* in_real, const void* kernel_half, double scale,
+                         void* spec, void* out_real) {
+    HERMES_REQUIRE(ctx && in_real && kernel_half && spec && out_real, "hermes_convolve_real: null argument");
+    HERMES_REQUIRE(J >= 1 && J <= 10, "hermes_convolve_real: J=%d unsupported", J);
+    if (J < LINES_MIN_J) {
+        int rc = run(ctx, J, 0, dbl, 1, in_real, spec);
+        if (rc == 0) rc = hermes_spectrum_mul(ctx, J, 1, dbl, spec, kernel_half, 0, scale);
+        return rc ? rc : run(ctx, J, 1, dbl, 1, spec, out_real);
+    }
+    HERMES_CHECK_HIP(hipSetDevice(ctx->device));
+    const int64_t nlines = (int64_t)1 << (2 * J);
+    if (int rc = run_plan(ctx, J, 0, dbl, nlines, 1, in_real, spec)) return rc;
+    const int rc = dbl ? conv_lines(ctx, J, (double2*)spec, hermes_twiddles_f64(ctx, J, -1),
+                                    hermes_twiddles_f64(ctx, J, 1), kernel_half, scale)
+                       : conv_lines(ctx, J, (float2*)spec, hermes_twiddles(ctx, J, -1), hermes_twiddles(ctx, J, 1),
+                                    kernel_half, scale);
+    return rc ? rc : run_plan(ctx, J, 1, dbl, nlines, 1, spec, out_real);
 }
 
 }  // extern "C"

@@ -141,9 +141,7 @@ class SFCField(HermesData):
         nx, ny, nz = eps.shape
         N = nx * ny * nz
         if tuple(K.shape) == (nx, ny, nz // 2 + 1) and not K.is_complex() and not eps.is_complex():
-            spec = kernels.rfftn(eps)
-            kernels.spectrum_mul(spec, K.to(torch.float64 if dbl else torch.float32), 1.0 / N)
-            conv = kernels.irfftn_unnormalized(spec, nx)
+            conv = kernels.convolve_real(eps, K.to(torch.float64 if dbl else torch.float32), 1.0 / N)
         elif tuple(K.shape) == (nx, ny, nz):
             cdt = torch.complex128 if dbl else torch.complex64
             ec = eps.to(cdt) if eps.is_complex() else torch.complex(eps, torch.zeros_like(eps)).to(cdt)

@@ -233,6 +233,22 @@ def spectrum_mul(spec, kernel, scale=1.0):
     return spec
 
 
+def convolve_real(x, kernel, scale=1.0):
+    """irfftn(rfftn(x) * kernel * scale), unnormalised: (L, L, L) real x, (L, L, L//2+1) real kernel of its dtype."""
+    L = x.shape[0]
+    if tuple(x.shape) != (L, L, L) or tuple(kernel.shape) != (L, L, L // 2 + 1):
+        raise ValueError(f"convolve_real: shapes {tuple(x.shape)} and {tuple(kernel.shape)}")
+    if x.dtype not in (torch.float32, torch.float64) or kernel.dtype != x.dtype:
+        raise ValueError(f"convolve_real: dtypes {x.dtype} and {kernel.dtype}")
+    dbl = x.dtype == torch.float64
+    x, kernel = x.contiguous(), kernel.contiguous()
+    spec = torch.empty(kernel.shape, dtype=torch.complex128 if dbl else torch.complex64, device=x.device)
+    out = torch.empty_like(x)
+    _lib.call("hermes_convolve_real", _lib.context(), _J_of(L), 1 if dbl else 0, ptr(x), ptr(kernel), float(scale),
+              ptr(spec), ptr(out))
+    return out
+
+
 PAIR_WINDOWS_PER_PASS = 2048  # one fused pass keeps a sum per window and wave in 64 KB of LDS
 
 

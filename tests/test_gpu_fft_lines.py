@@ -51,3 +51,20 @@ def test_full_spectrum(J, batch, inverse, dtype):
     _check(kernels.fftn_c2c(x, inverse=inverse), want, J, real)
     assert torch.equal(x, keep)
     _check(kernels.fftn_c2c(x, inverse=inverse, out=x), want, J, real)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("J", [6, 7, 8, 9])
+def test_convolution(J, dtype):
+    """Two transforms and products of O(1): the bound of a transform of twice the levels."""
+    L = 1 << J
+    x = _field((L, L, L), dtype)
+    f = _field((L // 2 + 1,), dtype, 4)  # a product symmetric under k -> -k, as windows are
+    full = torch.cat([f, f[1:-1].flip(0)])
+    k = full[:, None, None] * full[None, :, None] * f
+    keep = x.clone()
+    got = kernels.convolve_real(x, k, 1.0 / L ** 3)
+    spec = torch.fft.rfftn(x.double())
+    spec *= k.double()
+    _check(got, torch.fft.irfftn(spec, s=(L, L, L)), 2 * J, dtype)
+    assert torch.equal(x, keep)
