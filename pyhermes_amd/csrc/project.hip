@@ -645,7 +645,7 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
     int* slots = nullptr;
     if (n > 0 && worst <= RESERVE_BYTES) {
         slots = (int*)hermes_workspace(ctx, WS_PROJ_SLOT, sizeof(int) * 8 * (size_t)n);
-        HERMES_REQUIRE(slots, "%s%s", hermes_last_error(), ctx->capturing ? " (hermes_project_reserve sizes it)" : "");
+        if (!slots) (void)hipGetLastError();  // no room, or a capture that did not reserve it: the fill counts again
     }
     if (slots && ntiles <= LDS_TILES) {
         // more particles per workgroup aggregate better, once there are workgroups enough to fill the chip
