@@ -357,7 +357,8 @@ int hermes_interpolate(hermes_ctx *ctx, int J, const double *grid, const double 
 
 /* Box-random-centre triplet estimator for one (R1, R2, mu) (grid units):
  * sum_rot sum_i n1[i] n2(c_i + o2) n3(c_i + o3) / (n_rot n), with the per-rotation
- * uniforms (a, b, c) given on the host (n_rot x 3).  Replaces
+ * uniforms (a, b, c) given on the host (n_rot x 3).  phi: 3 phi_res samples; 1024 to a
+ * cell is the resolution of the fast kernels, any other is taken too.  Replaces
  * estimate_triplet_product_box_random_centers, corr3pcf_kernels.py:100-140. */
 int hermes_mc_triplet_box(hermes_ctx *ctx, int J, double R1, double R2, double mu, const double *spos,
                           const double *n1, int64_t n, int n_rot, const double *abc_host, const double *g2,

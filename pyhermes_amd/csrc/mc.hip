@@ -244,8 +244,9 @@ __global__ void k_triplet_offsets(double R1, double R2, double mu, const double*
 }
 
 // blockIdx.y: rotation (strided); blockIdx.x: centres (strided); per-block partial sums.  Bound by random lines of
-// the grids and the latency of their loads.
-template <int LAYOUT>
+// the grids and the latency of their loads.  SPHI: the scaling function in LDS, for its usual 1024 samples to a cell;
+// tables of another resolution are read where they are (plain layout only).
+template <int LAYOUT, bool SPHI = true>
 __global__ __launch_bounds__(MC_THREADS, 4) void k_triplet_box(const double* __restrict__ spos,
                                                                const double* __restrict__ n1, int64_t n, int n_rot,
                                                                const double* __restrict__ off,
@@ -253,10 +254,17 @@ __global__ __launch_bounds__(MC_THREADS, 4) void k_triplet_box(const double* __r
                                                                const double* __restrict__ g3,
                                                                const double* __restrict__ phi, int lg, int res,
                                                                double* __restrict__ partial) {
-    __shared__ double sphi[3 * 1024];
+    static_assert(SPHI || LAYOUT == GRID_PLAIN, "a table in global memory goes with the plain layout");
+    __shared__ double sphi[SPHI ? 3 * 1024 : 1];
     __shared__ double sh[MC_THREADS / 64];
-    load_phi(sphi, phi, threadIdx.x, MC_THREADS);
-    __syncthreads();
+    if constexpr (SPHI) {
+        load_phi(sphi, phi, threadIdx.x, MC_THREADS);
+        __syncthreads();
+    }
+    auto value = [&](const double* g, double x, double y, double z) {
+        if constexpr (SPHI) return interp<LAYOUT>(g, sphi, lg, res, x, y, z);
+        else return interp_at<GRID_PLAIN, false>(g, phi, lg, res, x, y, z);
+    };
     double s = 0.0;
     for (int r = blockIdx.y; r < n_rot; r += gridDim.y) {
         const double* o = off + 6 * r;
@@ -265,8 +273,8 @@ __global__ __launch_bounds__(MC_THREADS, 4) void k_triplet_box(const double* __r
              q += (int64_t)gridDim.x * MC_THREADS) {
             const int64_t mine = q + (threadIdx.x & 63), p = mine < n ? mine : n - 1;
             const double x = spos[3 * p], y = spos[3 * p + 1], z = spos[3 * p + 2];
-            const double v2 = interp<LAYOUT>(g2, sphi, lg, res, x + o[0], y + o[1], z + o[2]);
-            const double v3 = interp<LAYOUT>(g3, sphi, lg, res, x + o[3], y + o[4], z + o[5]);
+            const double v2 = value(g2, x + o[0], y + o[1], z + o[2]);
+            const double v3 = value(g3, x + o[3], y + o[4], z + o[5]);
             if (mine < n) s += n1[p] * v2 * v3;
         }
     }
@@ -719,6 +727,7 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     HERMES_REQUIRE(ctx && spos && n1 && abc_host && g2 && g3 && phi && out_host, "hermes_mc_triplet_box: null arg");
     HERMES_REQUIRE(J >= 2 && J <= 10, "J=%d unsupported", J);
     HERMES_REQUIRE(n > 0 && n_rot > 0, "need centres and rotations");
+    HERMES_REQUIRE(phi_res >= 1, "phi_res must be positive");
     HERMES_CHECK_HIP(hipSetDevice(ctx->device));
     // about 2048 workgroups: the centres by the rotations
     const int nbx = (int)hermes_blocks(n, MC_THREADS, 2048);
@@ -731,13 +740,15 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     k_triplet_offsets<<<hermes_blocks(n_rot, 64), 64, 0, ctx->stream>>>(R1, R2, mu, d_abc, n_rot, d_off);
     HERMES_LAUNCH_CHECK();
     const double* g[2] = {g2, g3};
-    const int layout = grid_layout(ctx, J, 2.0 * (double)n * n_rot, g, 2);
+    // the LDS table and the packed fractions of the faster layouts hold 1024 samples to a cell
+    const int layout = phi_res == 1024 ? grid_layout(ctx, J, 2.0 * (double)n * n_rot, g, 2) : -1;
     auto go = [&](auto kernel) {
         kernel<<<dim3(nbx, nby), MC_THREADS, 0, ctx->stream>>>(spos, n1, n, n_rot, d_off, g[0], g[1], phi, J, phi_res, ws);
     };
     if (layout == GRID_BRICK) go(k_triplet_box<GRID_BRICK>);
     else if (layout == GRID_ALIGNED) go(k_triplet_box<GRID_ALIGNED>);
-    else go(k_triplet_box<GRID_PLAIN>);
+    else if (layout == GRID_PLAIN) go(k_triplet_box<GRID_PLAIN>);
+    else go(k_triplet_box<GRID_PLAIN, false>);
     HERMES_LAUNCH_CHECK();
     HERMES_CHECK_HIP(hermes_reduce::sum_columns(ctx->stream, ws, 1, nb, 1, nullptr, ws + nb));
     double s = 0.0;

@@ -87,3 +87,34 @@ def test_bricks_keep_non_finite_cells_apart(phi):
     got = kernels.mc_triplet_box(*args, dev(clean), dev(n1), abc, dev(bad), dev(bad), phi)
     assert np.isfinite(got) and got == want
     assert not np.isfinite(kernels.mc_triplet_box(*args, dev(spos), dev(n1 * 0 + 1), abc, dev(bad), dev(bad), phi))
+
+
+@pytest.mark.parametrize("level,offset", [(9, 0), (9, 1), (11, 0), (4, 0)])
+def test_triplet_with_another_table_resolution(level, offset):
+    """2^level samples of the scaling function to a cell instead of 1024, through the C entry: the table is read
+    with the caller's resolution (a grid and point count that take the bricks at 1024)."""
+    import ctypes
+    from oracle.scaling import sample_scaling_function
+    from pyhermes_amd import _lib, kernels
+    import torch
+    L, n, n_rot, res = 128, 40_003, 9, 1 << level
+    phi = sample_scaling_function("db2", level)
+    assert phi.size == 3 * res
+    g2, g3 = _grid(L, 4), _grid(L, 5)
+    rng = np.random.default_rng(level)
+    spos = rng.uniform(-2.0 * L, 3.0 * L, size=(n, 3))
+    n1, abc = rng.normal(size=n), rng.random((n_rot, 3))
+    dev = [kernels.as_device(a, torch.float64) for a in (spos, n1, phi)]
+    gd = [_device(g2, offset), _device(g3, offset)]
+    got = np.zeros(1)
+    dp = ctypes.POINTER(ctypes.c_double)
+    print(f"triplet with {res} samples to a cell, offset={offset}", flush=True)
+    _lib.call("hermes_mc_triplet_box", _lib.context(), 7, 0.2 * L, 0.35 * L, -0.3, dev[0].data_ptr(), dev[1].data_ptr(),
+              n, n_rot, abc.ctypes.data_as(dp), gd[0].data_ptr(), gd[1].data_ptr(), dev[2].data_ptr(), res,
+              got.ctypes.data_as(dp))
+    ref, mag = 0.0, 0.0
+    for a, b, c in abc:
+        o = omc.triangle_offsets(0.2 * L, 0.35 * L, -0.3, 2 * np.pi * a, 2 * b - 1, 2 * np.pi * c)
+        t = n1 * omc.interpolate(g2, spos, phi, o[:3], res) * omc.interpolate(g3, spos, phi, o[3:], res)
+        ref, mag = ref + t.sum(), mag + np.abs(t).sum()
+    assert abs(got[0] - ref / (n * n_rot)) <= 1e-12 * mag / (n * n_rot)
