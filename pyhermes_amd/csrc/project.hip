@@ -108,7 +108,9 @@ __device__ __forceinline__ int replica_tile(const TileGeom& g, const int X[2], c
 }
 
 // err: a word set on invalid positions (device memory, or pinned host memory that the host reads after the wait).
-// slots (may be NULL): slots[k n + p] = slot of particle p in the tile of its replica k.
+// SLOTS: slots[k n + p] = slot of particle p in the tile of its replica k; otherwise (catalogues too large to keep
+// them) the atomics return nothing and no wave waits for them.
+template <bool SLOTS>
 __global__ void k_proj_count(const double* __restrict__ pos, int64_t n, double sf, int res, TileGeom g,
                              int* __restrict__ tile_count, int32_t* __restrict__ cell_out,
                              int32_t* __restrict__ frac_out, int* err, int* __restrict__ slots) {
@@ -131,7 +133,7 @@ __global__ void k_proj_count(const double* __restrict__ pos, int64_t n, double s
         for (int k = 0; k < 8; ++k) {
             const int t = act ? replica_tile(g, X, Y, Z, nx, ny, nz, k) : -1;
             const int slot = wave_add(tile_count, t < 0 ? 0 : t, t >= 0);
-            if (slots && t >= 0) slots[(int64_t)k * n + p] = slot;
+            if (SLOTS && t >= 0) slots[(int64_t)k * n + p] = slot;
         }
     }
 }
@@ -657,8 +659,9 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
             k_proj_count_lds<1><<<(unsigned)((n + 255) / 256), 256, lds, st>>>(pos, n, sf, phi_res, g, ntiles, count,
                                                                               cell_out, frac_out, errp, slots);
     } else {
-        k_proj_count<<<hermes_blocks(n, 256, 4096), 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out,
-                                                                  errp, slots);
+        const unsigned nb = hermes_blocks(n, 256, 4096);
+        if (slots) k_proj_count<true><<<nb, 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out, errp, slots);
+        else k_proj_count<false><<<nb, 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out, errp, nullptr);
     }
     HERMES_LAUNCH_CHECK();
     if (nscan > 1) {
