@@ -50,6 +50,7 @@ void* hermes_workspace(hermes_ctx* ctx, int slot, size_t bytes) {
     size_t grow = bytes + bytes / 4;
     void* p = nullptr;
     if (hipMalloc(&p, grow) != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next call's launch checks
         hermes_set_error("hipMalloc of %zu bytes for workspace slot %d failed", grow, slot);
         return nullptr;
     }

@@ -696,10 +696,7 @@ static int grid_layout(hermes_ctx* ctx, int J, double points, const double** g, 
     }
     if (J < 7 || points * 8.0 < (double)n * copies || copies * n * sizeof(double) > ((size_t)4 << 30)) return plain;
     double* ws = (double*)hermes_workspace(ctx, WS_SPEC, copies * n * sizeof(double));
-    if (!ws) {
-        (void)hipGetLastError();
-        return plain;
-    }
+    if (!ws) return plain;
     for (int k = 0; k < copies; ++k)
         k_brick<<<hermes_blocks((int64_t)n, 256, 16384), 256, 0, ctx->stream>>>(distinct[k], J, ws + k * n);
     for (int i = 0; i < n_grid; ++i) g[i] = ws + of[i] * n;

@@ -592,6 +592,15 @@ struct TileWs {
     }
 };
 
+// Waits for the stream when a call that has work in flight returns early: that work may still store to the context's
+// host word, which the next call clears from the host.
+struct DrainOnReturn {
+    hermes_ctx* ctx;
+    ~DrainOnReturn() {
+        if (ctx) (void)hipStreamSynchronize(ctx->stream);
+    }
+};
+
 int ilog2(int v) {
     int r = 0;
     while ((1 << r) < v) ++r;
@@ -638,10 +647,12 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
     // Invalid positions are projected at the origin (in bounds) and flagged: under stream capture in the
     // context's sticky error word, eagerly in a pinned host word read before the call returns (and fails).
     int* errp = ctx->dev_err;
+    DrainOnReturn drain{nullptr};
     if (!ctx->capturing) {
         errp = hermes_host_word(ctx);
         HERMES_REQUIRE(errp, "%s", hermes_last_error());
         *(volatile int*)errp = 0;
+        drain.ctx = ctx;
     }
     HERMES_REQUIRE(errp, "hermes_project: no device error word");
 
@@ -653,7 +664,7 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
     int* slots = nullptr;
     if (n > 0 && worst <= RESERVE_BYTES) {
         slots = (int*)hermes_workspace(ctx, WS_PROJ_SLOT, sizeof(int) * 8 * (size_t)n);
-        if (!slots) (void)hipGetLastError();  // no room, or a capture that did not reserve it: the fill counts again
+        // without room, or in a capture that did not reserve it, the fill counts again
     }
     if (slots && ntiles <= LDS_TILES) {
         // more particles per workgroup aggregate better, once there are workgroups enough to fill the chip
@@ -714,6 +725,7 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
     }
     HERMES_LAUNCH_CHECK();
     if (!ctx->capturing) {  // invalid positions were projected at the origin (in bounds)
+        drain.ctx = nullptr;
         if (hermes_poll_stream(ctx)) return 1;
         HERMES_REQUIRE(*(volatile int*)errp == 0, "hermes_project: non-finite or out-of-range particle positions");
     }

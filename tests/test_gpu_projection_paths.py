@@ -132,3 +132,30 @@ def test_capture_without_room_for_slots(phi, J, n):
         kernels.graph_destroy(graph)
         want = kernels.project(pos, w, J, BOX, phi, want64=True)["eps64"]
     assert all(torch.equal(g, want) for g in got)
+
+
+def test_refused_workspace_leaves_no_error_behind(phi):
+    """A call whose records cannot be had fails with work in flight that meets an invalid position; the next call must
+    be refused neither for the allocation's error nor for that position."""
+    import torch
+    from pyhermes_amd import kernels
+    J, n = 5, 1 << 24
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    pos = torch.rand((n, 3), generator=gen, device="cuda", dtype=torch.float64) * BOX
+    pos[n // 2, 1] = float("inf")
+    w = torch.ones(n, dtype=torch.float64, device="cuda")
+    good, gw = pos[:4096].clone(), w[:4096].clone()
+    want = kernels.project(good, gw, J, BOX, phi, want64=True)["eps64"]
+    kernels.release_workspaces()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    print(f"projection with its records refused: {free / 2**30:.0f} GiB free", flush=True)
+    fill = torch.empty(max(free - (3 << 29), 1 << 20), dtype=torch.uint8, device="cuda")  # leaves 1.5 GiB; records: 2.5
+    torch.cuda._sleep(30_000_000)
+    with pytest.raises(RuntimeError, match="hermes_project failed"):
+        kernels.project(pos, w, J, BOX, phi)
+    got = kernels.project(good, gw, J, BOX, phi, want64=True)["eps64"]
+    del fill
+    kernels.release_workspaces()
+    torch.cuda.empty_cache()
+    assert torch.equal(got, want)
