@@ -203,6 +203,10 @@ __device__ inline double win_sphere_f64(double k, double R) {
     return 3 * (s - q * c) / (q2 * q);
 }
 
+// The same as a call, for kernels that take any window: inlined, the three Bessel ranges double their registers (the
+// general pair reduction: 290 and one wave per SIMD; 150 and three with the call).
+__device__ __attribute__((noinline)) double los_perp_call(bool ring, double t) { return los_perp_f64(ring, t); }
+
 // Line-of-sight windows (window_functions.py:164-319).  Along a coordinate axis they are even in every
 // component of k, so the octant folds apply to them as to the isotropic ones; along any other direction
 // they are only even under k -> -k (the half-spectrum sums still apply, the octant sharing does not).
@@ -219,7 +223,7 @@ __device__ inline double los_window_f64(int type, double ki, double kj, double k
         kperp2 = u * u + v * v;
     }
     const double qpar = 2.0 * HERMES_PI * kpar * H;
-    const double perp = los_perp_f64(type == HERMES_WIN_RING || type == HERMES_WIN_CYLSHELL, sqrt(kperp2) * R);
+    const double perp = los_perp_call(type == HERMES_WIN_RING || type == HERMES_WIN_CYLSHELL, sqrt(kperp2) * R);
     const double par = (type == HERMES_WIN_RING || type == HERMES_WIN_DISK)
                            ? cos(qpar)
                            : (qpar == 0.0 ? 1.0 : sin(qpar) / qpar);
@@ -300,6 +304,7 @@ __device__ inline double radial_profile_f64(const hermes_radial_profile& p, int 
 
 // Transfer function of a real window at signed k: the isotropic and line-of-sight ones and the m = 0 multipoles.
 // general = false compiles out the non-axis line-of-sight branch (for callers that never see axis-3 descriptors).
+template <bool LOS = true>
 __device__ inline double real_window_f64(const hermes_window_desc& d, double ki, double kj, double kk,
                                          bool general = true) {
     if (d.type == HERMES_WIN_SHELL_MULTIPOLE) {
@@ -307,7 +312,7 @@ __device__ inline double real_window_f64(const hermes_window_desc& d, double ki,
         if (k == 0.0) return d.l == 0 ? sqrt(0.25 / HERMES_PI) : 0.0;
         return jl_f64(d.l, k * d.a0) * yl0_f64(d.l, kk / k);
     }
-    return iso_window_f64(d.type, ki, kj, kk, d.a0, d.a1, d.axis, general ? d.los : nullptr);
+    return iso_window_f64<LOS>(d.type, ki, kj, kk, d.a0, d.a1, d.axis, general ? d.los : nullptr);
 }
 
 // ------------------------------------------------------------------ FP32 fast path

@@ -179,6 +179,7 @@ __global__ void k_spec_mul(int64_t n, T* __restrict__ spec, const T* __restrict_
 // ---------------------------------------------------------------- pair reduction
 // Window value at signed lattice alias (ax, ay, az), FP32 fast path for shells and
 // shell multipoles; other window types use the FP64 formula.
+template <bool LOS>
 __device__ __forceinline__ float window_value_f32(const hermes_window_desc& d, int ax, int ay, int az, int L,
                                                   float cnorm) {
     double n2 = (double)ax * ax + (double)ay * ay + (double)az * az;
@@ -194,14 +195,17 @@ __device__ __forceinline__ float window_value_f32(const hermes_window_desc& d, i
     }
     double inv_L = 1.0 / L;
     // reached only by passes without non-axis line-of-sight windows
-    return (float)iso_window_f64(d.type, ax * inv_L, ay * inv_L, az * inv_L, d.a0, d.a1, d.axis, nullptr);
+    return (float)iso_window_f64<LOS>(d.type, ax * inv_L, ay * inv_L, az * inv_L, d.a0, d.a1, d.axis, nullptr);
 }
 
 // One thread per octant representative (x, y, z) in [0, L/2]^3; its kernel value is
 // shared by the (up to) 4 modes (x|L-x, y|L-y, z) of the half spectrum.  GEN: the pass holds a
 // line-of-sight window along a non-axis direction (descriptor axis 3), whose value differs between the 4
-// modes; it is a separate instantiation so the other passes keep their register budget.
-template <typename C, bool FP64, bool GEN>
+// modes.  LOS: it holds a line-of-sight window at all.  Both are separate instantiations, so that the other passes
+// keep their register budget (124 registers and four waves per SIMD without, 150 to 162 and three with them; FP32
+// spectra, 20 shells and a sphere at L = 512: 7.1 ms, 16.4 with the Bessel series inlined and 290 registers; 20 shells
+// and a disk: 8.5, 17.3).
+template <typename C, bool FP64, bool GEN, bool LOS>
 __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __restrict__ F1,
                                                              const C* __restrict__ F2, const double* __restrict__ P,
                                                              const hermes_window_desc* __restrict__ descs,
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __r
                             int ax = (a & 4) ? x - L : x, ay = (a & 2) ? y - L : y, az = (a & 1) ? z - L : z;
                             int ix = ax < 0 ? -ax : ax, iy = ay < 0 ? -ay : ay, iz = az < 0 ? -az : az;
                             double p = P[ix] * P[iy] * P[iz];
-                            const double w = real_window_f64(d, sx * ax * inv_L, sy * ay * inv_L, az * inv_L);
+                            const double w = real_window_f64<LOS>(d, sx * ax * inv_L, sy * ay * inv_L, az * inv_L);
                             km += FP64 ? p * w : (double)((float)p * (float)w);
                         }
                         kb += pm * km;
@@ -270,9 +274,9 @@ __global__ __launch_bounds__(RED_THREADS) void k_pair_reduce(int L, const C* __r
                         double p = P[ix] * P[iy] * P[iz];
                         if (FP64) {
                             double inv_L = 1.0 / L;
-                            kb += p * real_window_f64(d, ax * inv_L, ay * inv_L, az * inv_L, GEN);
+                            kb += p * real_window_f64<LOS>(d, ax * inv_L, ay * inv_L, az * inv_L, GEN);
                         } else {
-                            kb += (double)((float)p * window_value_f32(d, ax, ay, az, L, cnorms[b]));
+                            kb += (double)((float)p * window_value_f32<LOS>(d, ax, ay, az, L, cnorms[b]));
                         }
                     }
                     kb *= power;
@@ -1198,20 +1202,25 @@ static int pair_reduce_impl(hermes_ctx* ctx, int J, int dbl, const void* F1, con
     HERMES_CHECK_HIP(hipMemcpyAsync(d_desc, descs, sizeof(hermes_window_desc) * n_desc, hipMemcpyHostToDevice, ctx->stream));
     HERMES_CHECK_HIP(hipMemcpyAsync(d_cn, cn.data(), sizeof(float) * n_desc, hipMemcpyHostToDevice, ctx->stream));
     size_t shmem = sizeof(double) * (RED_THREADS / 64) * n_desc;
-    bool gen = false;
-    for (int b = 0; b < n_desc; ++b) gen = gen || (descs[b].type >= HERMES_WIN_RING && descs[b].axis == 3);
-    if (dbl && gen)
-        k_pair_reduce<double2, true, true><<<nblocks, RED_THREADS, shmem, ctx->stream>>>(
-            L, (const double2*)F1, (const double2*)F2, P, d_desc, d_cn, n_desc, partial);
-    else if (dbl)
-        k_pair_reduce<double2, true, false><<<nblocks, RED_THREADS, shmem, ctx->stream>>>(
-            L, (const double2*)F1, (const double2*)F2, P, d_desc, d_cn, n_desc, partial);
-    else if (gen)
-        k_pair_reduce<float2, false, true><<<nblocks, RED_THREADS, shmem, ctx->stream>>>(
-            L, (const float2*)F1, (const float2*)F2, P, d_desc, d_cn, n_desc, partial);
-    else
-        k_pair_reduce<float2, false, false><<<nblocks, RED_THREADS, shmem, ctx->stream>>>(
-            L, (const float2*)F1, (const float2*)F2, P, d_desc, d_cn, n_desc, partial);
+    bool gen = false, los = false;
+    for (int b = 0; b < n_desc; ++b) {
+        los = los || descs[b].type >= HERMES_WIN_RING;
+        gen = gen || (descs[b].type >= HERMES_WIN_RING && descs[b].axis == 3);
+    }
+    auto go = [&](auto kernel, auto* f1, auto* f2) {
+        kernel<<<nblocks, RED_THREADS, shmem, ctx->stream>>>(L, f1, f2, P, d_desc, d_cn, n_desc, partial);
+    };
+    if (dbl) {
+        auto f1 = (const double2*)F1, f2 = (const double2*)F2;
+        if (gen) go(k_pair_reduce<double2, true, true, true>, f1, f2);
+        else if (los) go(k_pair_reduce<double2, true, false, true>, f1, f2);
+        else go(k_pair_reduce<double2, true, false, false>, f1, f2);
+    } else {
+        auto f1 = (const float2*)F1, f2 = (const float2*)F2;
+        if (gen) go(k_pair_reduce<float2, false, true, true>, f1, f2);
+        else if (los) go(k_pair_reduce<float2, false, false, true>, f1, f2);
+        else go(k_pair_reduce<float2, false, false, false>, f1, f2);
+    }
     HERMES_LAUNCH_CHECK();
     HERMES_CHECK_HIP(sum_columns(ctx->stream, partial, nblocks, n_desc, d_out));
     HERMES_CHECK_HIP(hipMemcpyAsync(out_host, d_out, sizeof(double) * n_desc, hipMemcpyDeviceToHost, ctx->stream));
