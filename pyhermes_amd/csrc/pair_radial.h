@@ -144,10 +144,15 @@ constexpr int radial_threads() {
 
 __host__ __device__ inline int tetra(int n) { return n * (n + 1) * (n + 2) / 6; }
 
+// Radii whose sums are reduced together.
+constexpr int radial_step(int lmax) { return lmax == 0 ? 4 : 1; }
+
 // Aliases whose state (6 + LMAX / 2 doubles each) a thread holds at a time: all eight in 256 registers up to l = 4;
 // beyond, eight leave 160 registers in scratch, four 60.
 constexpr int radial_aliases(int lmax) { return lmax <= 4 ? 8 : 4; }
 
+// Workgroup (row, group): blocks row, row + gridDim.x, ... and the `per` radii from group * per on (all of them unless
+// the rows alone leave SIMDs idle, see radial_groups).
 template <int LMAX, bool ROT, int BT, typename C>
 __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, const C* __restrict__ F1,
                                                                       const C* __restrict__ F2,
@@ -155,10 +160,10 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
                                                                       const double* __restrict__ radii, int nu,
                                                                       double R0, double dR,
                                                                       const int* __restrict__ chan, int nch, int nblk,
-                                                                      double* __restrict__ partial) {
+                                                                      int per, double* __restrict__ partial) {
     constexpr int NT = radial_threads<BT>(), NW = NT / 64, B3 = BT * BT * BT, PER = B3 / NT;
     constexpr int NE = LMAX / 2 + 1;         // even orders
-    constexpr int UC = LMAX == 0 ? 4 : 1;    // radii per reduction
+    constexpr int UC = radial_step(LMAX);    // radii per reduction
     constexpr int NA = radial_aliases(LMAX);
     constexpr int NQ = (UC * NE + 3) / 4;    // groups of four wave sums
     constexpr double XMIN = radial_xmin(LMAX);
@@ -168,6 +173,7 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
     __shared__ int cnt[PER * NW];
     const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
     const int half = L / 2;
+    const int ub = blockIdx.y * per, ue = min(nu, ub + per);
     for (int i = tid; i < NW * nch; i += NT) wacc[i] = 0.0;
     for (int blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
         int bi = (int)cbrtf(6.0f * (float)blk);
@@ -286,8 +292,8 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
                         chn[g] = (lane % 16 == 0 && n < UC * NE && u < nu) ? chan[u * (LMAX + 1) + 2 * (n % NE)] : -1;
                     }
                 };
-                fetch(0);
-                for (int u0 = 0; u0 < nu; u0 += UC) {
+                fetch(ub);
+                for (int u0 = ub; u0 < ue; u0 += UC) {
                     double kb[NQ * 4], Ru[UC], iRu[UC], sum[NQ];
                     int ch[NQ];
 #pragma unroll
@@ -351,7 +357,9 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
         }
     }
     __syncthreads();
-    for (int b = tid; b < nch; b += NT) {
+    for (int i = ub * (LMAX + 1) + tid; i < ue * (LMAX + 1); i += NT) {  // the channels of these radii
+        const int b = chan[i];
+        if (b < 0) continue;
         double s = 0.0;
         for (int w = 0; w < NW; ++w) s += wacc[w * nch + b];
         partial[(int64_t)blockIdx.x * nch + b] = s;

@@ -901,10 +901,21 @@ static std::vector<double> radius_table(const RadialChannels& ch) {
 
 static int radial_block_side(int J) { return J >= 8 ? 8 : 4; }
 
-// Rows of partial sums (workgroups) of the radial kernel: a block triple each, at most max_rows.
-static int radial_rows(int J, int max_rows) {
+// Rows of partial sums (workgroups) of the radial kernel: a block triple each while there are no more than 2048.
+static int radial_rows(int J) {
     const int nb = ((1 << J) / 2 + 1 + radial_block_side(J) - 1) / radial_block_side(J);
-    return std::min(max_rows, hermes_pair::tetra(nb));
+    return std::min(2048, hermes_pair::tetra(nb));
+}
+
+// Groups of radii, `per` in each.  Without rotated phases every radius costs a sin/cos per alias, a serial chain that
+// one wave per block of positions does not hide on small grids: there the radii are split (their channels are disjoint,
+// so a row of partial sums serves all groups) until a wave per SIMD is there; from L = 128 on the blocks fill the chip.
+// 30 log-spaced shells, FP32 spectra, whole calls: L = 64 106 us with all radii in one group, 53 now.
+static int radial_groups(int rows, int waves, int rot, int nu, int step, int* per) {
+    const int steps = (nu + step - 1) / step;
+    const int groups = rot ? 1 : std::max(1, std::min(steps, 1024 / (rows * waves)));
+    *per = (steps + groups - 1) / groups * step;
+    return (nu + *per - 1) / *per;
 }
 
 static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int rows, const void* F1, const void* F2,
@@ -913,12 +924,15 @@ static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int rows
     using namespace hermes_pair;
     const int L = 1 << J, bt = radial_block_side(J), nb = (L / 2 + 1 + bt - 1) / bt, nblk = tetra(nb);
     hipError_t e = hipSuccess;
+    int per = nu;
+    const int groups = radial_groups(rows, bt == 8 ? 4 : 1, rot, nu, radial_step(LM), &per);
     auto go = [&](auto kernel, int threads, auto* f1, auto* f2) {
         const size_t shmem = sizeof(double) * (threads / 64) * nch;
         if (shmem > 32 * 1024)  // beside up to 25 KB of powers
             e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         if (e == hipSuccess)
-            kernel<<<rows, threads, shmem, st>>>(L, f1, f2, P, d_radii, nu, R0, dR, d_chan, nch, nblk, partial);
+            kernel<<<dim3(rows, groups), threads, shmem, st>>>(L, f1, f2, P, d_radii, nu, R0, dR, d_chan, nch, nblk, per,
+                                                               partial);
     };
 #define HERMES_RADIAL(LMV, ROT)                                                                                      \
     do {                                                                                                             \
@@ -960,11 +974,6 @@ static size_t pair_partial_bytes(int rows, int n) {
     return sizeof(double) * ((size_t)rows * n + (size_t)((rows + 63) / 64) * n + n);
 }
 
-static int pair_blocks(int J) {
-    const int Lh = (1 << J) / 2 + 1;
-    return (int)hermes_blocks((int64_t)Lh * Lh * Lh, RED_THREADS, 2048);
-}
-
 // The radial path of hermes_pair_reduce.  Returns false (rc untouched) when it does not apply;
 // true with rc = the status otherwise.
 static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, const void* F2, const double* P,
@@ -976,7 +985,8 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     const int nu = ch.nu, nch = ch.nch;
     const size_t off_chan = sizeof(double) * 2 * nu;
     const size_t off_part = ((off_chan + sizeof(int) * ch.chan.size() + 255) / 256) * 256;
-    const size_t need = off_part + pair_partial_bytes(nblocks, nch);
+    const int rows = radial_rows(J);
+    const size_t need = off_part + pair_partial_bytes(std::max(nblocks, rows), nch);
     char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);
     if (!ws) {
         rc = fixed_ws ? 2 : 1;
@@ -986,7 +996,6 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     int* d_chan = (int*)(ws + off_chan);
     double* d_out = (double*)(ws + off_part);
     double* partial = d_out + nch;
-    const int rows = radial_rows(J, nblocks);
     auto fail = [&](hipError_t e) {
         hermes_set_error("pair reduction: %s", hipGetErrorString(e));
         rc = 1;
@@ -1117,7 +1126,7 @@ int hermes_pair_plan_create(hermes_ctx* ctx, int J, int dbl, const hermes_window
     p->R0 = ch.R0;
     p->dR = ch.dR;
     p->n_desc = n_desc;
-    p->nblocks = radial_rows(J, pair_blocks(J));
+    p->nblocks = radial_rows(J);
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t o_chan = al(sizeof(double) * 2 * ch.nu), o_chof = o_chan + al(sizeof(int) * ch.chan.size()),
                  o_fac = o_chof + al(sizeof(int) * n_desc), o_part = o_fac + al(sizeof(double) * n_desc),

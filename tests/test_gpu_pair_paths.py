@@ -81,3 +81,17 @@ def test_mixed_axes_keep_the_general_kernel(phi):
     got = kernels.pair_reduce(F1, F2, P, descs)
     one = np.array([kernels.pair_reduce(F1, F2, P, [d])[0] for d in descs])
     assert np.abs(got - one).max() <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("J,n,ells,dtype", [(2, 5, (0,), "float32"), (3, 30, (0, 2), "float64"), (4, 9, (0, 10), "float32"),
+                                            (5, 31, (0,), "float64"), (6, 30, (0,), "float32"), (6, 13, (2, 4), "float64")])
+def test_radial_kernel_with_split_radii(phi, J, n, ells, dtype):
+    """Unevenly spaced radii on small grids, split over workgroups (groups of one and of several steps, a ragged last
+    one); the first radius carries one order only, so the groups' channel counts differ."""
+    import torch
+    from pyhermes_amd import kernels
+    R = np.geomspace(0.02, 0.4, n) * (1 << J)
+    descs = [kernels.window_desc("shell_multipole", r, l=l) if l else kernels.window_desc("shell", r)
+             for l in ells for r in (R[1:] if l == ells[-1] and len(ells) > 1 else R)]
+    print(f"radial split J={J} n={n} l={ells} {dtype}", flush=True)
+    _compare(phi, J, getattr(torch, dtype), descs, 300 + J)
