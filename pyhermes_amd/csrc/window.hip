@@ -984,9 +984,13 @@ static bool pair_reduce_radial(hermes_ctx* ctx, int J, int dbl, const void* F1, 
     rc = 0;
     const int nu = ch.nu, nch = ch.nch;
     const size_t off_chan = sizeof(double) * 2 * nu;
-    const size_t off_part = ((off_chan + sizeof(int) * ch.chan.size() + 255) / 256) * 256;
+    const size_t off_part = (off_chan + sizeof(int) * ch.chan.size() + 7) / 8 * 8;
     const int rows = radial_rows(J);
-    const size_t need = off_part + pair_partial_bytes(std::max(nblocks, rows), nch);
+    // asked for: one double per radius, the channels and the partial sums with their group sums, whose room the second
+    // double of a radius takes (nch >= nu); more only on the small grids, far from the fixed scratch's size
+    const size_t asked = (sizeof(double) * nu + sizeof(int) * ch.chan.size() + 255) / 256 * 256 +
+                         pair_partial_bytes(nblocks, nch);
+    const size_t need = std::max(asked, off_part + sizeof(double) * ((size_t)rows + 1) * nch);
     char* ws = pair_workspace(ctx, fixed_ws, fixed_cap, need);
     if (!ws) {
         rc = fixed_ws ? 2 : 1;

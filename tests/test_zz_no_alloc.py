@@ -100,3 +100,17 @@ def test_noalloc_rejects_requests_beyond_its_scratch(phi):
     ok = _call("hermes_pair_reduce", J, True, F1, F2, Pd, descs[:8])
     again = _call("hermes_pair_reduce_noalloc", J, True, F1, F2, Pd, descs[:8])
     np.testing.assert_array_equal(again, ok)
+
+
+def test_noalloc_serves_what_just_fits_its_scratch(phi):
+    """503 radii with one l = 4 window each at L = 256 ask for 8,388,280 of the 8,388,608 bytes; 504 do not fit."""
+    import torch
+    from pyhermes_amd import _lib, kernels
+    print("noalloc edge of its scratch: J=8 503 and 504 windows", flush=True)
+    J, L = 8, 256
+    descs = [kernels.window_desc("shell_multipole", R, l=4) for R in np.linspace(1.0, 60.0, 504)]
+    got, want = _case(phi, J, True, descs[:503], 41)
+    assert np.all(np.isfinite(want))
+    np.testing.assert_array_equal(got, want)
+    with pytest.raises(RuntimeError, match="status 2"):
+        _case(phi, J, True, descs, 41)
