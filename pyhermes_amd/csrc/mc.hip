@@ -675,13 +675,23 @@ __global__ __launch_bounds__(BK_THREADS) void k_bucket_scatter(const unsigned ch
 
 }  // namespace
 
+// Whether `items` lanes' work fills the rounds of waves that `waves` per SIMD give, the last one to a share of
+// `least`.  A wave on bricks walks eight rounds of lines a vertex, and a round of waves that is nearly empty costs as
+// much as a full one; a point per lane loses less there.
+static bool rounds_filled(hermes_ctx* ctx, double items, int waves, double least) {
+    const double rounds = items / (256.0 * waves * ctx->n_cu);
+    return rounds >= 3.0 || rounds >= least * std::ceil(rounds);
+}
+
 // Layout for `points` interpolations on the n_grid grids g (replaced by their bricked copies where they are made).
-// A copy reads and writes the grid once, which pays from about one point per 8 cells on (L = 512, 4e6 triangles, one per 11:
-// 3.9 against 3.4 ms; L = 256, 1e6, one per 6: 0.94 against 1.22); below L = 128 the grid
-// stays in the L2 caches and a point per lane is the faster way (2e7 uniform triangles: L = 64 3.8 ms, with bricks
-// 4.4; L = 128 8.8 and 7.2; L = 256 11.8 and 7.6; L = 512 21.3 and 12.5).  The copies are kept within 4 GiB.  Grids
-// not aligned to 16 bytes are bricked under the same rule or read by 8 bytes.
-static int grid_layout(hermes_ctx* ctx, int J, double points, const double** g, int n_grid) {
+// filled: by rounds_filled (2e5, 3e5 and 1e6 triangles at L = 128: 318, 369 and 974 us by a point per lane, 301, 441
+// and 832 with bricks).  A copy reads and writes the grid once, which pays from about one point per 14 cells on while
+// source and copy stay near the last-level cache (L = 256, 2.5e5 and 4e5 triangles: 407 and 603 us plain, 378 and 547
+// bricked), one per 8 up to 512 MiB of copies and one per 5 beyond (L = 512, 6e6: 4.8 ms plain, 5.1 bricked; 1e7: 7.4
+// and 7.2).  Below L = 128 the grid stays in the L2 caches and a point per lane is the faster way (2e7 uniform
+// triangles: L = 64 3.8 ms, with bricks 4.4; L = 128 8.8 and 7.2; L = 256 11.8 and 7.6).  The copies are kept within
+// 4 GiB.  Grids not aligned to 16 bytes are bricked under the same rule or read by 8 bytes.
+static int grid_layout(hermes_ctx* ctx, int J, double points, bool filled, const double** g, int n_grid) {
     const size_t n = (size_t)1 << (3 * J);
     bool aligned = true;
     for (int i = 0; i < n_grid; ++i) aligned = aligned && ((uintptr_t)g[i] & 15) == 0;
@@ -694,7 +704,9 @@ static int grid_layout(hermes_ctx* ctx, int J, double points, const double** g, 
         if (k == copies) distinct[copies++] = g[i];
         of[i] = k;
     }
-    if (J < 7 || points * 8.0 < (double)n * copies || copies * n * sizeof(double) > ((size_t)4 << 30)) return plain;
+    const double cells = (double)n * copies;
+    const double per = cells <= 0x1p24 ? 14.0 : (cells <= 0x1p26 ? 8.0 : 5.0);
+    if (J < 7 || !filled || points * per < cells || cells * sizeof(double) > 0x1p32) return plain;
     double* ws = (double*)hermes_workspace(ctx, WS_SPEC, copies * n * sizeof(double));
     if (!ws) return plain;
     for (int k = 0; k < copies; ++k)
@@ -737,8 +749,9 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     k_triplet_offsets<<<hermes_blocks(n_rot, 64), 64, 0, ctx->stream>>>(R1, R2, mu, d_abc, n_rot, d_off);
     HERMES_LAUNCH_CHECK();
     const double* g[2] = {g2, g3};
+    const double items = (double)n * n_rot;
     // the LDS table and the packed fractions of the faster layouts hold 1024 samples to a cell
-    const int layout = phi_res == 1024 ? grid_layout(ctx, J, 2.0 * (double)n * n_rot, g, 2) : -1;
+    const int layout = phi_res == 1024 ? grid_layout(ctx, J, 2.0 * items, rounds_filled(ctx, items, 6, 0.55), g, 2) : -1;
     auto go = [&](auto kernel) {
         kernel<<<dim3(nbx, nby), MC_THREADS, 0, ctx->stream>>>(spos, n1, n, n_rot, d_off, g[0], g[1], phi, J, phi_res, ws);
     };
@@ -815,7 +828,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
     unsigned long long* stats = acc_hi + 2 * (size_t)B;
     int64_t* over_list = (int64_t*)(ws + sizeof(unsigned long long) * n_acc);
     const double* g[3] = {g1, g2, g3};
-    const int layout = grid_layout(ctx, J, 3.0 * (double)n_samples, g, 3);
+    const double all = (double)n_samples, pilot = wf_cap > 0.0 ? 0.0 : (double)std::min(n_samples, PILOT);
+    const int layout = grid_layout(ctx, J, 3.0 * (all + pilot), rounds_filled(ctx, all, 4, 0.67), g, 3);
     // workgroups load the scaling function once and loop over samples
     auto launch = [&](auto brick, auto aligned, auto plain, const BinnedArgs& args, const int64_t* list, float* out) {
         auto kernel = layout == GRID_BRICK ? brick : (layout == GRID_ALIGNED ? aligned : plain);

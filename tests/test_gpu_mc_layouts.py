@@ -118,3 +118,49 @@ def test_triplet_with_another_table_resolution(level, offset):
         t = n1 * omc.interpolate(g2, spos, phi, o[:3], res) * omc.interpolate(g3, spos, phi, o[3:], res)
         ref, mag = ref + t.sum(), mag + np.abs(t).sum()
     assert abs(got[0] - ref / (n * n_rot)) <= 1e-12 * mag / (n * n_rot)
+
+
+@pytest.mark.parametrize("n,offset,same", [(200_003, 0, True), (200_003, 1, False), (262_145, 0, True), (400_001, 1, True)])
+def test_binned_sampler_rounds(phi, n, offset, same):
+    """Sample counts at both sides of the rule for bricks: a round of waves filled by three quarters (bricks), one
+    sample more than a round (plain), a round and a half (bricks)."""
+    from pyhermes_amd import kernels
+    L, nbins, r1r, r2r, seed = 128, (3, 4, 5), (1.5, 9.0), (2.0, 38.0), 23
+    g = [_grid(L, 1)] * 3 if same else [_grid(L, s) for s in (1, 2, 3)]
+    gd = [_device(g[0], offset)] * 3 if same else [_device(a, offset) for a in g]
+    print(f"binned rounds n={n} offset={offset} same={same}", flush=True)
+    ref = omc.binned_sampler(*g, phi, nbins, r1r, r2r, n, seed)
+    got = kernels.mc_binned(*gd, phi, nbins, r1r, r2r, n, seed)
+    assert np.array_equal(got[2], ref[2])
+    for a, b in zip(got[:2], ref[:2]):
+        np.testing.assert_allclose(a, b, rtol=1e-9, atol=1e-9 * np.abs(b).max())
+
+
+@pytest.mark.parametrize("n", [300_000, 400_000])
+def test_non_finite_cells_stay_apart_at_both_layouts(phi, n):
+    """Three quarters of a round of waves (bricks) and one that is just over (plain): a NaN or an infinite cell reaches
+    the triangles whose neighbourhoods hold it and no other."""
+    from pyhermes_amd import kernels
+    import torch
+    L = 128
+    g = _grid(L, 8)
+    bad = g.copy()
+    bad[5, 6, 7], bad[70, 3, 2] = np.nan, np.inf
+    rng = np.random.default_rng(4)
+    spos, abc = rng.uniform(0, L, size=(n, 3)), rng.random((1, 3))
+    args = (9.0, 14.0, 0.2)
+    o = omc.triangle_offsets(*args, *(2 * np.pi * abc[0, 0], 2 * abc[0, 1] - 1, 2 * np.pi * abc[0, 2]))
+    hit = np.zeros(n, bool)
+    for k in (0, 3):
+        c = np.floor(spos + o[k:k + 3]).astype(int)
+        for cell in ((5, 6, 7), (70, 3, 2)):
+            hit |= np.all((c - np.array(cell)) % L <= 2, axis=1)
+    assert 0 < hit.sum() < 300
+    clean = np.where(hit[:, None], spos[~hit][0], spos)
+    n1 = np.where(hit, 0.0, 1.0)
+    dev = lambda a: kernels.as_device(a, torch.float64)
+    print(f"non-finite cells n={n}", flush=True)
+    want = kernels.mc_triplet_box(*args, dev(clean), dev(n1), abc, dev(g), dev(g), phi)
+    got = kernels.mc_triplet_box(*args, dev(clean), dev(n1), abc, dev(bad), dev(bad), phi)
+    assert np.isfinite(got) and got == want
+    assert not np.isfinite(kernels.mc_triplet_box(*args, dev(spos), dev(n1 * 0 + 1), abc, dev(bad), dev(bad), phi))
