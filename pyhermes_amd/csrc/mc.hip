@@ -184,9 +184,19 @@ __global__ __launch_bounds__(256) void k_brick(const double* __restrict__ g, int
     }
 }
 
-// The scaling function in LDS, tap-interleaved; res = 1024.
-__device__ __forceinline__ void load_phi(double* sphi, const double* __restrict__ phi, int tid, int nt) {
-    for (int i = tid; i < 3 * 1024; i += nt) sphi[3 * (i & 1023) + (i >> 10)] = phi[i];
+// The scaling function in LDS, tap-interleaved; res = 1024.  All loads are in flight before the first store (a call of
+// 60,000 triangles is one workgroup to a CU and waits for them twice).
+template <int NT>
+__device__ __forceinline__ void load_phi(double* sphi, const double* __restrict__ phi, int tid) {
+    static_assert(3 * 1024 % NT == 0, "table staging");
+    double v[3 * 1024 / NT];
+#pragma unroll
+    for (int j = 0; j < 3 * 1024 / NT; ++j) v[j] = phi[tid + j * NT];
+#pragma unroll
+    for (int j = 0; j < 3 * 1024 / NT; ++j) {
+        const int i = tid + j * NT;
+        sphi[3 * (i & 1023) + (i >> 10)] = v[j];
+    }
 }
 
 __global__ void k_interpolate(const double* __restrict__ g, const double* __restrict__ spos, int64_t n,
@@ -258,7 +268,7 @@ __global__ __launch_bounds__(MC_THREADS, 4) void k_triplet_box(const double* __r
     __shared__ double sphi[SPHI ? 3 * 1024 : 1];
     __shared__ double sh[MC_THREADS / 64];
     if constexpr (SPHI) {
-        load_phi(sphi, phi, threadIdx.x, MC_THREADS);
+        load_phi<MC_THREADS>(sphi, phi, threadIdx.x);
         __syncthreads();
     }
     auto value = [&](const double* g, double x, double y, double z) {
@@ -489,7 +499,7 @@ __global__ __launch_bounds__(MC_THREADS, 4) void k_mc_binned(
     unsigned long long* __restrict__ stats, int64_t* __restrict__ over_list, float* __restrict__ rec) {
     __shared__ double red[MC_THREADS / 64];
     __shared__ double sphi[3 * 1024];
-    load_phi(sphi, phi, threadIdx.x, MC_THREADS);
+    load_phi<MC_THREADS>(sphi, phi, threadIdx.x);
     __syncthreads();
     const int B = A.nr1 * A.nr2 * A.nmu;
     double mx = 0.0;
