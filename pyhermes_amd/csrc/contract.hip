@@ -486,6 +486,8 @@ __global__ __launch_bounds__(64 * D2::WAVES, 4) void k_gram_auto(const float* __
 // plane is complete.  250 VALU instructions and 6 matrix instructions per wave and plane, where the eigen form in
 // all three directions took 54 matrix instructions, about 600 VALU instructions and uncoalesced loads (each lane
 // read its shell's taps from memory).  Bound by VALU and LDS.  11 x 15 shells at L = 128: 1417 us before, 388 us now.
+// FP32 sums go to FP64 after at most four planes, 96 products (the eigen form's chains: 108).  Against FP64 on the same
+// fields the largest error is 0.5 to 1.2e-7 of the largest entry at L = 32 to 128, the eigen form's 1.3 to 1.4e-7.
 // Step p (W = V): planes of V: p+2 into the operands, y taps of p+3, staged store of p+4, load of p+5; planes of U:
 // p finished, staged store of p+1, load of p+2.
 template <int NNEG>
@@ -683,7 +685,7 @@ __global__ __launch_bounds__(64 * D2X::WAVES, 3) void k_gram_cross(const float* 
             ustore(p + 1);                                                                          \
             uload(p + 2);                                                                           \
         }                                                                                           \
-        if ((p - x0) % 6 == 5 || p + 1 >= xend) { /* at most six planes in FP32 */                  \
+        if ((p - x0) % 4 == 3 || p + 1 >= xend) { /* at most four planes in FP32 */                 \
             _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                         \
                 acc_slot[j] += (double)accr[j];                                                     \
                 accr[j] = 0.f;                                                                      \
