@@ -58,7 +58,7 @@ def _multipole_field_f64(geo, spec, edge, l, m, out):
 
 
 def _full_spectrum_f64(d):
-    c = torch.complex(d, torch.zeros_like(d))
+    c = torch.complex(d, torch.zeros_like(d)).contiguous()
     return kernels.fftn_c2c(c, out=c)
 
 
@@ -67,6 +67,7 @@ def ddd_multipole_plain_f64(geo, d1, d2, d3, R12_grid, R13_grid, l_min, l_max, r
     """One (r12, r13) set in FP64, term by term as the reference sequences it; the fields are transformed once per
     call.  d*: (L,L,L) float64."""
     N = geo.L ** 3
+    d1 = d1.contiguous()
     spec2 = _full_spectrum_f64(d2)
     spec3 = spec2 if d3 is d2 else _full_spectrum_f64(d3)
     F1, F2 = torch.empty_like(spec2), torch.empty_like(spec2)
