@@ -68,3 +68,27 @@ def test_convolution(J, dtype):
     spec *= k.double()
     _check(got, torch.fft.irfftn(spec, s=(L, L, L)), 2 * J, dtype)
     assert torch.equal(x, keep)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_convolution_of_the_largest_grid(dtype):
+    """L = 1024 (up to 147 KB of LDS in the fused pass), with a product of one filter per axis, so that the reference
+    is three passes of 1-D transforms."""
+    J = 10
+    L = 1 << J
+    x = _field((L, L, L), dtype)
+    f = _field((L // 2 + 1,), dtype, 4)
+    full = torch.cat([f, f[1:-1].flip(0)])
+    k = full[:, None, None] * full[None, :, None] * f
+    print(f"convolution J=10 {dtype}", flush=True)
+    got = kernels.convolve_real(x, k, 1.0 / L ** 3)
+    del k
+    want = x.double()
+    del x
+    shape = [(L // 2 + 1, 1, 1), (L // 2 + 1, 1), (L // 2 + 1,)]
+    for axis in range(3):
+        spec = torch.fft.rfft(want, dim=axis)
+        spec *= f.double().view(shape[axis])
+        want = torch.fft.irfft(spec, n=L, dim=axis)
+        del spec
+    _check(got, want, 2 * J, dtype)

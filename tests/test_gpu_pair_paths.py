@@ -95,3 +95,31 @@ def test_radial_kernel_with_split_radii(phi, J, n, ells, dtype):
              for l in ells for r in (R[1:] if l == ells[-1] and len(ells) > 1 else R)]
     print(f"radial split J={J} n={n} l={ells} {dtype}", flush=True)
     _compare(phi, J, getattr(torch, dtype), descs, 300 + J)
+
+
+def test_line_of_sight_tables_beyond_the_default_lds(phi):
+    """L = 1024: 70 KB of staged powers, above the dynamic LDS a kernel gets unasked.  Radii and heights keep the
+    arguments below 1000."""
+    import torch
+    from pyhermes_amd import kernels
+    L = 1024
+    types = ("ring", "disk", "cylshell", "cylinder")
+    descs = [kernels.window_desc(t, 0.02 * L * (i + 1), 0.015 * L * i, axis=1) for i, t in enumerate(types)]
+    print("line of sight J=10", flush=True)
+    _compare(phi, 10, torch.float32, descs, 210)
+
+
+@pytest.mark.parametrize("spacing", ["linear", "uneven"])
+def test_radial_pass_with_many_channels(phi, spacing):
+    """1500 radii at L = 256: 47 KB of channel sums beside the staged powers, above the dynamic LDS a kernel gets
+    unasked; a subset of the radii through the general kernel."""
+    import torch
+    from pyhermes_amd import kernels
+    J, L = 8, 256
+    R = np.linspace(0.01 * L, 0.3 * L, 1500) if spacing == "linear" else np.geomspace(0.01 * L, 0.3 * L, 1500)
+    descs = [kernels.window_desc("shell", r) for r in R]
+    F1, F2, P, scale = _spectra(phi, J, torch.float64, 11)
+    print(f"radial J=8 1500 channels {spacing}", flush=True)
+    got = kernels.pair_reduce(F1, F2, P, descs)
+    ref = kernels.pair_reduce(F1, F2, P, descs[::75] + [kernels.window_desc("sphere", 2.0)])[:-1]
+    assert np.abs(got[::75] - ref).max() <= 1e-12 * scale
