@@ -164,3 +164,41 @@ def test_non_finite_cells_stay_apart_at_both_layouts(phi, n):
     got = kernels.mc_triplet_box(*args, dev(clean), dev(n1), abc, dev(bad), dev(bad), phi)
     assert np.isfinite(got) and got == want
     assert not np.isfinite(kernels.mc_triplet_box(*args, dev(spos), dev(n1 * 0 + 1), abc, dev(bad), dev(bad), phi))
+
+
+@pytest.mark.parametrize("J", [9, 10])
+def test_triplet_on_the_largest_grids(phi, J):
+    """1.7e7 triangles on a 512^3 grid (bricks: 1 GiB of copies) and a 1024^3 one (its copy would pass 4 GiB: read as
+    it is), against gathers in torch."""
+    import torch
+    from pyhermes_amd import kernels
+    L, n, n_rot = 1 << J, (1 << 18) + 3, 64
+    gen = torch.Generator(device="cuda").manual_seed(J)
+    g = torch.randn((L, L, L), generator=gen, device="cuda", dtype=torch.float64)
+    spos = torch.rand((n, 3), generator=gen, device="cuda", dtype=torch.float64) * L
+    n1 = torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
+    abc = np.random.default_rng(J).random((n_rot, 3))
+    ph = kernels.as_device(phi, torch.float64)
+
+    def value(s):
+        c = torch.floor(s)
+        f = torch.clamp(((s - c) * 1024).long(), max=1023)
+        c = c.long()
+        out = torch.zeros(n, dtype=torch.float64, device="cuda")
+        for a in range(3):
+            for b in range(3):
+                for e in range(3):
+                    i = (((c[:, 0] - a) % L) * L + (c[:, 1] - b) % L) * L + (c[:, 2] - e) % L
+                    out += g.view(-1)[i] * ph[f[:, 0] + 1024 * a] * ph[f[:, 1] + 1024 * b] * ph[f[:, 2] + 1024 * e]
+        return out
+
+    args = (0.02 * L, 0.05 * L, 0.4)
+    print(f"triplet J={J}", flush=True)
+    got = kernels.mc_triplet_box(*args, spos, n1, abc, g, g, phi)
+    ref, mag = 0.0, 0.0
+    for a, b, c in abc:
+        o = torch.from_numpy(omc.triangle_offsets(*args, 2 * np.pi * a, 2 * b - 1, 2 * np.pi * c)).cuda()
+        t = n1 * value(spos + o[:3]) * value(spos + o[3:])
+        ref, mag = ref + float(t.sum()), mag + float(t.abs().sum())
+    kernels.release_workspaces()
+    assert abs(got - ref / (n * n_rot)) <= 1e-12 * mag / (n * n_rot)
