@@ -35,15 +35,17 @@ __device__ __forceinline__ double make_f64(unsigned lo, unsigned hi) {
 
 // a summed over the two half-waves in lanes 0..31, b in lanes 32..63.
 __device__ __forceinline__ double merge32(double a, double b) {
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
     return make_f64(lo[0], hi[0]) + make_f64(lo[1], hi[1]);
 }
 
 // Rows of 16 lanes: a summed over row pairs (0, 1) and (2, 3) in rows 0 and 2, b in rows 1 and 3.
 __device__ __forceinline__ double merge16(double a, double b) {
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
     return make_f64(lo[0], hi[0]) + make_f64(lo[1], hi[1]);
 }
 
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
     __shared__ int cnt[PER * NW];
     const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
     const int half = L / 2;
-    const int ub = blockIdx.y * per, ue = min(nu, ub + per);
+    const int ub = ROT ? 0 : blockIdx.y * per, ue = ROT ? nu : min(nu, ub + per);
     for (int i = tid; i < NW * nch; i += NT) wacc[i] = 0.0;
     for (int blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
         int bi = (int)cbrtf(6.0f * (float)blk);
@@ -195,7 +197,8 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
                 for (int q = 0; q < PER; ++q) {
                     const int r = tid + q * NT;
                     const int x = X * BT + r / (BT * BT), y = Y * BT + (r / BT) % BT, z = Z * BT + r % BT;
-                    const double p = octant_power<decltype(same)::value>(F1, F2, L, min(x, half), min(y, half), min(z, half));
+                    const double p = octant_power<decltype(same)::value>(F1, F2, L, min(x, half), min(y, half),
+                                                                         min(z, half));
                     pw[o * B3 + r] = (x <= half && y <= half && z <= half) ? p : 0.0;
                 }
             }
@@ -275,8 +278,8 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
                         sincospi(2.0 * (td - floor(td)), &sd[a], &cd[a]);
                     }
                 }
-                // radii and channels of the next step are fetched a step ahead, and the channels' sums are read before the
-                // step's arithmetic: two waves per SIMD do not cover their latencies
+                // radii and channels of the next step are fetched a step ahead, and the channels' sums are read before
+                // the step's arithmetic: two waves per SIMD do not cover their latencies
                 double Rn[UC], iRn[UC];
                 int chn[NQ];
                 auto fetch = [&](int u0) {
@@ -357,12 +360,16 @@ __global__ __launch_bounds__(radial_threads<BT>(), 2) void k_pair_radial(int L, 
         }
     }
     __syncthreads();
-    for (int i = ub * (LMAX + 1) + tid; i < ue * (LMAX + 1); i += NT) {  // the channels of these radii
-        const int b = chan[i];
-        if (b < 0) continue;
+    auto finish = [&](int b) {
         double s = 0.0;
         for (int w = 0; w < NW; ++w) s += wacc[w * nch + b];
         partial[(int64_t)blockIdx.x * nch + b] = s;
+    };
+    if constexpr (ROT) {
+        for (int b = tid; b < nch; b += NT) finish(b);
+    } else {  // the channels of these radii
+        for (int i = ub * (LMAX + 1) + tid; i < ue * (LMAX + 1); i += NT)
+            if (chan[i] >= 0) finish(chan[i]);
     }
 }
 
