@@ -89,8 +89,8 @@ int hermes_delta_f32(hermes_ctx *ctx, int64_t n, const float *eps, double a, dou
 int hermes_half_spectrum_f32(hermes_ctx *ctx, int J, const void *full, void *half);
 
 
-/* ---- 3-D FFTs (rocFFT plans; from 128^3 on the strided lines by own kernels), replacing scipy.fft rfftn / irfftn / fftn / ifftn in
- * convolution.py:284-295.  Unnormalised; batch transforms are contiguous
+/* ---- 3-D FFTs (rocFFT plans; from 128^3 on the strided lines by own kernels), replacing
+ * scipy.fft rfftn / irfftn / fftn / ifftn in convolution.py:284-295.  Unnormalised; batch transforms are contiguous
  * (batch, L, L, L).  c2r clobbers its input.  in == out selects in-place (c2c only). */
 int hermes_fft_r2c(hermes_ctx *ctx, int J, int batch, int dbl, const void *in_real, void *out_half);
 int hermes_fft_c2r(hermes_ctx *ctx, int J, int batch, int dbl, void *in_half, void *out_real);
@@ -206,8 +206,9 @@ int hermes_convolve_real(hermes_ctx *ctx, int J, int dbl, const void *in_real, c
  * corr2pcf.py:366-372): for every descriptor b,
  *   out[b] = sum_{k, full grid} K_b(k) Re(F1(k) conj F2(k))
  * from the half spectra F1, F2 (F2 may equal F1) in one pass over the spectrum.
- * The caller divides by N^2.  dbl: spectra are complex128 (FP64 evaluation)
- * or complex64 (FP32 evaluation); accumulation is FP64 and deterministic. */
+ * The caller divides by N^2.  dbl: spectra are complex128 or complex64.  Powers, sums and windows are
+ * FP64 (deterministic), but for complex64 spectra in a list that mixes kinds of windows or axes, whose thin
+ * shells and multipoles are evaluated in FP32. */
 int hermes_pair_reduce(hermes_ctx *ctx, int J, int dbl, const void *F1, const void *F2, const double *P,
                        const hermes_window_desc *descs, int n_desc, double *out_host);
 

@@ -751,7 +751,8 @@ int hermes_multipole_summand_f64(hermes_ctx* ctx, int J, const double* d1, const
     int xseg = L < 64 ? L : 64;
     while (xseg > 4 && nyz * (L / xseg) < 1024) xseg /= 2;
     const int nb = nyz * (L / xseg);
-    double* ws = (double*)hermes_workspace(ctx, WS_CONTRACT, sizeof(double) * (2 * (size_t)nb + 2 + 2 * (size_t)hermes_reduce::sum_scratch_rows(nb)));
+    const size_t scratch = 2 * (size_t)hermes_reduce::sum_scratch_rows(nb);
+    double* ws = (double*)hermes_workspace(ctx, WS_CONTRACT, sizeof(double) * (2 * (size_t)nb + 2 + scratch));
     HERMES_REQUIRE(ws, "%s", hermes_last_error());
     Gamma3 G;
     for (int i = 0; i < 9; ++i) G.g[i] = gamma3x3_host[i];
@@ -828,7 +829,7 @@ static int gram_launch(hermes_ctx* ctx, int J, const float* d1, const void* U, i
     HERMES_REQUIRE(!split || !g.cross, "hermes_multipole_gram_f32: split sums are for the auto Gram");
     const int row = split ? 512 : 256;
     double* ws = (double*)hermes_workspace(
-        ctx, WS_CONTRACT, sizeof(double) * ((size_t)nblocks * row + (size_t)hermes_reduce::sum_scratch_rows(nblocks) * row));
+        ctx, WS_CONTRACT, sizeof(double) * row * ((size_t)nblocks + (size_t)hermes_reduce::sum_scratch_rows(nblocks)));
     HERMES_REQUIRE(ws, "%s", hermes_last_error());
     const bool timed = ctx->time_gram && !ctx->capturing;
     size_t slot = 0;

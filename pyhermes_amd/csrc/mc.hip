@@ -31,8 +31,8 @@ constexpr double TWO_PI = 6.283185307179586476925286766559;
 //                 16-byte pair of the line, so each of the 4 or 8 lines that a 3 x 3 x 3 neighbourhood meets (6 on
 //                 average; 9 * 1.125 in the plain layout) is requested once, by one instruction
 // Interpolation at random points is bound by the lines a CU can have outstanding, not by bytes or arithmetic: more
-// waves per SIMD or fewer lines read by one lane at a time do not help (2e7 triangles at L = 256: 11.1 ms with one
-// wave per SIMD, 11.8 with four, 13.9 with bricks read by one lane), fewer line requests do.
+// waves per SIMD or fewer lines read by one lane at a time do not help (whole calls of 2e7 triangles at L = 256:
+// 11.1 ms with one wave per SIMD, 11.8 with four, 13.9 with bricks read by one lane), fewer line requests do (7.6).
 enum GridLayout { GRID_PLAIN = 0, GRID_ALIGNED = 1, GRID_BRICK = 2 };
 
 template <int LAYOUT>
@@ -489,8 +489,8 @@ enum McPass { MC_PILOT = 0, MC_MAIN = 1, MC_FIXUP = 2 };
 // bit pattern of a non-negative double, whose integer order is the numeric order;
 // stats[1] counts overflow samples.  Fixed-point sums make the result
 // independent of the order of the atomics.
-// Bound by the random lines of the grids (see GridLayout).  2e7 uniform triangles at L = 256: 10.4 ms with one lane
-// per triangle and 27 loads per vertex, 7.0 ms with bricks.
+// Bound by the random lines of the grids (see GridLayout).  2e7 uniform triangles at L = 256, the main pass alone:
+// 10.4 ms with one lane per triangle and 27 loads per vertex, 7.0 ms with bricks.
 template <int PASS, int LAYOUT>
 __global__ __launch_bounds__(MC_THREADS, 4) void k_mc_binned(
     const double* __restrict__ g1, const double* __restrict__ g2, const double* __restrict__ g3,
@@ -698,9 +698,9 @@ static bool rounds_filled(hermes_ctx* ctx, double items, int waves, double least
 // and 832 with bricks).  A copy reads and writes the grid once, which pays from about one point per 14 cells on while
 // source and copy stay near the last-level cache (L = 256, 2.5e5 and 4e5 triangles: 407 and 603 us plain, 378 and 547
 // bricked), one per 8 up to 512 MiB of copies and one per 5 beyond (L = 512, 6e6: 4.8 ms plain, 5.1 bricked; 1e7: 7.4
-// and 7.2).  Below L = 128 the grid stays in the L2 caches and a point per lane is the faster way (2e7 uniform
-// triangles: L = 64 3.8 ms, with bricks 4.4; L = 128 8.8 and 7.2; L = 256 11.8 and 7.6).  The copies are kept within
-// 4 GiB.  Grids not aligned to 16 bytes are bricked under the same rule or read by 8 bytes.
+// and 7.2).  Below L = 128 the grid stays in the L2 caches and a point per lane is the faster way (whole calls of 2e7
+// uniform triangles: L = 64 3.8 ms, with bricks 4.4; L = 128 8.8 and 7.2; L = 256 11.8 and 7.6).  The copies are kept
+// within 4 GiB.  Grids not aligned to 16 bytes are bricked under the same rule or read by 8 bytes.
 static int grid_layout(hermes_ctx* ctx, int J, double points, bool filled, const double** g, int n_grid) {
     const size_t n = (size_t)1 << (3 * J);
     bool aligned = true;
@@ -761,9 +761,11 @@ int hermes_mc_triplet_box(hermes_ctx* ctx, int J, double R1, double R2, double m
     const double* g[2] = {g2, g3};
     const double items = (double)n * n_rot;
     // the LDS table and the packed fractions of the faster layouts hold 1024 samples to a cell
-    const int layout = phi_res == 1024 ? grid_layout(ctx, J, 2.0 * items, rounds_filled(ctx, items, 6, 0.55), g, 2) : -1;
+    const bool filled = rounds_filled(ctx, items, 6, 0.55);
+    const int layout = phi_res == 1024 ? grid_layout(ctx, J, 2.0 * items, filled, g, 2) : -1;
     auto go = [&](auto kernel) {
-        kernel<<<dim3(nbx, nby), MC_THREADS, 0, ctx->stream>>>(spos, n1, n, n_rot, d_off, g[0], g[1], phi, J, phi_res, ws);
+        kernel<<<dim3(nbx, nby), MC_THREADS, 0, ctx->stream>>>(spos, n1, n, n_rot, d_off, g[0], g[1], phi, J, phi_res,
+                                                               ws);
     };
     if (layout == GRID_BRICK) go(k_triplet_box<GRID_BRICK>);
     else if (layout == GRID_ALIGNED) go(k_triplet_box<GRID_ALIGNED>);
@@ -860,8 +862,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
     if (!(cap > 0.0)) {
         HERMES_CHECK_HIP(hipMemsetAsync(stats, 0, 2 * sizeof(unsigned long long), ctx->stream));
         A.n = n_samples < PILOT ? n_samples : PILOT;
-        launch(k_mc_binned<MC_PILOT, GRID_BRICK>, k_mc_binned<MC_PILOT, GRID_ALIGNED>, k_mc_binned<MC_PILOT, GRID_PLAIN>, A,
-               nullptr, nullptr);
+        launch(k_mc_binned<MC_PILOT, GRID_BRICK>, k_mc_binned<MC_PILOT, GRID_ALIGNED>,
+               k_mc_binned<MC_PILOT, GRID_PLAIN>, A, nullptr, nullptr);
         HERMES_LAUNCH_CHECK();
         if (read_stats()) return 1;
         cap = max_of();
@@ -875,8 +877,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
         // |w f| <= cap for every accumulated sample: each bin sum stays below 2^62
         A.scale_wf = ldexp(1.0, 62) / ((double)n_samples * cap);
         A.scale_wf2 = ldexp(1.0, 62) / ((double)n_samples * cap * cap);
-        launch(k_mc_binned<MC_MAIN, GRID_BRICK>, k_mc_binned<MC_MAIN, GRID_ALIGNED>, k_mc_binned<MC_MAIN, GRID_PLAIN>, A,
-               nullptr, record);
+        launch(k_mc_binned<MC_MAIN, GRID_BRICK>, k_mc_binned<MC_MAIN, GRID_ALIGNED>,
+               k_mc_binned<MC_MAIN, GRID_PLAIN>, A, nullptr, record);
         HERMES_LAUNCH_CHECK();
         if (read_stats()) return 1;
         if (st[1] == 0) break;
@@ -895,8 +897,8 @@ int hermes_mc_binned(hermes_ctx* ctx, int J, const double* g1, const double* g2,
         F.record = 0;
         F.scale_wf = scale_hi = ldexp(1.0, 62) / ((double)n_over * mx);
         F.scale_wf2 = scale_hi2 = ldexp(1.0, 62) / ((double)n_over * mx * mx);
-        launch(k_mc_binned<MC_FIXUP, GRID_BRICK>, k_mc_binned<MC_FIXUP, GRID_ALIGNED>, k_mc_binned<MC_FIXUP, GRID_PLAIN>, F,
-               over_list, nullptr);
+        launch(k_mc_binned<MC_FIXUP, GRID_BRICK>, k_mc_binned<MC_FIXUP, GRID_ALIGNED>,
+               k_mc_binned<MC_FIXUP, GRID_PLAIN>, F, over_list, nullptr);
         HERMES_LAUNCH_CHECK();
     }
     std::vector<long long> h(5 * (size_t)B);

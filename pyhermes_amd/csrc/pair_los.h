@@ -6,7 +6,7 @@
 //   out[b] = sum_perp A_b(perp) sum_par S(perp, par) B_b(par):
 // a matrix product S B on the FP64 matrix cores (rows perp, columns windows) whose result meets A_b in the
 // lane that holds it.  The Bessel function of A is evaluated once per (perp alias, window) instead of once per
-// (alias, window, position): L / 2 + 1 times 2 fewer.  200 ring windows at L = 128: 30.17 ms that way, 0.14 ms
+// (alias, window, position): L / 2 + 1 times 2 fewer.  200 ring windows at L = 128: 30.17 ms that way, 0.13 ms
 // now.
 // Bound by the Bessel functions (FP64 VALU): 4 (L/2 + 1)^2 of them per window.
 #pragma once

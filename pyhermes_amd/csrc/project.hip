@@ -192,7 +192,8 @@ __global__ __launch_bounds__(256) void k_proj_count_lds(const double* __restrict
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int t = replica_tile(g, X, Y, Z, nx, ny, nz, k);
-            if (t >= 0) slots[(int64_t)k * n + p] = lcount[t] + (int)(k % 2 ? rank[i][k / 2] >> 16 : rank[i][k / 2] & 0xffff);
+            const uint32_t r = k % 2 ? rank[i][k / 2] >> 16 : rank[i][k / 2] & 0xffff;
+            if (t >= 0) slots[(int64_t)k * n + p] = lcount[t] + (int)r;
         }
     }
 }
@@ -277,7 +278,8 @@ template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_proj_fill(const double* __restrict__ pos, const double* __restrict__ w,
                                                    int64_t n, double sf, int res, TileGeom g,
                                                    const int* __restrict__ off, int* __restrict__ cursor,
-                                                   const int* __restrict__ slots, ProjRec* __restrict__ rec, unsigned long long* __restrict__ wmax) {
+                                                   const int* __restrict__ slots, ProjRec* __restrict__ rec,
+                                                   unsigned long long* __restrict__ wmax) {
     __shared__ double wred[4];
     double mw = 0.0;
     const int m = g.L - 1;
@@ -677,8 +679,8 @@ extern "C" int hermes_project(hermes_ctx* ctx, const double* pos, const double* 
                                                                               cell_out, frac_out, errp, slots);
     } else {
         const unsigned nb = hermes_blocks(n, 256, 4096);
-        if (slots) k_proj_count<true><<<nb, 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out, errp, slots);
-        else k_proj_count<false><<<nb, 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out, errp, nullptr);
+        auto kernel = slots ? k_proj_count<true> : k_proj_count<false>;
+        kernel<<<nb, 256, 0, st>>>(pos, n, sf, phi_res, g, count, cell_out, frac_out, errp, slots);
     }
     HERMES_LAUNCH_CHECK();
     if (nscan > 1) {

@@ -68,7 +68,8 @@ __global__ __launch_bounds__(256, 2) void k_build_rfft(int L, const double* __re
 // The same for a line of sight off the axes (descriptor axis 3), even only under k -> -k: every position sums its
 // signed aliases (the mirror alias L - x sits at k = -(L - x) / L).
 template <typename T>
-__global__ __launch_bounds__(256, 2) void k_build_rfft_general(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
+__global__ __launch_bounds__(256, 2) void k_build_rfft_general(int L, const double* __restrict__ P,
+                                                               hermes_window_desc d, T* __restrict__ out) {
     const int Lh = L / 2 + 1;
     const int64_t n = (int64_t)L * L * Lh;
     const double inv_L = 1.0 / L;
@@ -144,7 +145,8 @@ __global__ __launch_bounds__(256, 2) void k_build_full(int L, const double* __re
 
 // A real window along a line of sight off the axes (descriptor axis 3), position by position.
 template <typename T>
-__global__ __launch_bounds__(256, 2) void k_build_full_general(int L, const double* __restrict__ P, hermes_window_desc d, T* __restrict__ out) {
+__global__ __launch_bounds__(256, 2) void k_build_full_general(int L, const double* __restrict__ P,
+                                                               hermes_window_desc d, T* __restrict__ out) {
     const int64_t n = (int64_t)L * L * L;
     const double inv_L = 1.0 / L;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -931,8 +933,8 @@ static hipError_t launch_radial(hipStream_t st, int J, int dbl, int LM, int rows
         if (shmem > 32 * 1024)  // beside up to 25 KB of powers
             e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         if (e == hipSuccess)
-            kernel<<<dim3(rows, groups), threads, shmem, st>>>(L, f1, f2, P, d_radii, nu, R0, dR, d_chan, nch, nblk, per,
-                                                               partial);
+            kernel<<<dim3(rows, groups), threads, shmem, st>>>(L, f1, f2, P, d_radii, nu, R0, dR, d_chan, nch, nblk,
+                                                               per, partial);
     };
 #define HERMES_RADIAL(LMV, ROT)                                                                                      \
     do {                                                                                                             \
@@ -1061,8 +1063,8 @@ static bool pair_reduce_los(hermes_ctx* ctx, int J, int dbl, const void* F1, con
     double* partial = d_out + n_desc;
     hipError_t e = hipMemcpyAsync(d_desc, descs, sizeof(hermes_window_desc) * n_desc, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess) return fail(e);
-    k_los_par_table<<<hermes_blocks((int64_t)los_par_pad(L) * ncol, 256, 4096), 256, 0, ctx->stream>>>(L, P, d_desc, n_desc,
-                                                                                                ncol, tab);
+    const unsigned tab_blocks = hermes_blocks((int64_t)los_par_pad(L) * ncol, 256, 4096);
+    k_los_par_table<<<tab_blocks, 256, 0, ctx->stream>>>(L, P, d_desc, n_desc, ncol, tab);
     if ((e = hipGetLastError()) != hipSuccess) return fail(e);
     const size_t shmem = sizeof(double) * ((size_t)los_par_pad(L) * LOS_PITCH + (size_t)tpb * 16);
     auto go = [&](auto kernel, auto* f1, auto* f2) {
