@@ -8,10 +8,12 @@
 static thread_local char g_last_error[1024] = "";
 
 void hermes_set_error(const char* fmt, ...) {
+    char text[sizeof(g_last_error)];  // the arguments may be the last error itself
     va_list ap;
     va_start(ap, fmt);
-    vsnprintf(g_last_error, sizeof(g_last_error), fmt, ap);
+    vsnprintf(text, sizeof(text), fmt, ap);
     va_end(ap);
+    memcpy(g_last_error, text, strlen(text) + 1);
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
