@@ -148,9 +148,13 @@ def test_refused_workspace_leaves_no_error_behind(phi):
     want = kernels.project(good, gw, J, BOX, phi, want64=True)["eps64"]
     kernels.release_workspaces()
     torch.cuda.empty_cache()
-    free = torch.cuda.mem_get_info()[0]
-    print(f"projection with its records refused: {free / 2**30:.0f} GiB free", flush=True)
-    fill = torch.empty(max(free - (3 << 29), 1 << 20), dtype=torch.uint8, device="cuda")  # leaves 1.5 GiB; records: 2.5
+    print("projection with its records refused", flush=True)
+    fill, chunk = [torch.empty(int(0.98 * torch.cuda.mem_get_info()[0]), dtype=torch.uint8, device="cuda")], 1 << 28
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        while True:
+            fill.append(torch.empty(chunk, dtype=torch.uint8, device="cuda"))
+    del fill[-5:]  # 1.25 GiB for the slots and the tiles; the records ask for 2.5
+    torch.cuda.empty_cache()
     torch.cuda._sleep(30_000_000)
     with pytest.raises(RuntimeError, match="hermes_project failed .*hipMalloc of .* for workspace slot"):
         kernels.project(pos, w, J, BOX, phi)
